@@ -35,6 +35,7 @@
 
 #include <rocprofiler-sdk-roctx/roctx.h>
 
+#include "jacobi_dev.hpp"
 #include "jacobi_host.hpp"
 
 namespace cfm {
@@ -47,18 +48,6 @@ __global__ void reset_sync_kernel(GridSync *s, unsigned long long limit_ticks, i
         s->spin_limit_ticks = limit_ticks;
     }
     for (int b = t; b < grid; b += gridDim.x * blockDim.x) s->arrive[b] = 0;
-}
-
-// ------------------------------------------------------------ pass clock --
-// Phase timers of the Jacobi kernels (TIMED builds, A.timers set): the time
-// between barriers goes to the sweeps, the wait at the device-wide barrier to
-// the barrier.
-template <bool TIMED>
-__device__ __forceinline__ bool pass_barrier(const JacobiArgs &A, unsigned int &epoch, PhaseClock<TIMED> &clk) {
-    clk.mark(CFM_PHASE_SPMV);
-    const bool ok = grid_barrier(A.sync, epoch);
-    clk.mark(CFM_PHASE_BARRIER);
-    return ok;
 }
 
 typedef double v2f64 __attribute__((ext_vector_type(2)));
@@ -136,42 +125,6 @@ __device__ __forceinline__ T lane_dn1(T v) {
     }
 }
 
-// The same shifts with zeros shifted in at lane 0 / lane 63 (bound_ctrl): no copy
-// of the old value into the destination first, for callers that replace those
-// two lanes anyway.
-template <typename T>
-__device__ __forceinline__ T lane_up1z(T v) {
-    static_assert(sizeof(T) == 8 || sizeof(T) == 4, "4- or 8-byte values");
-    if constexpr (sizeof(T) == 8) {
-        union {
-            T t;
-            int i[2];
-        } a, r;
-        a.t = v;
-        r.i[0] = __builtin_amdgcn_mov_dpp(a.i[0], 0x138 /* wave_shr:1 */, 0xf, 0xf, true);
-        r.i[1] = __builtin_amdgcn_mov_dpp(a.i[1], 0x138, 0xf, 0xf, true);
-        return r.t;
-    } else {
-        return __builtin_bit_cast(T, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x138, 0xf, 0xf, true));
-    }
-}
-template <typename T>
-__device__ __forceinline__ T lane_dn1z(T v) {
-    static_assert(sizeof(T) == 8 || sizeof(T) == 4, "4- or 8-byte values");
-    if constexpr (sizeof(T) == 8) {
-        union {
-            T t;
-            int i[2];
-        } a, r;
-        a.t = v;
-        r.i[0] = __builtin_amdgcn_mov_dpp(a.i[0], 0x130 /* wave_shl:1 */, 0xf, 0xf, true);
-        r.i[1] = __builtin_amdgcn_mov_dpp(a.i[1], 0x130, 0xf, 0xf, true);
-        return r.t;
-    } else {
-        return __builtin_bit_cast(T, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x130, 0xf, 0xf, true));
-    }
-}
-
 // Interior stores of the new field: it is not read again before the next
 // sweep, by which time it has left the caches, so it may bypass them.
 #ifndef CFM_JACOBI_NT_STORE
@@ -203,16 +156,6 @@ __device__ __forceinline__ void load_row(const T *__restrict__ p, int x, int nx,
     }
 #pragma unroll
     for (int e = 0; e < VX; ++e) v[e] = (row_ok && x + e < nx) ? p[x + e] : T(0);
-}
-
-// Maps the workgroup index so that consecutive logical workgroups share an
-// XCD; returns the global wavefront index.
-__device__ __forceinline__ int xcd_wave_id() {
-    const int g = gridDim.x;
-    const int b = blockIdx.x;
-    int lb = b;
-    if ((g & 7) == 0) lb = (b & 7) * (g >> 3) + (b >> 3);
-    return lb * (blockDim.x >> 6) + (threadIdx.x >> 6);
 }
 
 // ------------------------------------------------------------------ 3D ----
@@ -2604,6 +2547,11 @@ cfm_status cfm::jacobi_configure(const cfm_jacobi_params *p, JacobiConfig *c) {
     c->chunks = (interior + c->chunk_len - 1) / c->chunk_len;
     c->norm_slots = p->norm_every > 0 ? (p->niter + p->norm_every - 1) / p->norm_every : 0;
     c->spin_ticks = spin_ticks(p->spin_limit_us);
+    c->norm_grid = c->grid;
+    // the defaults (nothing about the kernel asked for) may go to the register tiles
+    if (p->variant == CFM_JACOBI_PERSISTENT && p->time_block == 0 && p->tile_rows <= 0 && p->block_threads <= 0 &&
+        p->grid_blocks <= 0 && p->chunks <= 0)
+        c->tile = jacobi_tile_configure(*p, c);
     int rate_khz = 0;
     if (hipDeviceGetAttribute(&rate_khz, hipDeviceAttributeWallClockRate, c->dev.device) ==
             hipSuccess &&
@@ -2629,6 +2577,11 @@ cfm_status cfm::jacobi_enqueue(const cfm_jacobi_params &p, const JacobiConfig &c
     A.chunk_len = c.chunk_len;
     A.ntx = c.ntx;
     A.nty = c.nty;
+    A.tile_sx = c.tile_sx;
+    A.tile_sy = c.tile_sy;
+    A.tile_hx = c.tile_hx;
+    A.tile_hy = c.tile_hy;
+    A.depth = c.depth;
     A.norm_part = norm_part;
     A.sync = sync;
     A.timers = p.variant == CFM_JACOBI_LAUNCH_PER_ITER ? nullptr : timers;
@@ -2704,6 +2657,13 @@ int cfm::jacobi_passes(const cfm_jacobi_params &p, const JacobiConfig &c) {
     return (p.niter + c.sweeps_per_pass - 1) / c.sweeps_per_pass;
 }
 
+int cfm::jacobi_swaps(const cfm_jacobi_params &p, const JacobiConfig &c) {
+    if (!c.tile) return jacobi_passes(p, c);
+    // periodic rows: the first sweep is a pass of its own
+    const int first = p.bc == CFM_BC_PERIODIC ? std::min(p.niter, 1) : 0;
+    return first + (p.niter - first + c.depth - 1) / c.depth;
+}
+
 void cfm::jacobi_fill_timing(cfm_timing *t, const cfm_jacobi_params &p, const JacobiConfig &c, float ms,
                              double wall_ms, int coop) {
     if (!t) return;
@@ -2762,7 +2722,7 @@ static cfm_status jacobi_run(cfm_jacobi_plan *pl, double *norms, int norm_cap, i
         produced = c.norm_slots;
     }
     if (norm_count) *norm_count = produced;
-    pl->cur ^= jacobi_passes(p, c) & 1;
+    pl->cur ^= jacobi_swaps(p, c) & 1;
     jacobi_fill_timing(t, p, c, ms,
                 std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - w0).count(), coop);
     return CFM_OK;

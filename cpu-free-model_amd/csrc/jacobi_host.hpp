@@ -18,6 +18,9 @@ struct JacobiArgs {
     int chunks;       // chunks along the streamed axis
     int chunk_len;
     int ntx, nty;     // tiles along x and y (nty = 1 in 2D)
+    int tile_sx, tile_sy;  // register tiles: columns and rows a tile owns
+    int tile_hx, tile_hy;  // and loads beyond them on each side
+    int depth;             // sweeps per pass of the register tiles
     int no_compute;
     double *norm_part;  // [slot][gridDim.x]
     GridSync *sync;
@@ -36,21 +39,29 @@ struct JacobiConfig {
     KernelFn kernel = nullptr;
     bool t2 = false;  // more than one sweep per pass (the two-/three-/four-sweep kernels)
     int sweeps_per_pass = 1;
+    bool tile = false;  // the register-tile kernels (jacobi_tile.hip)
+    int tile_sx = 0, tile_sy = 0, tile_hx = 0, tile_hy = 0, depth = 0;
     int grid = 0;
+    int norm_grid = 0;  // the streaming kernel's grid, which the no-allocation entry point's limit goes by
     int chunks = 0, chunk_len = 0, ntx = 0, nty = 0, rows = 0, block = 256;
     unsigned long long spin_ticks = 0;
 };
 
 // Validates p and fills c for the current device.
 cfm_status jacobi_configure(const cfm_jacobi_params *p, JacobiConfig *c);
+// Takes c to a register-tile kernel where that is the faster one; false leaves it as it is.
+bool jacobi_tile_configure(const cfm_jacobi_params &p, JacobiConfig *c);
 // Enqueues one run of p.niter sweeps on `stream` (barrier reset, then the
 // persistent launch or one launch per sweep) over b0 (current field) and b1;
 // timers (may be null): per-workgroup phase ticks; *coop as launch_persistent
 // reports it (-1 without a persistent launch).
 cfm_status jacobi_enqueue(const cfm_jacobi_params &p, const JacobiConfig &c, void *b0, void *b1, GridSync *sync,
                           double *norm_part, unsigned long long *timers, hipStream_t stream, int *coop);
-// Passes over HBM of one run (its parity says which array holds the result).
+// Passes of one run, as time_block counts them.
 int jacobi_passes(const cfm_jacobi_params &p, const JacobiConfig &c);
+// Times that one run changes arrays (its parity says which array holds the result): its passes,
+// or the register tiles' own trips through memory.
+int jacobi_swaps(const cfm_jacobi_params &p, const JacobiConfig &c);
 void jacobi_fill_timing(cfm_timing *t, const cfm_jacobi_params &p, const JacobiConfig &c, float ms, double wall_ms,
                         int coop);
 

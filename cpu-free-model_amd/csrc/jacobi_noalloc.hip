@@ -70,10 +70,12 @@ extern "C" cfm_status cfm_jacobi_run_noalloc(const cfm_jacobi_params *p, void *f
     cfm_status st = jacobi_configure(p, &c);
     if (st != CFM_OK) return st;
     const size_t slots = p->variant == CFM_JACOBI_NO_COMPUTE ? 0 : (size_t)c.norm_slots;
-    if (slots * (size_t)c.grid + slots > kScratchDoubles)
+    if (slots * (size_t)c.norm_grid + slots > kScratchDoubles)
         return CFM_FAIL(CFM_EINVAL,
                         "jacobi_noalloc: %zu norm slots x %d workgroups exceed the %zu-double scratch array "
-                        "(fewer norms, or a plan)", slots, c.grid, kScratchDoubles);
+                        "(fewer norms, or a plan)", slots, c.norm_grid, kScratchDoubles);
+    // a register-tile grid may be the larger one; it runs on any number of workgroups
+    if (c.tile && slots > 0) c.grid = (int)std::min((size_t)c.grid, kScratchDoubles / slots - 1);
     unsigned char *base = nullptr;
     st = scratch_ptr(c.dev.device, &base);
     if (st != CFM_OK) return st;
@@ -109,7 +111,7 @@ extern "C" cfm_status cfm_jacobi_run_noalloc(const cfm_jacobi_params *p, void *f
     }
     if (norm_count) *norm_count = produced;
     // the result is in `work` after an odd number of passes: copy it back
-    if (jacobi_passes(*p, c) & 1) {
+    if (jacobi_swaps(*p, c) & 1) {
         CFM_HIP(hipMemcpyAsync(field, work, bytes, hipMemcpyDeviceToDevice, stream));
         CFM_HIP(hipStreamSynchronize(stream));
     }
