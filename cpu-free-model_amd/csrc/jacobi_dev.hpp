@@ -9,10 +9,10 @@ namespace cfm {
 // Phase timers of the Jacobi kernels (TIMED builds, A.timers set): the time
 // between barriers goes to the sweeps, the wait at the device-wide barrier to
 // the barrier.
-template <bool TIMED>
+template <bool THROUGH = false, bool TIMED>
 __device__ __forceinline__ bool pass_barrier(const JacobiArgs &A, unsigned int &epoch, PhaseClock<TIMED> &clk) {
     clk.mark(CFM_PHASE_SPMV);
-    const bool ok = grid_barrier(A.sync, epoch);
+    const bool ok = THROUGH ? grid_barrier_through(A.sync, epoch) : grid_barrier(A.sync, epoch);
     clk.mark(CFM_PHASE_BARRIER);
     return ok;
 }

@@ -30,6 +30,45 @@ struct VecAt {
     typedef T type __attribute__((ext_vector_type(N), aligned(sizeof(T))));
 };
 
+// A lane's N elements at row[x .. x+N), and one of them.  THROUGH: past the L2 (scope bit sc1), for
+// grid_barrier_through; rows are then shorter than 2 GiB.
+constexpr int kSc1 = 16;  // buffer instructions' cache policy bit
+template <bool THROUGH, typename T, int N>
+__device__ __forceinline__ typename VecAt<T, N>::type load_at(const T *row, int x) {
+    typedef typename VecAt<T, N>::type V;
+    if constexpr (THROUGH) {
+        static_assert(sizeof(T) * N == 16, "one 16-byte vector");
+        const auto rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)row, (short)0, 0x7fffffff, 0x00020000);
+        return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b128(rsrc, x * (int)sizeof(T), 0, kSc1));
+    } else {
+        return *reinterpret_cast<const V *>(row + x);
+    }
+}
+template <bool THROUGH, typename T>
+__device__ __forceinline__ T load_one(const T *p) {
+    if constexpr (THROUGH)
+        return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else
+        return *p;
+}
+template <bool THROUGH, typename T, int N, typename V>
+__device__ __forceinline__ void store_at(T *row, int x, V v) {
+    if constexpr (THROUGH) {
+        typedef unsigned int U4 __attribute__((ext_vector_type(4)));
+        const auto rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)row, (short)0, 0x7fffffff, 0x00020000);
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(U4, v), rsrc, x * (int)sizeof(T), 0, kSc1);
+    } else {
+        *reinterpret_cast<V *>(row + x) = v;
+    }
+}
+template <bool THROUGH, typename T>
+__device__ __forceinline__ void store_one(T *p, T v) {
+    if constexpr (THROUGH)
+        __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else
+        *p = v;
+}
+
 // ------------------------------------------------------------------ 2D ----
 // WAVES wavefronts, one above the other; each spans the tile's C columns (VX
 // per lane) and holds R rows.  The rows just outside a wavefront's own come
@@ -141,7 +180,7 @@ struct Place2D {
 
 // One tile, one pass.  EDGE = false: the tile touches no face and none of the pass's sweeps wants
 // its update norm, so nothing is tested per row or column.
-template <bool EDGE, typename T, int VX, int R, int WAVES>
+template <bool EDGE, bool THROUGH, typename T, int VX, int R, int WAVES>
 __device__ __forceinline__ void pass_tile2d(const JacobiArgs &A, const Place2D &P, const T *__restrict__ src,
                                             T *__restrict__ dst, int steps, int it, bool first,
                                             typename Tile2D<T, VX, R, WAVES>::Edge &edge, double *lds) {
@@ -170,7 +209,7 @@ __device__ __forceinline__ void pass_tile2d(const JacobiArgs &A, const Place2D &
         const T *p = src + (size_t)row * nx + P.x0;
 #pragma unroll
         for (int r = 0; r < R; ++r) {
-            const V v = *reinterpret_cast<const V *>(p + (size_t)r * nx + t.lane * VX);
+            const V v = load_at<THROUGH, T, VX>(p + (size_t)r * nx, t.lane * VX);
 #pragma unroll
             for (int e = 0; e < VX; ++e) t.a[r][e] = v[e];
         }
@@ -181,21 +220,24 @@ __device__ __forceinline__ void pass_tile2d(const JacobiArgs &A, const Place2D &
 #pragma unroll
             for (int e = 0; e < VX; ++e) t.a[r][e] = T(0);
             if (!EDGE || (row >= 0 && row < ny)) {  // uniform
-                const T *p = src + (size_t)row * nx + x;
+                const T *p = src + (size_t)row * nx;
                 if (lane_in) {
-                    const V v = *reinterpret_cast<const V *>(p);
+                    const V v = load_at<THROUGH, T, VX>(p, x);
 #pragma unroll
                     for (int e = 0; e < VX; ++e) t.a[r][e] = v[e];
                 } else {
 #pragma unroll
                     for (int e = 0; e < VX; ++e)
-                        if (x + e >= 0 && x + e < nx) t.a[r][e] = p[e];
+                        if (x + e >= 0 && x + e < nx) t.a[r][e] = load_one<THROUGH>(p + x + e);
                 }
             }
             ++row;
             if (P.wrap && row == ny - 1) row = 1;
         }
     }
+    // wait for the loads here: left to the first use, they are waited for again before every store
+    // below (a pass could have no sweeps, for all the compiler knows), and so is each store before it
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
     double acc = 0.0;
     if constexpr (!EDGE) {
         for (int s = 0; s < steps; ++s) t.template sweep<false, false>(edge[s & 1], acc);
@@ -224,20 +266,21 @@ __device__ __forceinline__ void pass_tile2d(const JacobiArgs &A, const Place2D &
             V v;
 #pragma unroll
             for (int e = 0; e < VX; ++e) v[e] = t.a[r][e];
-            T *p = dst + (size_t)(y + r) * nx + x;
+            T *p = dst + (size_t)(y + r) * nx;
             if (whole) {
-                *reinterpret_cast<V *>(p) = v;
+                store_at<THROUGH, T, VX>(p, x, v);
             } else {
 #pragma unroll
                 for (int e = 0; e < VX; ++e)
-                    if (x + e >= P.xo && x + e < P.xo_end && x + e >= 1 && x + e <= nx - 2) p[e] = v[e];
+                    if (x + e >= P.xo && x + e < P.xo_end && x + e >= 1 && x + e <= nx - 2)
+                        store_one<THROUGH, T>(p + x + e, v[e]);
             }
             if (periodic && (y + r == 1 || y + r == ny - 2)) {
 #pragma unroll
                 for (int e = 0; e < VX; ++e)
                     if (x + e >= P.xo && x + e < P.xo_end) {
-                        if (y + r == ny - 2) dst[x + e] = v[e];
-                        if (y + r == 1) dst[(size_t)(ny - 1) * nx + x + e] = v[e];
+                        if (y + r == ny - 2) store_one<THROUGH, T>(dst + x + e, v[e]);
+                        if (y + r == 1) store_one<THROUGH, T>(dst + (size_t)(ny - 1) * nx + x + e, v[e]);
                     }
             }
         }
@@ -245,9 +288,13 @@ __device__ __forceinline__ void pass_tile2d(const JacobiArgs &A, const Place2D &
 }
 
 // (128 registers a lane at most: two 8-wavefront workgroups, or one of 16, per CU)
+// Shapes for fields of few tiles go past the L2 (a tile is read once a pass, and each pass's
+// lines are another workgroup's by the next): the light barrier is worth more than the L2's hits
+// on the halos.  The shape for fields of many tiles keeps the L2.
 template <typename T, int VX, int R, int WAVES, bool TIMED>
 __global__ void __launch_bounds__(64 * WAVES, 4) jacobi2d_tile_kernel(JacobiArgs A) {
     constexpr int C = 64 * VX;
+    constexpr bool THROUGH = WAVES > 8;
     __shared__ typename Tile2D<T, VX, R, WAVES>::Edge edge;
     __shared__ double lds[WAVES];
     __shared__ unsigned long long clk_lds[kClockWords];
@@ -279,15 +326,15 @@ __global__ void __launch_bounds__(64 * WAVES, 4) jacobi2d_tile_kernel(JacobiArgs
             P.y0 = P.yo - A.tile_hy;
             const bool face = P.x0 < 1 || P.x0 + C > nx - 1 || (!P.wrap && (P.y0 < 1 || P.y0 + R * WAVES > ny - 1));
             if (face || norm)  // uniform over the workgroup
-                pass_tile2d<true, T, VX, R, WAVES>(A, P, src, dst, steps, it, u == first, edge, lds);
+                pass_tile2d<true, THROUGH, T, VX, R, WAVES>(A, P, src, dst, steps, it, u == first, edge, lds);
             else
-                pass_tile2d<false, T, VX, R, WAVES>(A, P, src, dst, steps, it, u == first, edge, lds);
+                pass_tile2d<false, THROUGH, T, VX, R, WAVES>(A, P, src, dst, steps, it, u == first, edge, lds);
             // the next tile's first publication must not overtake this one's last reads
             __syncthreads();
         }
         k += steps;
         if (k < A.niter) {
-            if (!pass_barrier(A, epoch, clk)) return;
+            if (!pass_barrier<THROUGH>(A, epoch, clk)) return;
         }
     }
     clk.mark(CFM_PHASE_SPMV);
@@ -329,24 +376,26 @@ Split2D split2d(const cfm_jacobi_params &p, const Shape2D &s, int depth) {
 // MI355X:
 //   * a wavefront's row costs its vector instructions (4 cycles each at 2.4 GHz): 12 per 2 FP64
 //     points and 18 per 4 FP32 points, 16 and 22 where faces are masked, on 4 SIMDs;
-//   * 0.1 us per sweep for the workgroup barrier and the LDS rows;
-//   * 9 us per pass for the device-wide barrier and the tile's first loads, none if one workgroup
-//     does it all;
+//   * a sweep's workgroup barrier and LDS rows: 0.2 us for 16 wavefronts, 0.05 where a second
+//     workgroup on the CU fills the wait;
+//   * a pass's device-wide barrier, first loads and last stores: 5.5 us past the L2, 9 us with the
+//     barrier's two fences, 2 us if one workgroup does it all;
 //   * the part of the field's traffic (at 5 TB/s) that a second workgroup on the CU does not hide.
-// At 16384^2 FP64 in 14-row, 8-wavefront tiles it gives 875, 1310 and 1770 us for depths 8, 12 and
-// 16, measured 900, 1322 and 1780; at 1024^2 in 6-row tiles 21 for depth 16, measured 24.
+// At 16384^2 FP64 in 14-row, 8-wavefront tiles it gives 890, 1330 and 1800 us for depths 8, 12 and
+// 16, measured 900, 1322 and 1780; at 1024^2 in 6-row tiles 16.1 and 23.2 for depths 12 and 20,
+// measured 17.2 and 24.9.
 double pass_us(const cfm_jacobi_params &p, const Shape2D &s, int depth, int cus) {
     const Split2D o = split2d(p, s, depth);
     if (o.ntx < 1) return 1e30;
     const bool f64 = p.prec == CFM_F64;
     const double tiles = (double)o.ntx * o.nty;
-    const bool one_round = tiles <= cus;
-    const double row = (f64 ? (one_round ? 64 : 48) : (one_round ? 88 : 72)) / 2400.0;
+    const bool pairs = s.waves <= 8;  // two workgroups per CU
     const double rounds = std::ceil(tiles / cus);
-    const int per_cu = s.waves > 8 ? 1 : 2;
+    const bool at_once = rounds <= (pairs ? 2 : 1);  // a pass then lasts as long as its tiles with faces
+    const double row = (f64 ? (at_once ? 64 : 48) : (at_once ? 88 : 72)) / 2400.0;
     const double traffic = 2.0 * (f64 ? 8 : 4) * p.nx * (double)p.ny / 5.0e6;
-    return (tiles > 1 ? 9.0 : 2.0) + 1.07 * rounds * depth * (s.r * s.waves / 4) * row +
-           0.1 * depth * std::ceil(tiles / (cus * per_cu)) + (per_cu > 1 ? 0.5 : 0.75) * traffic;
+    return (tiles > 1 ? (pairs ? 9.0 : 5.5) : 2.0) + 1.07 * rounds * depth * (s.r * s.waves / 4) * row +
+           (pairs ? 0.05 * std::ceil(rounds / 2) : 0.2 * rounds) * depth + (pairs ? 0.5 : 0.75) * traffic;
 }
 
 }  // namespace
