@@ -254,12 +254,43 @@ inline void summarize_phases(const unsigned long long *ticks, int workgroups, do
 }
 
 // --------------------------------------------------------- reductions ----
+// v + (v of lane ^ 32), and v + (v of lane ^ 16): the two halves of a permlane swap of v with
+// itself are the value of either side, and a+b == b+a exactly.
+__device__ __forceinline__ double xor32_sum(double v) {
+    const unsigned lo = __builtin_bit_cast(unsigned long long, v), hi = __builtin_bit_cast(unsigned long long, v) >> 32;
+    const auto l = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+    const auto h = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+    return __builtin_bit_cast(double, (unsigned long long)h[0] << 32 | l[0]) +
+           __builtin_bit_cast(double, (unsigned long long)h[1] << 32 | l[1]);
+}
+__device__ __forceinline__ double xor16_sum(double v) {
+    const unsigned lo = __builtin_bit_cast(unsigned long long, v), hi = __builtin_bit_cast(unsigned long long, v) >> 32;
+    const auto l = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+    const auto h = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+    return __builtin_bit_cast(double, (unsigned long long)h[0] << 32 | l[0]) +
+           __builtin_bit_cast(double, (unsigned long long)h[1] << 32 | l[1]);
+}
+// v + (v moved by a DPP control within rows of 16 lanes)
+template <int CTRL>
+__device__ __forceinline__ double dpp_sum(double v) {
+    const unsigned lo = __builtin_bit_cast(unsigned long long, v), hi = __builtin_bit_cast(unsigned long long, v) >> 32;
+    const unsigned l = __builtin_amdgcn_mov_dpp(lo, CTRL, 0xf, 0xf, true);
+    const unsigned h = __builtin_amdgcn_mov_dpp(hi, CTRL, 0xf, 0xf, true);
+    return v + __builtin_bit_cast(double, (unsigned long long)h << 32 | l);
+}
+
 // xor butterfly over the 64 lanes of a wavefront: offsets 32,16,8,4,2,1.
-// Every lane ends with the same value because a+b == b+a exactly.
+// Every lane ends with the same value because a+b == b+a exactly.  All in the
+// vector unit, where shuffles through the LDS cost a round trip for each offset:
+// a rotation by 8 within 16 lanes is xor 8, and once lanes i and i^8 agree, a
+// rotation by 4 is xor 4.
 __device__ __forceinline__ double wave_butterfly(double v) {
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) v = v + __shfl_xor(v, off, kWave);
-    return v;
+    v = xor32_sum(v);
+    v = xor16_sum(v);
+    v = dpp_sum<0x128>(v);  // row_ror:8
+    v = dpp_sum<0x124>(v);  // row_ror:4
+    v = dpp_sum<0x4e>(v);   // quad_perm:[2,3,0,1]
+    return dpp_sum<0xb1>(v);  // quad_perm:[1,0,3,2]
 }
 
 // Sum over a 256-thread workgroup: butterfly per wavefront, then

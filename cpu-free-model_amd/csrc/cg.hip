@@ -36,33 +36,9 @@
 
 #include <rocprofiler-sdk-roctx/roctx.h>
 
-#include "cg_common.hpp"
+#include "cg_args.hpp"
 
 namespace cfm {
-
-struct CgArgs {
-    int n;
-    int nchunks;
-    Sell A64;  // FP64 values
-    Sell A32;  // FP32 values (IR only)
-    const double *b;
-    const double *x0;
-    double *x;
-    double *v[6];        // work vectors (meaning depends on the method)
-    float *f[4];         // FP32 work vectors (IR)
-    double *part;        // partial sums, [8][nchunks]
-    double *hist;
-    int hist_cap;
-    int max_iter;
-    double tol;
-    int quirk;
-    int max_outer;
-    double inner_tol;
-    int *info;           // [0] status, [1] iterations, [2] outer iterations
-    GridSync *sync;
-    unsigned long long *timers;  // phase-timer build: [workgroup][kTimerSlots] ticks
-};
-
 
 // Iterate the rows this thread owns: sub-block `sub_` of workgroup b takes
 // chunk c = b*SUB + sub_ (+ multiples of gridDim.x*SUB); inside a chunk its
@@ -87,27 +63,6 @@ struct CgArgs {
         }                                                                                   \
         CHUNK_END                                                                           \
     }
-
-// Store that writes through the XCD's L2 (a relaxed agent-scope atomic store:
-// a vector store with scope bit sc1 on gfx950) instead of leaving a dirty
-// line there for the next device barrier's release to write back.  Measured
-// on the 128^3 Poisson system: Standard CG (s, x, r, p; three barriers per
-// iteration) 82.1 -> 76.4 us per iteration; the refinement's FP32 inner
-// iteration (s, d, r, p) 60.6 -> 59.7 us; Pipelined CG (one barrier per
-// iteration) gains only for w, the vector the next SpMV gathers (71.6 -> 70.7
-// us), and runs slower with its other vectors written through.  Being a
-// compiler-visible store, it is counted in the compiler's own wait counters.
-// Ordering against other workgroups comes only from the device barrier (a
-// workgroup barrier, then one thread's agent-scope release, which the HIP
-// memory model makes cumulative over the workgroup's earlier stores; an
-// agent-scope acquire on exit); the relaxed atomic adds no ordering of its own.
-__device__ __forceinline__ void store_wt(double *p, double v) {
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-__device__ __forceinline__ void store_wt(float *p, float v) {
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
 
 // =============================================================== phases ===
 // Standard CG.  v[0]=r, v[1]=p, v[2]=s.  part: [0]=gamma, [1]=delta, [2]=bb.
@@ -373,17 +328,6 @@ struct IrPhases {
 };
 
 // ======================================================= persistent kernels
-__device__ __forceinline__ void write_info(const CgArgs &A, int status, int iters, int outer) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        A.info[0] = status;
-        A.info[1] = iters;
-        A.info[2] = outer;
-    }
-}
-__device__ __forceinline__ void write_hist(const CgArgs &A, int k, double v) {
-    if (blockIdx.x == 0 && threadIdx.x == 0 && A.hist && k < A.hist_cap) A.hist[k] = v;
-}
-
 // The persistent kernels.  TIMED builds a second copy that records every
 // workgroup's time per phase (PhaseClock); the default build has no timer code.
 template <int SUB, bool TIMED>
@@ -625,8 +569,6 @@ __global__ void __launch_bounds__(256 * SUB) k_reduce(CgArgs A, int i0, int i1, 
 
 using namespace cfm;
 
-using CgKernelFn = void (*)(CgArgs);
-
 // The kernels of one workgroup shape (SUB sub-blocks of 256 threads).
 struct CgKernels {
     CgKernelFn standard, pipelined, ir;
@@ -675,7 +617,7 @@ static hipError_t launch(void (*f)(Args...), dim3 grid, dim3 block, hipStream_t 
 struct cfm_cg_plan {
     cfm_cg_params p{};
     DeviceProps dev{};
-    int n = 0, nnz = 0, nslices = 0, nchunks = 0;
+    int n = 0, nnz = 0, nslices = 0, nchunks = 0, entries = 0;
     int *slice_ptr = nullptr, *scol = nullptr;
     double *sval = nullptr;
     float *sval32 = nullptr;
@@ -693,6 +635,7 @@ struct cfm_cg_plan {
     int grid = 0;
     int sub = 4;  // 256-thread sub-blocks per workgroup
     CgKernels K{};
+    CgKernelFn persistent = nullptr;
     unsigned long long spin_ticks = 0;
     double clock_khz = 100000.0;           // s_memrealtime rate
     unsigned long long *timers = nullptr;  // phase_timers: [grid][kTimerSlots] ticks
@@ -861,6 +804,7 @@ extern "C" cfm_status cfm_cg_plan_create(int n, int nnz, const int *rowptr, cons
     pl->nnz = nnz;
     pl->ndiag = dia ? (int)doffs.size() : 0;
     pl->nslices = (int)sp.size() - 1;
+    pl->entries = sp.back();
     pl->nchunks = (n + kChunk - 1) / kChunk;
     auto fail = [&](cfm_status s) {
         cfm_cg_plan_destroy(pl);
@@ -922,6 +866,20 @@ extern "C" cfm_status cfm_cg_plan_create(int n, int nnz, const int *rowptr, cons
     const int max_grid = std::min(per_cu * pl->dev.cus, kMaxGrid);
     int want = p->grid_blocks > 0 ? p->grid_blocks : max_grid;
     pl->grid = std::max(1, std::min({want, max_grid, (pl->nchunks + pl->sub - 1) / pl->sub}));
+    pl->persistent = pl->K.persistent(p->method, p->phase_timers);
+    // a SELL-64 system that fits the chip's registers, unless a launch shape is asked for
+    if (p->mode == CFM_CG_PERSISTENT && !dia && p->block_threads <= 0 && p->grid_blocks <= 0) {
+        int width = 0;
+        for (int s = 0; s < pl->nslices; ++s) width = std::max(width, (sp[s + 1] - sp[s]) / 64);
+        const CgResident res = cg_resident(p->method, pl->nchunks, width, p->phase_timers != 0, pl->dev);
+        if (res.fn && hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void *)res.fn, kThreads * res.sub,
+                                                                   0) == hipSuccess &&
+            per_cu >= 1) {
+            pl->persistent = res.fn;
+            pl->sub = res.sub;
+            pl->grid = res.grid;
+        }
+    }
     int rate_khz = 0;
     const unsigned long long us = p->spin_limit_us > 0 ? p->spin_limit_us : 10000000ull;
     if (hipDeviceGetAttribute(&rate_khz, hipDeviceAttributeWallClockRate, pl->dev.device) != hipSuccess ||
@@ -961,6 +919,7 @@ static CgArgs make_args(cfm_cg_plan *pl) {
     CgArgs A{};
     A.n = pl->n;
     A.nchunks = pl->nchunks;
+    A.entries = pl->entries;
     const int npad = pl->nchunks * kChunk;
     A.A64 = Sell{pl->slice_ptr, pl->scol, pl->sval, pl->doff, pl->ndiag, pl->n, npad};
     A.A32 = Sell{pl->slice_ptr, pl->scol, pl->sval32, pl->doff, pl->ndiag, pl->n, npad};
@@ -1166,7 +1125,7 @@ extern "C" cfm_status cfm_cg_plan_solve(cfm_cg_plan *pl, double *hist, int hist_
         CFM_HIP(hipGetLastError());
         CFM_HIP(hipEventRecord(pl->ev0, pl->stream));
         void *args[] = {&A};
-        CFM_HIP(launch_persistent((const void *)pl->K.persistent(pl->p.method, timed), pl->grid, kThreads * pl->sub,
+        CFM_HIP(launch_persistent((const void *)pl->persistent, pl->grid, kThreads * pl->sub,
                                   args, pl->stream, &coop));
         CFM_HIP(hipEventRecord(pl->ev1, pl->stream));
         CFM_HIP(hipEventSynchronize(pl->ev1));

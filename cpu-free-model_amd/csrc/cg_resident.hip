@@ -1,0 +1,564 @@
+// Resident CG: the whole solve of a system that the chip can hold, with every
+// vector and the matrix in registers.
+//
+// Same recurrences, row-to-thread map and summation trees as cg.hip (so the
+// same bits); what changes is where things live.  A sub-block of 256 threads
+// owns one 1024-row chunk for the whole solve, four rows a thread; the rows'
+// entries, x, r, p, ... stay in its registers.  Only the vector that the SpMV
+// gathers and the chunk partials go through memory, past the L2 on both sides,
+// so the device barrier needs no L2 write-back or invalidate
+// (grid_barrier_through).
+//
+// Standard CG and the refinement keep the gathered entries of p as well: a row
+// gathers r after each update of r and forms its neighbours' p = r + beta p itself,
+// the owner's expression on the owner's values.  p is never published, and an
+// iteration has two barriers instead of three.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+
+#include "cg_args.hpp"
+
+namespace cfm {
+
+namespace {
+
+constexpr int kRows = 4;  // rows per thread: a chunk over a sub-block
+constexpr int kSc1 = 16;   // buffer instructions' cache policy bit: past the L2
+
+template <typename T>
+__device__ __forceinline__ T load_through(const T *p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// This thread's place: chunk c, rows c*1024 + i*256 + t.
+template <int SUB>
+struct Place {
+    int t, c;
+    bool in[kRows];
+    __device__ __forceinline__ explicit Place(const CgArgs &A) {
+        t = threadIdx.x & (kThreads - 1);
+        c = blockIdx.x * SUB + (threadIdx.x >> 8);
+#pragma unroll
+        for (int i = 0; i < kRows; ++i) in[i] = c < A.nchunks && row(i) < A.n;
+    }
+    __device__ __forceinline__ int row(int i) const { return c * kChunk + i * kThreads + t; }
+    __device__ __forceinline__ int slice(int i) const { return c * kSlicesPerChunk + i * 4 + (t >> 6); }
+};
+
+// The rows' entries in stored order.  Columns are kept as byte offsets into a vector of XT, -1 beyond
+// a row's end.  The gather is buffer loads (scope bit sc1: past the L2): their range check turns -1
+// into a zero, so all loads go out in one straight line, and they take the offset as it is, where plain loads would hold a 64-bit address for every entry.
+template <typename VT, typename XT, int W>
+struct Entries {
+    VT v[kRows][W];
+    int off[kRows][W];
+
+    template <int SUB>
+    __device__ __forceinline__ void load(const Sell &S, int entries, const Place<SUB> &P) {
+        const auto rc = __builtin_amdgcn_make_buffer_rsrc((void *)S.col, (short)0, entries * 4, 0x00020000);
+        const auto rv =
+            __builtin_amdgcn_make_buffer_rsrc((void *)S.val, (short)0, entries * (int)sizeof(VT), 0x00020000);
+#pragma unroll
+        for (int i = 0; i < kRows; ++i) {
+            int beg = 0, width = 0;
+            if (P.in[i]) {
+                beg = S.slice_ptr[P.slice(i)];
+                width = (S.slice_ptr[P.slice(i) + 1] - beg) >> 6;
+            }
+#pragma unroll
+            for (int j = 0; j < W; ++j) {
+                const int e = beg + 64 * j + (P.t & 63);
+                const int c = __builtin_amdgcn_raw_buffer_load_b32(rc, j < width ? e * 4 : -1, 0, 0);
+                if constexpr (sizeof(VT) == 8)
+                    v[i][j] = __builtin_bit_cast(
+                        VT, __builtin_amdgcn_raw_buffer_load_b64(rv, j < width ? e * 8 : -1, 0, 0));
+                else
+                    v[i][j] = __builtin_bit_cast(
+                        VT, __builtin_amdgcn_raw_buffer_load_b32(rv, j < width ? e * 4 : -1, 0, 0));
+                off[i][j] = j < width && c >= 0 ? c * (int)sizeof(XT) : -1;
+            }
+        }
+    }
+    // x: n elements (a resident system is far below 2 GiB)
+    __device__ __forceinline__ void gather(const XT *x, int n, XT (&g)[kRows][W]) const {
+        const auto rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)x, (short)0, n * (int)sizeof(XT), 0x00020000);
+#pragma unroll
+        for (int i = 0; i < kRows; ++i)
+#pragma unroll
+            for (int j = 0; j < W; ++j)
+                if constexpr (sizeof(XT) == 8)
+                    g[i][j] = __builtin_bit_cast(XT, __builtin_amdgcn_raw_buffer_load_b64(rsrc, off[i][j], 0, kSc1));
+                else
+                    g[i][j] = __builtin_bit_cast(XT, __builtin_amdgcn_raw_buffer_load_b32(rsrc, off[i][j], 0, kSc1));
+    }
+    // The row sum over gathered entries: sell_row's chain.  Entries beyond a row's end are 0 * 0,
+    // which leaves the sum as it is (skipping them instead held a lane mask per entry).
+    __device__ __forceinline__ XT row_sum(int i, const XT (&g)[kRows][W]) const {
+        XT acc = XT(0);
+#pragma unroll
+        for (int j = 0; j < W; ++j) acc = fma((XT)v[i][j], g[i][j], acc);
+        return acc;
+    }
+};
+
+// sub_sum of K values with one pair of workgroup barriers; lds holds K * 4 * SUB doubles.
+template <int SUB, int K>
+__device__ __forceinline__ void sub_sums(double (&v)[K], double *lds) {
+#pragma unroll
+    for (int k = 0; k < K; ++k) v[k] = wave_butterfly(v[k]);
+    __syncthreads();  // lds may still be read from a previous call
+    if ((threadIdx.x & 63) == 0)
+#pragma unroll
+        for (int k = 0; k < K; ++k) lds[k * 4 * SUB + (threadIdx.x >> 6)] = v[k];
+    __syncthreads();
+    const int w0 = (threadIdx.x >> 8) * 4;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        const double *l = lds + k * 4 * SUB + w0;
+        v[k] = (l[0] + l[1]) + (l[2] + l[3]);
+    }
+}
+
+// Chunk sums of K per-thread values into part[which[k]].
+template <int SUB, int K>
+__device__ __forceinline__ void put_partials(const CgArgs &A, const Place<SUB> &P, double (&v)[K], const int (&which)[K],
+                                             double *lds) {
+    sub_sums<SUB, K>(v, lds);
+    if (P.t == 0 && P.c < A.nchunks)
+#pragma unroll
+        for (int k = 0; k < K; ++k) store_wt(&A.part[which[k] * A.nchunks + P.c], v[k]);
+}
+
+// reduce_partials of K partial arrays at once (the same order of additions).
+template <int SUB, int K>
+__device__ __forceinline__ void get_partials(const CgArgs &A, const int (&which)[K], double (&v)[K], double *lds) {
+#pragma unroll
+    for (int k = 0; k < K; ++k) v[k] = 0.0;
+#pragma unroll
+    for (int u = 0; u < SUB; ++u) {  // (a grid of SUB chunks a workgroup is at most 256 workgroups)
+        const int j = (threadIdx.x & (kThreads - 1)) + u * kThreads;
+        if (j < A.nchunks)
+#pragma unroll
+            for (int k = 0; k < K; ++k) v[k] = v[k] + load_through(&A.part[which[k] * A.nchunks + j]);
+    }
+    sub_sums<SUB, K>(v, lds);
+}
+
+// r = b - A x0 of this thread's rows, <b,b> and <r,r> along the way.
+template <int SUB, int W>
+__device__ __forceinline__ void first_residual(const CgArgs &A, const Place<SUB> &P, const Entries<double, double, W> &M,
+                                               double (&x)[kRows], double (&r)[kRows], double &rr, double &bb) {
+    double g[kRows][W];
+    M.gather(A.x0, A.n, g);
+    rr = bb = 0.0;
+#pragma unroll
+    for (int i = 0; i < kRows; ++i) {
+        x[i] = r[i] = 0.0;
+        if (P.in[i]) {
+            const double bi = A.b[P.row(i)];
+            x[i] = A.x0[P.row(i)];
+            r[i] = fma(-1.0, M.row_sum(i, g), bi);
+            rr = fma(r[i], r[i], rr);
+            bb = fma(bi, bi, bb);
+        }
+    }
+}
+
+// Buffer stores past the L2: the range check drops rows beyond the system, and one offset a thread
+// serves all its rows.
+template <int SUB, typename T>
+__device__ __forceinline__ void publish(const CgArgs &A, const Place<SUB> &P, T *to, const T (&v)[kRows]) {
+    const auto rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)to, (short)0, A.n * (int)sizeof(T), 0x00020000);
+#pragma unroll
+    for (int i = 0; i < kRows; ++i) {
+        const int off = P.row(i) * (int)sizeof(T);
+        if constexpr (sizeof(T) == 8) {
+            typedef unsigned int U2 __attribute__((ext_vector_type(2)));
+            __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(U2, v[i]), rsrc, off, 0, kSc1);
+        } else {
+            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v[i]), rsrc, off, 0, kSc1);
+        }
+    }
+}
+
+// This thread's rows of a vector it published itself.
+template <int SUB>
+__device__ __forceinline__ void own_rows(const CgArgs &A, const Place<SUB> &P, const double *from, double (&v)[kRows]) {
+    const auto rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)from, (short)0, A.n * 8, 0x00020000);
+#pragma unroll
+    for (int i = 0; i < kRows; ++i)
+        v[i] = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(rsrc, P.row(i) * 8, 0, kSc1));
+}
+
+// Standard CG.  part: [0]=gamma, [1]=delta, [2]=bb; v[0]: r as the others gather it.  With two
+// sub-blocks (256 registers a lane) x stays in memory, where only its own thread touches it.
+template <int SUB, int W, bool TIMED>
+__global__ void __launch_bounds__(256 * SUB) cg_standard_resident(CgArgs A) {
+    __shared__ double lds[8 * SUB];
+    __shared__ unsigned long long clk_lds[kClockWords];
+    PhaseClock<TIMED> clk{clk_lds};
+    clk.start();
+    unsigned int epoch = 0;
+    const Place<SUB> P(A);
+    Entries<double, double, W> M;
+    M.load(A.A64, A.entries, P);
+    double x[kRows], r[kRows], p[kRows], pg[kRows][W];
+    double two[2];
+    first_residual(A, P, M, x, r, two[0], two[1]);
+    if (SUB > 1) publish(A, P, A.x, x);
+    publish(A, P, A.v[0], r);
+    put_partials<SUB, 2>(A, P, two, {0, 2}, lds);
+    clk.mark(CFM_PHASE_OTHER);
+    if (!grid_barrier_through(A.sync, epoch)) return;
+    clk.mark(CFM_PHASE_BARRIER);
+    M.gather(A.v[0], A.n, pg);  // p starts as r
+#pragma unroll
+    for (int i = 0; i < kRows; ++i) p[i] = r[i];
+    get_partials<SUB, 2>(A, {0, 2}, two, lds);
+    double gamma = two[0];
+    const double thr = A.tol > 0.0 ? A.tol * A.tol * two[1] : 0.0;
+    write_hist(A, 0, gamma);
+    clk.mark(CFM_PHASE_REDUCE);
+    int k = 0, status = CFM_OK;
+    bool converged = gamma <= thr;
+    while (!converged && k < A.max_iter) {
+        double s[kRows], one[1] = {0.0};
+#pragma unroll
+        for (int i = 0; i < kRows; ++i) {
+            s[i] = M.row_sum(i, pg);
+            if (P.in[i]) one[0] = fma(p[i], s[i], one[0]);
+        }
+        put_partials<SUB, 1>(A, P, one, {1}, lds);
+        clk.mark(CFM_PHASE_SPMV);
+        if (!grid_barrier_through(A.sync, epoch)) return;
+        clk.mark(CFM_PHASE_BARRIER);
+        get_partials<SUB, 1>(A, {1}, one, lds);
+        const double delta = one[0];
+        clk.mark(CFM_PHASE_REDUCE);
+        if (!(delta > 0.0) || !is_finite(delta)) {
+            status = CFM_EBREAKDOWN;
+            break;
+        }
+        const double alpha = gamma / delta;
+        one[0] = 0.0;
+        if (SUB > 1) own_rows(A, P, A.x, x);
+#pragma unroll
+        for (int i = 0; i < kRows; ++i) {
+            x[i] = fma(alpha, p[i], x[i]);
+            r[i] = fma(-alpha, s[i], r[i]);
+            if (P.in[i]) one[0] = fma(r[i], r[i], one[0]);
+        }
+        if (SUB > 1) publish(A, P, A.x, x);
+        publish(A, P, A.v[0], r);
+        put_partials<SUB, 1>(A, P, one, {0}, lds);
+        clk.mark(CFM_PHASE_UPDATE);
+        if (!grid_barrier_through(A.sync, epoch)) return;
+        clk.mark(CFM_PHASE_BARRIER);
+        double rg[kRows][W];
+        M.gather(A.v[0], A.n, rg);  // on its way while the partials are summed
+        get_partials<SUB, 1>(A, {0}, one, lds);
+        const double gamma_new = one[0];
+        ++k;
+        write_hist(A, k, gamma_new);
+        clk.mark(CFM_PHASE_REDUCE);
+        if (gamma_new <= thr) {
+            converged = true;
+            break;
+        }
+        const double beta = gamma_new / gamma;
+#pragma unroll
+        for (int i = 0; i < kRows; ++i) {
+            p[i] = fma(beta, p[i], r[i]);
+#pragma unroll
+            for (int j = 0; j < W; ++j) pg[i][j] = fma(beta, pg[i][j], rg[i][j]);
+        }
+        gamma = gamma_new;
+    }
+    if (status == CFM_OK && !converged && A.tol > 0.0) status = CFM_ENOTCONV;
+    if (SUB == 1)
+#pragma unroll
+        for (int i = 0; i < kRows; ++i)
+            if (P.in[i]) A.x[P.row(i)] = x[i];
+    write_info(A, status, k, 0);
+    clk.mark(CFM_PHASE_OTHER);
+    clk.flush(A.timers);
+}
+
+// Pipelined CG.  part as in cg.hip: [0,1] = delta, [2,3] = gamma (by iteration parity), [4] = bb.
+// v[0]: r (for w0 only), v[4], v[5]: w by iteration parity.
+template <int SUB, int W, bool TIMED>
+__global__ void __launch_bounds__(256 * SUB) cg_pipelined_resident(CgArgs A) {
+    __shared__ double lds[8 * SUB];
+    __shared__ unsigned long long clk_lds[kClockWords];
+    PhaseClock<TIMED> clk{clk_lds};
+    clk.start();
+    unsigned int epoch = 0;
+    const Place<SUB> P(A);
+    Entries<double, double, W> M;
+    M.load(A.A64, A.entries, P);
+    double x[kRows], r[kRows], z[kRows], s[kRows], p[kRows], w[kRows], g[kRows][W];
+    double one[1], two[2];
+    first_residual(A, P, M, x, r, two[0], one[0]);
+    publish(A, P, A.v[0], r);
+    put_partials<SUB, 1>(A, P, one, {4}, lds);
+    clk.mark(CFM_PHASE_OTHER);
+    if (!grid_barrier_through(A.sync, epoch)) return;
+    clk.mark(CFM_PHASE_BARRIER);
+    M.gather(A.v[0], A.n, g);
+    two[0] = two[1] = 0.0;
+#pragma unroll
+    for (int i = 0; i < kRows; ++i) {
+        w[i] = M.row_sum(i, g);
+        z[i] = s[i] = p[i] = 0.0;
+        if (P.in[i]) {
+            two[0] = fma(r[i], r[i], two[0]);
+            two[1] = fma(r[i], w[i], two[1]);
+        }
+    }
+    publish(A, P, A.v[4], w);
+    put_partials<SUB, 2>(A, P, two, {0, 2}, lds);
+    clk.mark(CFM_PHASE_OTHER);
+    if (!grid_barrier_through(A.sync, epoch)) return;
+    clk.mark(CFM_PHASE_BARRIER);
+    get_partials<SUB, 1>(A, {4}, one, lds);
+    const double thr = A.tol > 0.0 ? A.tol * A.tol * one[0] : 0.0;
+    double alpha = 0.0, beta = 0.0, delta_prev = 0.0;
+    int k = 0, status = CFM_OK;
+    bool converged = false;
+    for (;;) {
+        const int buf = k & 1;
+        M.gather(A.v[4 + buf], A.n, g);  // on its way while the partials are summed
+        get_partials<SUB, 2>(A, {0 + buf, 2 + buf}, two, lds);
+        const double delta = two[0], gam = two[1];
+        write_hist(A, k, delta);
+        clk.mark(CFM_PHASE_REDUCE);
+        if (delta <= thr) {
+            converged = true;
+            break;
+        }
+        if (k >= A.max_iter) break;
+        double denom;
+        if (A.quirk ? (k > 1) : (k > 0)) {
+            beta = delta / delta_prev;
+            denom = gam - (beta / alpha) * delta;
+        } else {
+            beta = 0.0;
+            denom = gam;
+        }
+        if (!(denom > 0.0) || !is_finite(denom)) {
+            status = CFM_EBREAKDOWN;
+            break;
+        }
+        alpha = delta / denom;
+        two[0] = two[1] = 0.0;
+#pragma unroll
+        for (int i = 0; i < kRows; ++i) {
+            z[i] = fma(beta, z[i], M.row_sum(i, g));
+            s[i] = fma(beta, s[i], w[i]);
+            p[i] = fma(beta, p[i], r[i]);
+            x[i] = fma(alpha, p[i], x[i]);
+            r[i] = fma(-alpha, s[i], r[i]);
+            w[i] = fma(-alpha, z[i], w[i]);
+            if (P.in[i]) {
+                two[0] = fma(r[i], r[i], two[0]);
+                two[1] = fma(r[i], w[i], two[1]);
+            }
+        }
+        publish(A, P, A.v[5 - buf], w);
+        put_partials<SUB, 2>(A, P, two, {1 - buf, 3 - buf}, lds);
+        clk.mark(CFM_PHASE_SPMV);
+        if (!grid_barrier_through(A.sync, epoch)) return;
+        clk.mark(CFM_PHASE_BARRIER);
+        delta_prev = delta;
+        ++k;
+    }
+    if (status == CFM_OK && !converged && A.tol > 0.0) status = CFM_ENOTCONV;
+#pragma unroll
+    for (int i = 0; i < kRows; ++i)
+        if (P.in[i]) A.x[P.row(i)] = x[i];
+    write_info(A, status, k, 0);
+    clk.mark(CFM_PHASE_OTHER);
+    clk.flush(A.timers);
+}
+
+// Row i of A x in FP64 for the refinement: the FP64 values are read again each time (there are few
+// refinements), the columns are the ones at hand.
+template <int SUB, int W>
+__device__ __forceinline__ double row_sum64(const CgArgs &A, const Place<SUB> &P, const Entries<float, float, W> &M,
+                                            int i, const double *x) {
+    const auto rv = __builtin_amdgcn_make_buffer_rsrc((void *)A.A64.val, (short)0, A.entries * 8, 0x00020000);
+    const auto rx = __builtin_amdgcn_make_buffer_rsrc((void *)x, (short)0, A.n * 8, 0x00020000);
+    const int e = (P.in[i] ? A.A64.slice_ptr[P.slice(i)] : 0) + (P.t & 63);
+    double v[W], g[W], acc = 0.0;
+#pragma unroll
+    for (int j = 0; j < W; ++j) {
+        const bool ok = M.off[i][j] >= 0;
+        v[j] = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(rv, ok ? (e + 64 * j) * 8 : -1, 0, 0));
+        g[j] = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(rx, ok ? M.off[i][j] * 2 : -1, 0, kSc1));
+    }
+#pragma unroll
+    for (int j = 0; j < W; ++j) acc = fma(v[j], g[j], acc);
+    return acc;
+}
+
+// FP32 inner CG inside FP64 refinement.  part: [0]=rr (outer), [1]=g, [2]=delta, [3]=bb.
+// f[0]: the inner residual as the others gather it; A.x likewise between refinements.
+template <int SUB, int W, bool TIMED>
+__global__ void __launch_bounds__(256 * SUB) cg_ir_resident(CgArgs A) {
+    __shared__ double lds[12 * SUB];
+    __shared__ unsigned long long clk_lds[kClockWords];
+    PhaseClock<TIMED> clk{clk_lds};
+    clk.start();
+    unsigned int epoch = 0;
+    const Place<SUB> P(A);
+    Entries<float, float, W> M;
+    M.load(A.A32, A.entries, P);
+    double thr = 0.0;
+    int outer = 0, inner_total = 0, status = CFM_ENOTCONV;
+    for (;;) {
+        const bool first = outer == 0;
+        float rf[kRows], p[kRows], d[kRows], pg[kRows][W];
+        double three[3];
+        {
+            double r[kRows];
+            three[0] = three[2] = 0.0;
+#pragma unroll
+            for (int i = 0; i < kRows; ++i) {
+                const double ax = row_sum64(A, P, M, i, first ? A.x0 : A.x);
+                r[i] = 0.0;
+                if (P.in[i]) {
+                    const double bi = A.b[P.row(i)];
+                    r[i] = fma(-1.0, ax, bi);
+                    three[0] = fma(r[i], r[i], three[0]);
+                    three[2] = fma(bi, bi, three[2]);
+                }
+            }
+            if (first) {
+                double x[kRows];
+                own_rows(A, P, A.x0, x);
+                publish(A, P, A.x, x);
+            }
+            three[1] = 0.0;
+#pragma unroll
+            for (int i = 0; i < kRows; ++i) {
+                rf[i] = p[i] = (float)r[i];
+                d[i] = 0.0f;
+                if (P.in[i]) three[1] = fma((double)rf[i], (double)rf[i], three[1]);
+            }
+        }
+        publish(A, P, A.f[0], rf);
+        put_partials<SUB, 3>(A, P, three, {0, 1, 3}, lds);
+        clk.mark(CFM_PHASE_OTHER);
+        if (!grid_barrier_through(A.sync, epoch)) return;
+        clk.mark(CFM_PHASE_BARRIER);
+        M.gather(A.f[0], A.n, pg);  // p starts as the residual
+        get_partials<SUB, 3>(A, {0, 1, 3}, three, lds);
+        if (first) thr = A.tol * A.tol * three[2];
+        const double rr = three[0];
+        write_hist(A, outer, rr);
+        clk.mark(CFM_PHASE_REDUCE);
+        if (rr <= thr) {
+            status = CFM_OK;
+            break;
+        }
+        if (outer == A.max_outer) break;
+        double g = three[1];
+        // no refinement is solved beyond half the outer target
+        const double thr_in = fmax(A.inner_tol * A.inner_tol * g, 0.25 * thr);
+        int j = 0;
+        bool brk = false;
+        while (j < A.max_iter) {
+            float s[kRows];
+            double one[1] = {0.0};
+#pragma unroll
+            for (int i = 0; i < kRows; ++i) {
+                s[i] = M.row_sum(i, pg);
+                if (P.in[i]) one[0] = fma((double)p[i], (double)s[i], one[0]);
+            }
+            put_partials<SUB, 1>(A, P, one, {2}, lds);
+            clk.mark(CFM_PHASE_SPMV);
+            if (!grid_barrier_through(A.sync, epoch)) return;
+            clk.mark(CFM_PHASE_BARRIER);
+            get_partials<SUB, 1>(A, {2}, one, lds);
+            const double delta = one[0];
+            clk.mark(CFM_PHASE_REDUCE);
+            if (!(delta > 0.0) || !is_finite(delta)) {
+                brk = true;
+                break;
+            }
+            const float af = (float)(g / delta);
+            one[0] = 0.0;
+#pragma unroll
+            for (int i = 0; i < kRows; ++i) {
+                d[i] = fmaf(af, p[i], d[i]);
+                rf[i] = fmaf(-af, s[i], rf[i]);
+                if (P.in[i]) one[0] = fma((double)rf[i], (double)rf[i], one[0]);
+            }
+            publish(A, P, A.f[0], rf);
+            put_partials<SUB, 1>(A, P, one, {1}, lds);
+            clk.mark(CFM_PHASE_UPDATE);
+            if (!grid_barrier_through(A.sync, epoch)) return;
+            clk.mark(CFM_PHASE_BARRIER);
+            float rg[kRows][W];
+            M.gather(A.f[0], A.n, rg);
+            get_partials<SUB, 1>(A, {1}, one, lds);
+            const double gn = one[0];
+            clk.mark(CFM_PHASE_REDUCE);
+            ++j;
+            if (gn <= thr_in) break;
+            const float bf = (float)(gn / g);
+#pragma unroll
+            for (int i = 0; i < kRows; ++i) {
+                p[i] = fmaf(bf, p[i], rf[i]);
+#pragma unroll
+                for (int e = 0; e < W; ++e) pg[i][e] = fmaf(bf, pg[i][e], rg[i][e]);
+            }
+            g = gn;
+        }
+        inner_total += j;
+        double x[kRows];
+        own_rows(A, P, A.x, x);
+#pragma unroll
+        for (int i = 0; i < kRows; ++i) x[i] = x[i] + (double)d[i];
+        publish(A, P, A.x, x);
+        clk.mark(CFM_PHASE_UPDATE);
+        if (!grid_barrier_through(A.sync, epoch)) return;
+        clk.mark(CFM_PHASE_BARRIER);
+        ++outer;
+        if (brk && j == 0) {
+            status = CFM_EBREAKDOWN;
+            break;
+        }
+    }
+    write_info(A, status, inner_total, outer);
+    clk.flush(A.timers);
+}
+
+template <int SUB, int W>
+CgKernelFn resident_fn(int method, bool timed) {
+    switch (method) {
+        case CFM_CG_STANDARD: return timed ? cg_standard_resident<SUB, W, true> : cg_standard_resident<SUB, W, false>;
+        case CFM_CG_PIPELINED:
+            return timed ? cg_pipelined_resident<SUB, W, true> : cg_pipelined_resident<SUB, W, false>;
+        default: return timed ? cg_ir_resident<SUB, W, true> : cg_ir_resident<SUB, W, false>;
+    }
+}
+
+}  // namespace
+
+CgResident cg_resident(int method, int nchunks, int max_width, bool timed, const DeviceProps &dev) {
+    CgResident o;
+    const int cus = std::min(dev.cus, kThreads);  // (get_partials reads one partial a thread and sub-block)
+    if (max_width > 7 || nchunks > 2 * cus) return o;
+    // one chunk per workgroup while there is a CU for each, else two
+    o.sub = nchunks <= cus ? 1 : 2;
+    o.grid = (nchunks + o.sub - 1) / o.sub;
+    if (o.sub == 1)
+        o.fn = max_width <= 3 ? resident_fn<1, 3>(method, timed) : resident_fn<1, 7>(method, timed);
+    else
+        o.fn = max_width <= 3 ? resident_fn<2, 3>(method, timed) : resident_fn<2, 7>(method, timed);
+    return o;
+}
+
+}  // namespace cfm
