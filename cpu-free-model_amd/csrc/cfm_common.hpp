@@ -115,6 +115,8 @@ __device__ __forceinline__ bool grid_barrier(GridSync *s, unsigned int &epoch) {
 // write back or invalidate, one workgroup after the other: 56 ns for each of the 32 workgroups on an
 // XCD.  Measured alone at 256 workgroups: 1.6 us a barrier, 5.2 us with the fences (1.25 and 1.34
 // at 8).  Every wavefront waits for its own stores first, as an agent-scope release would.
+// ACQUIRE: with the invalidate, for a phase that reads others' data through the caches (3.3 us).
+template <bool ACQUIRE = false>
 __device__ __forceinline__ bool grid_barrier_through(GridSync *s, unsigned int &epoch) {
     __shared__ int s_abort;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -151,6 +153,7 @@ __device__ __forceinline__ bool grid_barrier_through(GridSync *s, unsigned int &
         if (threadIdx.x < kGoCopies && !s_abort)
             __hip_atomic_store(&s->go[32 * threadIdx.x], e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
+    if (ACQUIRE && threadIdx.x == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     __syncthreads();
     // (the compiler moves no access across)
     asm volatile("" ::: "memory");
@@ -190,6 +193,14 @@ inline cfm_status barrier_timeout(const char *what, int cooperative) {
                           : "ordinary launch: another process held the cooperative-launch grant, so "
                             "co-residency of the workgroups was not guaranteed");
     return CFM_ETIMEOUT;
+}
+
+// Maps the workgroup index so that consecutive logical workgroups share an
+// XCD (workgroup i runs on XCD i % 8).
+__device__ __forceinline__ int xcd_block_id() {
+    const int g = gridDim.x;
+    const int b = blockIdx.x;
+    return (g & 7) == 0 ? (b & 7) * (g >> 3) + (b >> 3) : b;
 }
 
 // -------------------------------------------------------- phase timers ----

@@ -772,19 +772,27 @@ extern "C" cfm_status cfm_cg_plan_create(int n, int nnz, const int *rowptr, cons
     std::vector<int> sp, sc, doffs;
     std::vector<double> sv;
     const int npad = (n + kChunk - 1) / kChunk * kChunk;
-    // auto: DIA for Pipelined CG on large systems (measured 70 vs 80 us per
-    // iteration at 128^3 = 2.1M rows, where the index-free matrix and the vectors
-    // fit the MALL); SELL-64 for small systems (64^3: 27.8 vs 22.2 us per
-    // iteration, latency-bound, where the 8-wide SELL loop wins), for Standard CG
-    // and for the FP32 refinement
+    // auto: DIA for the systems whose matrix the resident kernels stream (96^3 and 128^3, us per
+    // iteration, SELL-64 / DIA: Standard 25.5 / 21.7 and 41.5 / 34.8, Pipelined 19.3 / 16.7 and
+    // 40.4 / 31.0, the refinement 21.9 / 16.6 and 33.4 / 23.8), and beyond them for Pipelined CG
+    // (general kernels at 128^3: Pipelined 70 vs 80, Standard 89.6 vs 81.9, the refinement 72.4 vs
+    // 62.1).  Smaller systems hold their SELL-64 entries in registers.
+    DeviceProps dev;
+    const cfm_status dst = current_device_props(&dev);
+    if (dst != CFM_OK) return dst;
     constexpr int kDiaMinRows = 1 << 20;
+    const bool resident_ok = p->mode == CFM_CG_PERSISTENT && p->block_threads <= 0 && p->grid_blocks <= 0;
     bool dia = false;
     if (p->matrix_format == 2 ||
-        (p->matrix_format == 0 && p->method == CFM_CG_PIPELINED && n >= kDiaMinRows)) {
+        (p->matrix_format == 0 && ((p->method == CFM_CG_PIPELINED && n >= kDiaMinRows) ||
+                                   (resident_ok && cg_resident_streams(npad / kChunk, dev))))) {
         dia = build_dia(n, npad, rp, cp, vp, index_base, doffs, sv);
         if (!dia && p->matrix_format == 2)
             return CFM_FAIL(CFM_ENOTSUP, "cg: DIA storage needs a banded matrix (<= %d diagonals, sorted rows)",
                             kMaxDiag);
+        // (with more diagonals than the resident kernels take, only Pipelined CG gains)
+        if (dia && p->matrix_format == 0 && p->method != CFM_CG_PIPELINED && (int)doffs.size() > kResidentDiag)
+            dia = false;
     }
     cfm_status st = CFM_OK;
     if (dia) {
@@ -810,8 +818,7 @@ extern "C" cfm_status cfm_cg_plan_create(int n, int nnz, const int *rowptr, cons
         cfm_cg_plan_destroy(pl);
         return s;
     };
-    st = current_device_props(&pl->dev);
-    if (st != CFM_OK) return fail(st);
+    pl->dev = dev;
     // slices are read per chunk: pad the slice table to whole chunks
     const int nslices_pad = pl->nchunks * kSlicesPerChunk;
     const int last_off = sp.back();
@@ -867,11 +874,11 @@ extern "C" cfm_status cfm_cg_plan_create(int n, int nnz, const int *rowptr, cons
     int want = p->grid_blocks > 0 ? p->grid_blocks : max_grid;
     pl->grid = std::max(1, std::min({want, max_grid, (pl->nchunks + pl->sub - 1) / pl->sub}));
     pl->persistent = pl->K.persistent(p->method, p->phase_timers);
-    // a SELL-64 system that fits the chip's registers, unless a launch shape is asked for
-    if (p->mode == CFM_CG_PERSISTENT && !dia && p->block_threads <= 0 && p->grid_blocks <= 0) {
-        int width = 0;
-        for (int s = 0; s < pl->nslices; ++s) width = std::max(width, (sp[s + 1] - sp[s]) / 64);
-        const CgResident res = cg_resident(p->method, pl->nchunks, width, p->phase_timers != 0, pl->dev);
+    // a system whose vectors fit the chip's registers, unless a launch shape is asked for
+    if (resident_ok) {
+        int width = pl->ndiag;
+        for (int s = 0; s < pl->nslices && !dia; ++s) width = std::max(width, (sp[s + 1] - sp[s]) / 64);
+        const CgResident res = cg_resident(p->method, pl->nchunks, width, dia, p->phase_timers != 0, pl->dev);
         if (res.fn && hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void *)res.fn, kThreads * res.sub,
                                                                    0) == hipSuccess &&
             per_cu >= 1) {

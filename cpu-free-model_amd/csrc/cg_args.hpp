@@ -64,12 +64,15 @@ __device__ __forceinline__ void write_hist(const CgArgs &A, int k, double v) {
 
 using CgKernelFn = void (*)(CgArgs);
 
-// The resident kernel (cg_resident.hip) for a SELL-64 system of this method whose rows hold at
-// most max_width entries, with its workgroup and grid; null where it does not apply.
+// The resident kernel (cg_resident.hip) for a system of this method, stored as DIA or as SELL-64
+// with at most max_width diagonals or entries a row, with its workgroup and grid; null where it does not apply.
 struct CgResident {
     CgKernelFn fn = nullptr;
     int sub = 0, grid = 0;
 };
-CgResident cg_resident(int method, int nchunks, int max_width, bool timed, const DeviceProps &dev);
+constexpr int kResidentDiag = 8;  // diagonals they take at most
+// whether a system of nchunks chunks is one whose matrix they stream
+bool cg_resident_streams(int nchunks, const DeviceProps &dev);
+CgResident cg_resident(int method, int nchunks, int max_width, bool dia, bool timed, const DeviceProps &dev);
 
 }  // namespace cfm

@@ -53,14 +53,6 @@ __device__ __forceinline__ T lane_dn1z(T v) {
     }
 }
 
-// Maps the workgroup index so that consecutive logical workgroups share an
-// XCD (workgroup i runs on XCD i % 8).
-__device__ __forceinline__ int xcd_block_id() {
-    const int g = gridDim.x;
-    const int b = blockIdx.x;
-    return (g & 7) == 0 ? (b & 7) * (g >> 3) + (b >> 3) : b;
-}
-
 // The global wavefront index under the same map.
 __device__ __forceinline__ int xcd_wave_id() { return xcd_block_id() * (blockDim.x >> 6) + (threadIdx.x >> 6); }
 

@@ -216,8 +216,9 @@ typedef struct {
     int block_threads;   /* 256, 512, 768 or 1024 (256-row sub-blocks per workgroup); 0 = auto */
     int x0_guard;        /* batched plans: nonzero restarts a system from x0 = 0 when
                             ||b - A x0|| > ||b|| (the guard for learned initial guesses) */
-    int matrix_format;   /* 0 = auto (single-system Pipelined with >= 2^20 rows: DIA when the CSR
-                            is banded with <= 16 diagonals and sorted rows; otherwise SELL-64),
+    int matrix_format;   /* 0 = auto (single systems of more than 2^19 rows whose vectors fit the
+                            registers, and Pipelined with >= 2^20 rows: DIA when the CSR is banded
+                            with <= 8 diagonals (Pipelined: 16) and sorted rows; otherwise SELL-64),
                             1 = SELL-64, 2 = DIA (every system of a batch; ENOTSUP if not banded);
                             an auto batched plan holds SELL-64 and, when every system is banded,
                             DIA beside it for the autotuner to choose (solves start on SELL-64) */
