@@ -26,46 +26,13 @@
 #include <string>
 #include <vector>
 
-#include "cg_common.hpp"
+#include "cg_batch_args.hpp"
 #include "unet.hpp"
 
 namespace cfm {
 
 constexpr int kMaxSys = 4096;
 constexpr int kMaxOverlap = 64;  // systems handled per pass of a workgroup's range
-
-enum { kActive = 0, kConverged = 1, kBreakdown = 2, kMaxIter = 3 };
-
-struct BatchArgs {
-    int nsys;
-    int total_chunks;
-    const int *sys_chunk0;  // [nsys+1] first chunk of each system
-    const int *sys_rows;    // [nsys] real rows of each system
-    Sell A;                 // SELL-64 over the padded global rows
-    const double *b;
-    const double *x0;
-    double *x, *r, *z, *s, *p;
-    double *w[2];
-    double *part;      // [5][total_chunks]: delta buf0/1, gamma buf0/1, <b,b>
-    double *st_alpha;  // [2][nsys]
-    double *st_delta;  // [2][nsys]
-    int *fin;          // [nsys] iteration at which the system finished (INT_MAX: running)
-    int *status;       // [nsys] final state (kConverged, kBreakdown, kMaxIter)
-    int *iters;        // [nsys]
-    double *hist;      // [nsys][hist_cap] or null
-    int hist_cap;
-    int max_iter;
-    double tol;
-    int quirk;
-    int x0_guard;      // restart a system from x0 = 0 when <r0,r0> > <b,b>
-    int *x0_rejected;  // [nsys] 1 where the guard restarted the system
-    // DIA storage (dmax > 0): a(row, row + doff[sy*dmax + d]) at dval[d*dpad + row]
-    const double *dval;
-    const int *doff;
-    int dmax;
-    long long dpad;
-    GridSync *sync;
-};
 
 constexpr int kNoDiag = 1 << 30;  // offset of an unused diagonal slot: never inside a system
 
@@ -500,6 +467,12 @@ struct cfm_cg_batch_plan {
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     int sub = 4, grid = 0;
+    // the resident kernel, its grid and rounds (null where it does not apply); resident: in use
+    BatchResidentFn res_fn = nullptr;
+    int res_grid = 0, res_rounds = 0;
+    TeamSlot *res_slots = nullptr;
+    TeamSync *team = nullptr;
+    bool resident = false;
     unsigned long long spin_ticks = 0;
 };
 
@@ -519,7 +492,7 @@ extern "C" void cfm_cg_batch_plan_destroy(cfm_cg_batch_plan *pl) {
     void *ptrs[] = {pl->sys_chunk0, pl->sys_rows, pl->slice_ptr, pl->scol, pl->sval, pl->b, pl->x0, pl->x,
                     pl->r, pl->z, pl->s, pl->pv, pl->w[0], pl->w[1], pl->part, pl->st_alpha, pl->st_delta,
                     pl->hist, pl->fin, pl->status, pl->iters, pl->x0_rejected, pl->features, pl->dval, pl->doff,
-                    pl->sync};
+                    pl->sync, pl->res_slots, pl->team};
     for (void *q : ptrs)
         if (q) (void)hipFree(q);
     if (pl->ev0) (void)hipEventDestroy(pl->ev0);
@@ -539,6 +512,34 @@ static cfm_status batch_configure(cfm_cg_batch_plan *pl, int sub, int grid) {
     const int max_grid = std::min(per_cu * pl->dev.cus, kMaxGrid);
     pl->sub = sub;
     pl->grid = std::max(1, std::min(grid > 0 ? grid : max_grid, max_grid));
+    pl->resident = false;
+    return CFM_OK;
+}
+
+// Puts the resident kernel in use; CFM_ENOTSUP where the plan has none.
+static cfm_status batch_use_resident(cfm_cg_batch_plan *pl) {
+    if (!pl->res_fn) return CFM_ENOTSUP;
+    pl->sub = 1;
+    pl->grid = pl->res_grid;
+    pl->dia_on = false;
+    pl->resident = true;
+    return CFM_OK;
+}
+
+// The resident kernel's schedule, for SELL-64 plans whose systems each fit the chip.  With rounds a
+// workgroup may wait for members still at their previous systems, so a short watchdog keeps one round.
+static cfm_status batch_plan_resident(cfm_cg_batch_plan *pl, int max_width) {
+    int grid = 0, rounds = 0;
+    const BatchResidentFn fn = batch_resident_kernel(max_width, pl->dev, &grid);
+    if (!fn) return CFM_OK;
+    const std::vector<TeamSlot> slots = batch_resident_schedule(pl->h_chunk0, grid, &rounds);
+    if (slots.empty() || (rounds > 1 && pl->p.spin_limit_us > 0)) return CFM_OK;
+    CFM_HIP(hipMalloc((void **)&pl->res_slots, sizeof(TeamSlot) * slots.size()));
+    CFM_HIP(hipMalloc((void **)&pl->team, sizeof(TeamSync)));
+    CFM_HIP(hipMemcpy(pl->res_slots, slots.data(), sizeof(TeamSlot) * slots.size(), hipMemcpyHostToDevice));
+    pl->res_fn = fn;
+    pl->res_grid = grid;
+    pl->res_rounds = rounds;
     return CFM_OK;
 }
 
@@ -735,8 +736,15 @@ extern "C" cfm_status cfm_cg_batch_plan_create(int nsys, const int64_t *sys_row_
         return fail(CFM_EDEVICE);
     const int bt = p->block_threads > 0 ? p->block_threads : 1024;
     if (bt % 256 || bt > 1024) return fail(CFM_FAIL(CFM_EINVAL, "batched CG: block_threads %d", bt));
-    const cfm_status cs = batch_configure(pl, bt / 256, p->grid_blocks);
+    cfm_status cs = batch_configure(pl, bt / 256, p->grid_blocks);
     if (cs != CFM_OK) return fail(cs);
+    if (sell && p->block_threads <= 0 && p->grid_blocks <= 0) {
+        int width = 0;
+        for (long long sl = 0; sl < nslices; ++sl) width = std::max(width, (sp[sl + 1] - sp[sl]) / 64);
+        cs = batch_plan_resident(pl, width);
+        if (cs != CFM_OK) return fail(cs);
+        (void)batch_use_resident(pl);
+    }
     int rate_khz = 0;
     const unsigned long long us = p->spin_limit_us > 0 ? p->spin_limit_us : 10000000ull;
     if (hipDeviceGetAttribute(&rate_khz, hipDeviceAttributeWallClockRate, pl->dev.device) != hipSuccess ||
@@ -817,17 +825,24 @@ static cfm_status batch_run(cfm_cg_batch_plan *pl, int max_iter, double tol, int
     CFM_HIP(hipMemsetAsync(pl->x0_rejected, 0, sizeof(int) * pl->nsys, pl->stream));
     CFM_HIP(hipMemsetD32Async((hipDeviceptr_t)pl->fin, 0x7fffffff, pl->nsys, pl->stream));
     CFM_HIP(hipMemsetAsync(pl->iters, 0, sizeof(int) * pl->nsys, pl->stream));
-    hipLaunchKernelGGL(reset_sync_kernel, dim3(8), dim3(256), 0, pl->stream, pl->sync, pl->spin_ticks, pl->grid);
+    if (pl->resident)
+        hipLaunchKernelGGL(reset_team_kernel, dim3(kMaxTeamGrid / 256), dim3(256), 0, pl->stream, pl->team,
+                           pl->spin_ticks);
+    else
+        hipLaunchKernelGGL(reset_sync_kernel, dim3(8), dim3(256), 0, pl->stream, pl->sync, pl->spin_ticks, pl->grid);
     CFM_HIP(hipGetLastError());
     CFM_HIP(hipEventRecord(pl->ev0, pl->stream));
-    void *args[] = {&A};
-    CFM_HIP(launch_persistent((const void *)batch_kernel(pl->sub), pl->grid, 256 * pl->sub, args, pl->stream, coop));
+    BatchResidentArgs R{A, pl->res_slots, pl->res_rounds, pl->team};
+    void *args[] = {&A}, *rargs[] = {&R};
+    CFM_HIP(launch_persistent(pl->resident ? (const void *)pl->res_fn : (const void *)batch_kernel(pl->sub), pl->grid,
+                              256 * pl->sub, pl->resident ? rargs : args, pl->stream, coop));
     CFM_HIP(hipEventRecord(pl->ev1, pl->stream));
     CFM_HIP(hipEventSynchronize(pl->ev1));
     CFM_HIP(hipEventElapsedTime(ms, pl->ev0, pl->ev1));
-    GridSync hs{};
-    CFM_HIP(hipMemcpy(&hs, pl->sync, sizeof(hs), hipMemcpyDeviceToHost));
-    if (hs.abort) return barrier_timeout("cg batch", *coop);
+    unsigned int aborted = 0;
+    CFM_HIP(hipMemcpy(&aborted, pl->resident ? &pl->team->abort : &pl->sync->abort, sizeof(aborted),
+                      hipMemcpyDeviceToHost));
+    if (aborted) return barrier_timeout("cg batch", *coop);
     return CFM_OK;
 }
 
@@ -880,13 +895,14 @@ extern "C" cfm_status cfm_cg_batch_solve(cfm_cg_batch_plan *pl, int *iters, int 
 // Autotuner.  Screen: time `trial_iters` fixed iterations of the batch for each
 // workgroup shape (1, 2 or 4 sub-blocks of 256 threads), each grid size (1..occupancy
 // workgroups per CU) and each storage the plan holds (SELL-64, and DIA when an auto
-// plan's systems are banded).  Then time full solves (the plan's tol and max_iter,
+// plan's systems are banded), and the resident kernel where the plan has one.  Then time full solves (the plan's tol and max_iter,
 // from the current x0) of the kTuneFinalists fastest and keep the fastest solve: the
 // first iterations, where every system is active, do not show the tail, where the
 // few systems still iterating leave most of the grid waiting at barriers.  With a
 // cache file the winner is stored under a key of device, system count, row count and
 // tolerance, and looked up first.
 constexpr int kTuneFinalists = 3;
+constexpr int kTuneResident = 0;  // in place of a sub-block count: the resident kernel
 
 extern "C" cfm_status cfm_cg_batch_tune(cfm_cg_batch_plan *pl, int trial_iters, const char *cache_path,
                                         int *best_block, int *best_grid) {
@@ -898,6 +914,7 @@ extern "C" cfm_status cfm_cg_batch_tune(cfm_cg_batch_plan *pl, int trial_iters, 
         if (*q == ' ' || *q == '\t') *q = '_';
     const bool have_sell = pl->p.matrix_format != 2, have_dia = pl->dmax > 0;
     auto use = [&](int sub, int grid, bool dia) {
+        if (sub == kTuneResident) return batch_use_resident(pl);
         if ((dia && !have_dia) || (!dia && !have_sell)) return CFM_EINVAL;
         const cfm_status st = batch_configure(pl, sub, grid);
         if (st == CFM_OK) pl->dia_on = dia;
@@ -929,6 +946,13 @@ extern "C" cfm_status cfm_cg_batch_tune(cfm_cg_batch_plan *pl, int trial_iters, 
         float ms;
     };
     std::vector<Cand> cands;
+    if (use(kTuneResident, 0, false) == CFM_OK) {
+        float ms = 0.f;
+        int coop = -1;
+        const cfm_status st = batch_run(pl, trial_iters, 0.0, 0, &ms, &coop);
+        if (st != CFM_OK) return st;
+        cands.push_back({kTuneResident, pl->grid, false, ms});
+    }
     const int subs[] = {1, 2, 4};
     for (int storage = 0; storage < 2; ++storage) {
         const bool dia = storage == 1;

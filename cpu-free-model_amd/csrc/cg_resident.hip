@@ -17,19 +17,11 @@
 
 #include <algorithm>
 
-#include "cg_args.hpp"
+#include "cg_resident.hpp"
 
 namespace cfm {
 
 namespace {
-
-constexpr int kRows = 4;  // rows per thread: a chunk over a sub-block
-constexpr int kSc1 = 16;   // buffer instructions' cache policy bit: past the L2
-
-template <typename T>
-__device__ __forceinline__ T load_through(const T *p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
 
 // This thread's place: chunk c, rows c*1024 + i*256 + t.
 template <int SUB>
@@ -45,80 +37,6 @@ struct Place {
     __device__ __forceinline__ int row(int i) const { return c * kChunk + i * kThreads + t; }
     __device__ __forceinline__ int slice(int i) const { return c * kSlicesPerChunk + i * 4 + (t >> 6); }
 };
-
-// The rows' entries in stored order.  Columns are kept as byte offsets into a vector of XT, -1 beyond
-// a row's end.  The gather is buffer loads (scope bit sc1: past the L2): their range check turns -1
-// into a zero, so all loads go out in one straight line, and they take the offset as it is, where plain loads would hold a 64-bit address for every entry.
-template <typename VT, typename XT, int W>
-struct Entries {
-    VT v[kRows][W];
-    int off[kRows][W];
-
-    template <int SUB>
-    __device__ __forceinline__ void load(const Sell &S, int entries, const Place<SUB> &P) {
-        const auto rc = __builtin_amdgcn_make_buffer_rsrc((void *)S.col, (short)0, entries * 4, 0x00020000);
-        const auto rv =
-            __builtin_amdgcn_make_buffer_rsrc((void *)S.val, (short)0, entries * (int)sizeof(VT), 0x00020000);
-#pragma unroll
-        for (int i = 0; i < kRows; ++i) {
-            int beg = 0, width = 0;
-            if (P.in[i]) {
-                beg = S.slice_ptr[P.slice(i)];
-                width = (S.slice_ptr[P.slice(i) + 1] - beg) >> 6;
-            }
-#pragma unroll
-            for (int j = 0; j < W; ++j) {
-                const int e = beg + 64 * j + (P.t & 63);
-                const int c = __builtin_amdgcn_raw_buffer_load_b32(rc, j < width ? e * 4 : -1, 0, 0);
-                if constexpr (sizeof(VT) == 8)
-                    v[i][j] = __builtin_bit_cast(
-                        VT, __builtin_amdgcn_raw_buffer_load_b64(rv, j < width ? e * 8 : -1, 0, 0));
-                else
-                    v[i][j] = __builtin_bit_cast(
-                        VT, __builtin_amdgcn_raw_buffer_load_b32(rv, j < width ? e * 4 : -1, 0, 0));
-                off[i][j] = j < width && c >= 0 ? c * (int)sizeof(XT) : -1;
-            }
-        }
-    }
-    // x: n elements (a resident system is far below 2 GiB)
-    __device__ __forceinline__ void gather(const XT *x, int n, XT (&g)[kRows][W]) const {
-        const auto rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)x, (short)0, n * (int)sizeof(XT), 0x00020000);
-#pragma unroll
-        for (int i = 0; i < kRows; ++i)
-#pragma unroll
-            for (int j = 0; j < W; ++j)
-                if constexpr (sizeof(XT) == 8)
-                    g[i][j] = __builtin_bit_cast(XT, __builtin_amdgcn_raw_buffer_load_b64(rsrc, off[i][j], 0, kSc1));
-                else
-                    g[i][j] = __builtin_bit_cast(XT, __builtin_amdgcn_raw_buffer_load_b32(rsrc, off[i][j], 0, kSc1));
-    }
-    // The row sum over gathered entries: sell_row's chain.  Entries beyond a row's end are 0 * 0,
-    // which leaves the sum as it is (skipping them instead held a lane mask per entry).
-    __device__ __forceinline__ XT row_sum(int i, const XT (&g)[kRows][W]) const {
-        XT acc = XT(0);
-#pragma unroll
-        for (int j = 0; j < W; ++j) acc = fma((XT)v[i][j], g[i][j], acc);
-        return acc;
-    }
-};
-
-// sub_sum of K values with one pair of workgroup barriers; lds holds K * 4 * SUB doubles.
-template <int SUB, int K>
-__device__ __forceinline__ void sub_sums(double (&v)[K], double *lds) {
-#pragma unroll
-    for (int k = 0; k < K; ++k) v[k] = wave_butterfly(v[k]);
-    __syncthreads();  // lds may still be read from a previous call
-    if ((threadIdx.x & 63) == 0)
-#pragma unroll
-        for (int k = 0; k < K; ++k) lds[k * 4 * SUB + (threadIdx.x >> 6)] = v[k];
-    __syncthreads();
-    const int w0 = (threadIdx.x >> 8) * 4;
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-        const double *l = lds + k * 4 * SUB + w0;
-        v[k] = (l[0] + l[1]) + (l[2] + l[3]);
-    }
-}
 
 // Chunk sums of K per-thread values into part[which[k]].
 template <int SUB, int K>
@@ -202,7 +120,7 @@ __global__ void __launch_bounds__(256 * SUB) cg_standard_resident(CgArgs A) {
     unsigned int epoch = 0;
     const Place<SUB> P(A);
     Entries<double, double, W> M;
-    M.load(A.A64, A.entries, P);
+    M.load(A.A64, P.c, P.t, P.c < A.nchunks, 0);
     double x[kRows], r[kRows], p[kRows], pg[kRows][W];
     double two[2];
     first_residual(A, P, M, x, r, two[0], two[1]);
@@ -296,7 +214,7 @@ __global__ void __launch_bounds__(256 * SUB) cg_pipelined_resident(CgArgs A) {
     unsigned int epoch = 0;
     const Place<SUB> P(A);
     Entries<double, double, W> M;
-    M.load(A.A64, A.entries, P);
+    M.load(A.A64, P.c, P.t, P.c < A.nchunks, 0);
     double x[kRows], r[kRows], z[kRows], s[kRows], p[kRows], w[kRows], g[kRows][W];
     double one[1], two[2];
     first_residual(A, P, M, x, r, two[0], one[0]);
@@ -413,7 +331,7 @@ __global__ void __launch_bounds__(256 * SUB) cg_ir_resident(CgArgs A) {
     unsigned int epoch = 0;
     const Place<SUB> P(A);
     Entries<float, float, W> M;
-    M.load(A.A32, A.entries, P);
+    M.load(A.A32, P.c, P.t, P.c < A.nchunks, 0);
     double thr = 0.0;
     int outer = 0, inner_total = 0, status = CFM_ENOTCONV;
     for (;;) {

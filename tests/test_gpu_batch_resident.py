@@ -1,0 +1,59 @@
+"""The resident batch kernel (a team of workgroups per system, systems in rounds) against the CPU oracle, bit for bit,
+where its teams and rounds can go wrong."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(gpu, orc, systems, tol=0.0, max_iter=6, guard=0, bad=()):
+    srp, rp, col, val = gpu.block_diag(systems)
+    n = int(srp[-1])
+    b = gpu.uniform(5, 0, n) - 0.5
+    x0 = b / 20  # better than zero: all eigenvalues lie in (0, 20)
+    for s in bad:  # guesses far worse than zero
+        x0[srp[s]:srp[s + 1]] = 1e3
+    p = gpu.cg_params(method=gpu.CG_PIPELINED, tol=tol, max_iter=max_iter, x0_guard=guard)
+    with gpu.CgBatchPlan(srp, rp, col, val, p) as plan:
+        plan.set_rhs(b)
+        plan.set_x0(x0)
+        for _ in range(2):  # the second solve starts over
+            _, iters, _, hist, t = plan.solve(hist_cap=max_iter + 1)
+            x = plan.x()
+        rejected = plan.x0_rejected()
+    for s, (r, c, v) in enumerate(systems):
+        sl = slice(srp[s], srp[s + 1])
+        start = np.zeros(sl.stop - sl.start) if s in bad and guard else x0[sl]
+        _, ox, ohist, oit = orc.cg(orc.Csr(r, c, v), b[sl], x0=start, tol=tol, max_iter=max_iter, variant="pipelined")
+        assert iters[s] == oit and rejected[s] == (1 if guard and s in bad else 0)
+        assert np.array_equal(x[sl], ox) and np.array_equal(hist[s, :oit + 1], ohist)
+    return t
+
+
+def test_batch_resident_sizes(gpu, orc):
+    """One row, one chunk and one row more, rows of 3 and of 7 entries, in one round."""
+    systems = [gpu.tridiag(n, 1 + n) for n in (2, 63, 1024, 1025, 2047, 5000)]
+    t = _check(gpu, orc, systems)
+    assert t["block_threads"] == 256
+    _check(gpu, orc, systems + [gpu.poisson3d(9, 10, 11), gpu.poisson3d(1, 1, 1), gpu.poisson3d(16, 16, 16)])
+
+
+def test_batch_resident_rounds(gpu, orc):
+    """More chunks than workgroups: teams of several rounds, one of them as large as half the chip."""
+    systems = [gpu.poisson3d(8 + i % 7, 20, 30) for i in range(60)] + [gpu.poisson3d(64, 64, 64)] * 3
+    _check(gpu, orc, systems, tol=1e-6, max_iter=400)
+
+
+def test_batch_resident_largest_system(gpu, orc):
+    """A system of exactly 512 chunks, and one chunk more (the general kernel's)."""
+    small = gpu.tridiag(3000, 4)
+    t = _check(gpu, orc, [small, gpu.tridiag(524288, 3), small])
+    assert t["block_threads"] == 256
+    t = _check(gpu, orc, [small, gpu.tridiag(1048577, 3)])
+    assert t["block_threads"] == 1024
+
+
+@pytest.mark.parametrize("tol,max_iter", [(1e-7, 200), (0.0, 3)])
+def test_batch_resident_guard(gpu, orc, tol, max_iter):
+    systems = [gpu.poisson3d(10, 11, 12), gpu.poisson3d(20, 9, 14), gpu.tridiag(4000, 9)]
+    _check(gpu, orc, systems, tol=tol, max_iter=max_iter, guard=1, bad=(1,))
