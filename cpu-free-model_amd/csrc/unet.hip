@@ -15,7 +15,7 @@
 //
 // Backward data is the same kernel with the weights flipped in space and
 // transposed in channels; backward weights is a split-K MFMA GEMM over point
-// slabs (one workgroup per tap and slab, point blocks staged transposed in
+// slabs (one workgroup per slab, all taps, point blocks staged transposed in
 // LDS) followed by a fixed-order reduction of the slab partials.
 #include <hip/hip_runtime.h>
 
@@ -37,13 +37,6 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ float bf2f(bf16 v) { return (float)v; }
 __device__ __forceinline__ bf16 f2bf(float v) { return (bf16)v; }  // round to nearest even
-
-__device__ __forceinline__ int tap_off(int tap, int &dz, int &dy, int &dx) {
-    dz = tap / 9 - 1;
-    dy = (tap / 3) % 3 - 1;
-    dx = tap % 3 - 1;
-    return 0;
-}
 
 // ------------------------------------------------------------- conv fwd ---
 // Y = conv3x3x3(X) + bias, optional ReLU.  W is [Cout][Kp] BF16 (k = tap*Cin+ci,
@@ -298,174 +291,34 @@ __global__ void __launch_bounds__(64 * NW) conv3_fwd_xacc_kernel(const bf16 *__r
 }
 
 // ------------------------------------------------------ conv weight grad ---
-// partial[slab][co][k] = sum over points of slab: dZ[p][co] * Xs[p][k]
-// (M = 16 output channels, N = 16 k, K = 32 points per MFMA).  Each
-// wavefront owns one (co tile, k tile) pair over one slab of `slab` points.
-__global__ void __launch_bounds__(256) conv3_wgrad_kernel(const bf16 *__restrict__ X, int Cin,
-                                                          const bf16 *__restrict__ dZ, int Cout, int Kp,
-                                                          float *__restrict__ partial, int n, int npts, int slab,
-                                                          int ntile_k) {
-    const int lane = threadIdx.x & 63;
-    const int wid = blockIdx.x * 4 + (threadIdx.x >> 6);
-    const int ntile = (Cout / 16) * ntile_k;
-    const int s = blockIdx.y;
-    if (wid >= ntile) return;
-    const int mt = wid / ntile_k, kt = wid - mt * ntile_k;
-    const int nl = lane & 15, g = lane >> 4;
-    const int co = mt * 16 + nl;         // A row (lane's m)
-    const int kcol = kt * 16 + nl;       // B column (lane's n)
-    const int K = 27 * Cin;
-    int tap = 0, ci = 0, dz = 0, dy = 0, dx = 0;
-    const bool kvalid = kcol < K;
-    if (kvalid) {
-        tap = kcol / Cin;
-        ci = kcol - tap * Cin;
-        tap_off(tap, dz, dy, dx);
-    }
-    f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
-    const int pbeg = s * slab, pend = min(npts, pbeg + slab);
-    for (int pb = pbeg; pb < pend; pb += 32) {
-        bf16x8 av, bv;
-        // coordinates of the lane's first point, then stepped along x with carries
-        const int p8 = pb + 8 * g;
-        int x = p8 % n, y = (p8 / n) % n, z = (p8 / (n * n)) % n, b = p8 / (n * n * n);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const int p = p8 + j;
-            bf16 a = (bf16)0.0f, bb = (bf16)0.0f;
-            if (p < pend) {
-                a = dZ[(size_t)p * Cout + co];
-                if (kvalid) {
-                    const int zz = z + dz, yy = y + dy, xx = x + dx;
-                    if (zz >= 0 && zz < n && yy >= 0 && yy < n && xx >= 0 && xx < n)
-                        bb = X[((((size_t)b * n + zz) * n + yy) * n + xx) * Cin + ci];
-                }
-            }
-            av[j] = a;
-            bv[j] = bb;
-            if (++x == n) {
-                x = 0;
-                if (++y == n) {
-                    y = 0;
-                    if (++z == n) {
-                        z = 0;
-                        ++b;
-                    }
-                }
-            }
-        }
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bv, acc, 0, 0, 0);
-    }
-    // D[4g+i][nl] = dW[mt*16 + 4g + i][kt*16 + nl]
-    float *out = partial + (size_t)s * Cout * Kp;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) out[(size_t)(mt * 16 + 4 * g + i) * Kp + kt * 16 + nl] = acc[i];
-}
-
-// LDS-staged weight gradient for one tap: workgroup (tap, slab) computes
-// partial[slab][co][tap*CIN + ci] for all co < COUT, ci < CIN.  Per block of
-// 64 consecutive points it stages dZ (64 x COUT) and the tap-shifted input
-// (64 x CIN, zero where the neighbour leaves the grid) transposed in LDS,
-// [channel][point], so each lane's 8 consecutive points of one channel -- an
-// MFMA fragment along the point (K) dimension -- are one ds_read_b128.  The
-// (co tile, ci tile) pairs are spread over the four wavefronts.  The tap-26
-// workgroups also zero the padding columns [27*CIN, Kp).
-template <int CIN, int COUT>
-__global__ void __launch_bounds__(256) conv3_wgrad_lds_kernel(const bf16 *__restrict__ X, const bf16 *__restrict__ dZ,
-                                                              int Kp, float *__restrict__ partial, int n, int npts,
-                                                              int slab) {
-    constexpr int PB = 64;  // points per staged block
-    constexpr int MT = COUT / 16, KT = CIN / 16, T = MT * KT, TW = (T + 3) / 4;
-    static_assert(CIN % 16 == 0 && COUT % 16 == 0, "shape");
-    __shared__ __attribute__((aligned(16))) bf16 dzT[COUT * PB];
-    __shared__ __attribute__((aligned(16))) bf16 xT[CIN * PB];
-    const int tap = blockIdx.x, s = blockIdx.y;
-    const int dz = tap / 9 - 1, dy = (tap / 3) % 3 - 1, dx = tap % 3 - 1;
-    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int nl = lane & 15, g = lane >> 4;
-    f32x4 acc[TW];
-#pragma unroll
-    for (int i = 0; i < TW; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const bf16x8 zero8 = {(bf16)0.0f, (bf16)0.0f, (bf16)0.0f, (bf16)0.0f,
-                          (bf16)0.0f, (bf16)0.0f, (bf16)0.0f, (bf16)0.0f};
-    const int pbeg = s * slab, pend = min(npts, pbeg + slab);
-    for (int pb = pbeg; pb < pend; pb += PB) {
-        // stage dZ[pb..pb+63][*] and the tap-shifted X[pb..pb+63][*], transposed
-        for (int v = threadIdx.x; v < PB * (COUT / 8); v += 256) {
-            const int j = v / (COUT / 8), c8 = v % (COUT / 8);
-            const int p = pb + j;
-            const bf16x8 val = p < pend ? *reinterpret_cast<const bf16x8 *>(dZ + (size_t)p * COUT + 8 * c8) : zero8;
-#pragma unroll
-            for (int i = 0; i < 8; ++i) dzT[(8 * c8 + i) * PB + j] = val[i];
-        }
-        for (int v = threadIdx.x; v < PB * (CIN / 8); v += 256) {
-            const int j = v / (CIN / 8), c8 = v % (CIN / 8);
-            const int p = pb + j;
-            bf16x8 val = zero8;
-            if (p < pend) {
-                const int x = p % n, y = (p / n) % n, z = (p / (n * n)) % n, b = p / (n * n * n);
-                const int xx = x + dx, yy = y + dy, zz = z + dz;
-                if (xx >= 0 && xx < n && yy >= 0 && yy < n && zz >= 0 && zz < n)
-                    val = *reinterpret_cast<const bf16x8 *>(
-                        X + ((((size_t)b * n + zz) * n + yy) * n + xx) * CIN + 8 * c8);
-            }
-#pragma unroll
-            for (int i = 0; i < 8; ++i) xT[(8 * c8 + i) * PB + j] = val[i];
-        }
-        __syncthreads();
-#pragma unroll
-        for (int i = 0; i < TW; ++i) {
-            const int t = w + 4 * i;
-            if (t < T) {  // uniform per wavefront
-                const int mt = t / KT, kt = t % KT;
-#pragma unroll
-                for (int h = 0; h < PB / 32; ++h) {
-                    const bf16x8 av = *reinterpret_cast<const bf16x8 *>(&dzT[(mt * 16 + nl) * PB + 32 * h + 8 * g]);
-                    const bf16x8 bv = *reinterpret_cast<const bf16x8 *>(&xT[(kt * 16 + nl) * PB + 32 * h + 8 * g]);
-                    acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bv, acc[i], 0, 0, 0);
-                }
-            }
-        }
-        __syncthreads();  // the staged blocks are rewritten next
-    }
-    // D[4g+i][nl] = dW[mt*16 + 4g + i][tap*CIN + kt*16 + nl]
-    float *out = partial + (size_t)s * COUT * Kp;
-#pragma unroll
-    for (int i = 0; i < TW; ++i) {
-        const int t = w + 4 * i;
-        if (t < T) {
-            const int mt = t / KT, kt = t % KT;
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                out[(size_t)(mt * 16 + 4 * g + r) * Kp + tap * CIN + kt * 16 + nl] = acc[i][r];
-        }
-    }
-    if (tap == 26)
-        for (int e = threadIdx.x; e < COUT * (Kp - 27 * CIN); e += 256) {
-            const int co = e / (Kp - 27 * CIN), k = 27 * CIN + e % (Kp - 27 * CIN);
-            out[(size_t)co * Kp + k] = 0.f;
-        }
-}
-
-// Weight gradient for every tap at once, for grids whose x rows tile 64-point
-// blocks (n in 16, 32, 64): workgroup s computes partial[s][co][tap*CIN + ci]
-// over its slab.  Per block of 64 points (R = 64/n whole x rows of one plane)
-// it stages dZ once, transposed [co][point], and the 3 x (R+2) input rows
-// around the block once, transposed [ci][x] with a zero halo column at each
-// end (x = -1 and x = n): the tap-shifted input of every tap is then a window
-// of those rows, so nothing is staged per tap.  Wavefront w owns the taps of
-// WROWS (dz, dy) rows; a lane's B fragment (8 consecutive points of one input
-// channel, shifted by dx) comes from two aligned 16-byte LDS reads: dx = -1 is
-// the first, dx = +1 the dwords 1..4, dx = 0 a 2-byte byte-align of the pair.
-// Input channels below 16 are padded with zero rows (the first layer's 8).
+// Weight and bias gradients, every tap at once: workgroup s computes
+// partial[s][co][tap*CIN + ci] (and the sums of dZ, partial[s][COUT*Kp + co]) over its blocks.
+// A block is 64 points: R rows of at most 64 points of one plane, each padded to
+// a multiple of 8 (rows longer than 64 points go in segments), with zero dZ where
+// a point lies outside.  Per block it stages dZ once, transposed [co][point], and
+// the 3 x (R+2) input rows around the block once, transposed [ci][x] with the
+// columns x0 - 1 and x0 + W8 at the ends: the tap-shifted input of every tap is
+// then a window of those rows, so nothing is staged per tap.  Wavefront w owns
+// the taps of WROWS (dz, dy) rows; a lane's B fragment (8 consecutive points of
+// one input channel, shifted by dx) comes from two aligned 16-byte LDS reads:
+// dx = -1 is the first, dx = +1 the dwords 1..4, dx = 0 a 2-byte byte-align of
+// the pair.  Input channels below 16 are padded with zero rows (the first layer's
+// 8).  The bias gradient is one more product, with a B fragment of ones.
 // KS > 1 splits the input channels over KS workgroups per slab (blockIdx.y):
 // each stages and computes CIN / KS of them, which keeps the accumulators of
-// the wide layers in registers.
+// the wide layers in registers.  Bound by staging (loads and transposing LDS stores) with
+// two workgroups a CU to overlap it; other row lengths than 16, 32 and 64 went through a kernel
+// that staged the input anew for each of the 27 taps.
+struct WgradShape {
+    int n, nblk, per_slab;  // points along an edge; blocks, and blocks a workgroup takes
+    int w8, rows, nyb, nseg;  // a row's padded points, rows of a block, blocks along y and x
+    float inv_pairs;          // 1 / (w8 / 2 + 1)
+};
+
 template <int CIN, int COUT, int WROWS, int KS = 1>
 __global__ void __launch_bounds__(64 * 9 / WROWS) conv3_wgrad_rows_kernel(const bf16 *__restrict__ Xg,
                                                                         const bf16 *__restrict__ dZ, int Kp,
-                                                                        float *__restrict__ partial, int n, int npts,
-                                                                        int slab) {
+                                                                        float *__restrict__ partial, WgradShape S) {
     constexpr int CINX = CIN;            // channels per point of the input tensor
     constexpr int CW = CIN / KS;         // input channels of this workgroup
     constexpr int CINP = CW < 16 ? 16 : CW;
@@ -476,21 +329,23 @@ __global__ void __launch_bounds__(64 * 9 / WROWS) conv3_wgrad_rows_kernel(const 
     constexpr int DS = 72;  // dZ row stride (64 points + 8: spreads the 16 rows of a fragment over the banks)
     static_assert(CINP % 16 == 0 && COUT % 16 == 0 && CW % 8 == 0 && 9 % WROWS == 0, "shape");
     extern __shared__ __attribute__((aligned(16))) bf16 wg_lds[];
-    const int R = 64 / n, W = n + 8, ROWS = 3 * (R + 2);
+    const int n = S.n, W8 = S.w8, R = S.rows, W = W8 + 8, ROWS = 3 * (R + 2);
     bf16 *dzT = wg_lds;                 // [COUT][DS]
-    bf16 *xT = wg_lds + COUT * DS;      // [ROWS][CINP][W], x + 1 stored at column x + 1
+    bf16 *xT = wg_lds + COUT * DS;      // [ROWS][CINP][W], x stored at column x - x0 + 1
     const int s = blockIdx.x;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int nl = lane & 15, g = lane >> 4;
     const bf16x8 zero8 = {(bf16)0.0f, (bf16)0.0f, (bf16)0.0f, (bf16)0.0f,
                           (bf16)0.0f, (bf16)0.0f, (bf16)0.0f, (bf16)0.0f};
+    const bf16x8 one8 = {(bf16)1.0f, (bf16)1.0f, (bf16)1.0f, (bf16)1.0f,
+                         (bf16)1.0f, (bf16)1.0f, (bf16)1.0f, (bf16)1.0f};
     if (CW < CINP) {  // padded input channels: zero once, never overwritten
         for (int v = threadIdx.x; v < ROWS * (CINP - CW) * W; v += NTH) {
             const int c = CW + (v / W) % (CINP - CW), r = v / (W * (CINP - CW));
             xT[((size_t)r * CINP + c) * W + v % W] = (bf16)0.0f;
         }
     }
-    f32x4 acc[WROWS][3][MT][KT];
+    f32x4 acc[WROWS][3][MT][KT], accb[MT];
 #pragma unroll
     for (int a = 0; a < WROWS; ++a)
 #pragma unroll
@@ -499,33 +354,52 @@ __global__ void __launch_bounds__(64 * 9 / WROWS) conv3_wgrad_rows_kernel(const 
             for (int m = 0; m < MT; ++m)
 #pragma unroll
                 for (int k = 0; k < KT; ++k) acc[a][d][m][k] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const int n2 = n * n, n3 = n2 * n;
-    const int pbeg = s * slab, pend = min(npts, pbeg + slab);
-    for (int pb = pbeg; pb < pend; pb += 64) {
-        const int b = pb / n3, rem = pb - b * n3;
-        const int z = rem / n2, y0 = (rem / n) % n;
-        // stage dZ of the 64 points, transposed: two points per thread, so each LDS store
+#pragma unroll
+    for (int m = 0; m < MT; ++m) accb[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // this lane's first point in each of the two K steps: its row in the block and its column (a
+    // group beyond the last row multiplies zeros of dZ with any staged row)
+    int rq[2], xg[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const int q = 32 * h + 8 * g;
+        rq[h] = q / W8;
+        xg[h] = q - rq[h] * W8;
+        if (rq[h] >= R) rq[h] = 0;
+    }
+    const int blk_end = min(S.nblk, (s + 1) * S.per_slab);
+    for (int blk = s * S.per_slab; blk < blk_end; ++blk) {
+        int u = blk;
+        const int x0 = (u % S.nseg) * 64;
+        u /= S.nseg;
+        const int y0 = (u % S.nyb) * R;
+        u /= S.nyb;
+        const int z = u % n, b = u / n;
+        // stage dZ of the block, transposed: two points per thread, so each LDS store
         // writes one channel's pair of neighbouring points (4 bytes)
         for (int v = threadIdx.x; v < 32 * (COUT / 8); v += NTH) {
             const int j = 2 * (v / (COUT / 8)), c8 = v % (COUT / 8);
-            const u16x8 a0 = __builtin_bit_cast(u16x8, *reinterpret_cast<const bf16x8 *>(dZ + (size_t)(pb + j) * COUT + 8 * c8));
-            const u16x8 a1 =
-                __builtin_bit_cast(u16x8, *reinterpret_cast<const bf16x8 *>(dZ + (size_t)(pb + j + 1) * COUT + 8 * c8));
+            const int rr = j / W8, x = x0 + j - rr * W8, y = y0 + rr;
+            const bool row = rr < R && y < n;
+            const bf16 *p = dZ + ((((size_t)b * n + z) * n + y) * n + x) * COUT + 8 * c8;
+            u16x8 a0 = __builtin_bit_cast(u16x8, zero8), a1 = a0;
+            if (row && x < n) a0 = *reinterpret_cast<const u16x8 *>(p);
+            if (row && x + 1 < n) a1 = *reinterpret_cast<const u16x8 *>(p + COUT);
 #pragma unroll
             for (int i = 0; i < 8; ++i)
                 *reinterpret_cast<unsigned *>(&dzT[(8 * c8 + i) * DS + j]) = (unsigned)a0[i] | ((unsigned)a1[i] << 16);
         }
-        // stage the 3 x (R+2) input rows around the block, transposed, x = -1 .. n (n + 2 columns,
-        // two per thread as above)
-        for (int v = threadIdx.x; v < ROWS * (n / 2 + 1) * (CW / 8); v += NTH) {
-            const int c8 = v % (CW / 8);
-            const int xj = 2 * ((v / (CW / 8)) % (n / 2 + 1));
-            const int r = v / ((CW / 8) * (n / 2 + 1));
-            const int zz = z + r / (R + 2) - 1, yy = y0 + r % (R + 2) - 1;
+        // stage the 3 x (R+2) input rows around the block, transposed, x0 - 1 .. x0 + W8 (two
+        // columns per thread as above)
+        for (int v = threadIdx.x; v < ROWS * (W8 / 2 + 1) * (CW / 8); v += NTH) {
+            const int c8 = v % (CW / 8), pr = v / (CW / 8);
+            const int r = (int)(((float)pr + 0.5f) * S.inv_pairs);  // pr / (W8/2 + 1), exact below 2^20
+            const int xj = 2 * (pr - r * (W8 / 2 + 1));
+            const int rz = r >= 2 * (R + 2) ? 2 : r >= R + 2 ? 1 : 0;
+            const int zz = z + rz - 1, yy = y0 + r - rz * (R + 2) - 1;
             u16x8 a[2];
 #pragma unroll
             for (int e = 0; e < 2; ++e) {
-                const int xx = xj + e - 1;
+                const int xx = x0 + xj + e - 1;
                 bf16x8 val = zero8;
                 if (xx >= 0 && xx < n && yy >= 0 && yy < n && zz >= 0 && zz < n)
                     val = *reinterpret_cast<const bf16x8 *>(X + ((((size_t)b * n + zz) * n + yy) * n + xx) * CINX + 8 * c8);
@@ -540,18 +414,22 @@ __global__ void __launch_bounds__(64 * 9 / WROWS) conv3_wgrad_rows_kernel(const 
 #pragma unroll
         for (int h = 0; h < 2; ++h) {  // two K steps of 32 points
             const int q = 32 * h + 8 * g;  // this lane's first point in the block
-            const int rq = q / n, xg = q % n;
             bf16x8 av[MT];
 #pragma unroll
             for (int m = 0; m < MT; ++m) av[m] = *reinterpret_cast<const bf16x8 *>(&dzT[(m * 16 + nl) * DS + q]);
+            if (w == 0) {
+#pragma unroll
+                for (int m = 0; m < MT; ++m)
+                    accb[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[m], one8, accb[m], 0, 0, 0);
+            }
 #pragma unroll
             for (int a = 0; a < WROWS; ++a) {
                 const int rw = w * WROWS + a;  // (dz, dy) row index 0..8
                 const int dz = rw / 3, dy = rw % 3;  // offsets + 1
-                const int r = dz * (R + 2) + rq + dy;
+                const int r = dz * (R + 2) + rq[h] + dy;
 #pragma unroll
                 for (int k = 0; k < KT; ++k) {
-                    const bf16 *src = &xT[((size_t)r * CINP + k * 16 + nl) * W + xg];
+                    const bf16 *src = &xT[((size_t)r * CINP + k * 16 + nl) * W + xg[h]];
                     const bf16x8 lo = *reinterpret_cast<const bf16x8 *>(src);
                     const bf16x8 hi = *reinterpret_cast<const bf16x8 *>(src + 8);
                     typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
@@ -574,7 +452,7 @@ __global__ void __launch_bounds__(64 * 9 / WROWS) conv3_wgrad_rows_kernel(const 
         __syncthreads();  // the staged rows are rewritten next
     }
     // D[4g+i][nl] = dW[m*16 + 4g + i][tap*CIN + k*16 + nl], tap = 9 dz + 3 dy + dx (offsets + 1)
-    float *out = partial + (size_t)s * COUT * Kp;
+    float *out = partial + (size_t)s * COUT * (Kp + 1);
 #pragma unroll
     for (int a = 0; a < WROWS; ++a) {
         const int rw = w * WROWS + a;
@@ -593,31 +471,42 @@ __global__ void __launch_bounds__(64 * 9 / WROWS) conv3_wgrad_rows_kernel(const 
                 }
         }
     }
-    if (blockIdx.y == 0)
-    for (int e = threadIdx.x; e < COUT * (Kp - 27 * CIN); e += NTH) {  // the zero-padded K tail
-        const int co = e / (Kp - 27 * CIN), k = 27 * CIN + e % (Kp - 27 * CIN);
-        out[(size_t)co * Kp + k] = 0.f;
+    // (the K tail [27 CIN, Kp) is left as it is: nothing reads it)
+    if (w == 0 && blockIdx.y == 0 && nl == 0) {
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) out[(size_t)COUT * Kp + m * 16 + 4 * g + i] = accb[m][i];
     }
 }
 
-// out[i] = sum_s partial[s][i] (fixed order s = 0, 1, ...), i < count.  Eight
-// loads are issued before their eight in-order adds, so the memory latency is
+// The slabs' sums, part[s][i] in the fixed order s = 0, 1, ..., for i < COUT (Kp + 1), taken
+// from the kernel layout (co, k = tap*Cin + ci; then the bias) to the master order [Cout][Cin_real][27]
+// and [Cout].  Eight loads are issued before their eight in-order adds, so the memory latency is
 // paid once per eight slabs instead of once per slab.
-__global__ void reduce_slabs_kernel(const float *__restrict__ partial, int nslab, size_t count,
-                                    float *__restrict__ out) {
-    const size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
+__global__ void reduce_slabs_kernel(const float *__restrict__ part, int nslab, int Cout, int Cin_real, int Cin, int Kp,
+                                    float *__restrict__ g, float *__restrict__ gb) {
+    const int count = Cout * (Kp + 1);
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= count) return;
+    const bool bias = i >= Cout * Kp;
+    const int co = i / Kp, k = i - co * Kp;
+    const int tap = k / Cin, ci = k - tap * Cin;
+    if (!bias && (tap >= 27 || ci >= Cin_real)) return;  // the K tail, padded input channels
     float a = 0.f;
     int s = 0;
     for (; s + 8 <= nslab; s += 8) {
         float v[8];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = partial[(size_t)(s + j) * count + i];
+        for (int j = 0; j < 8; ++j) v[j] = part[(size_t)(s + j) * count + i];
 #pragma unroll
         for (int j = 0; j < 8; ++j) a += v[j];
     }
-    for (; s < nslab; ++s) a += partial[(size_t)s * count + i];
-    out[i] = a;
+    for (; s < nslab; ++s) a += part[(size_t)s * count + i];
+    if (bias)
+        gb[i - Cout * Kp] = a;
+    else
+        g[((size_t)co * Cin_real + ci) * 27 + tap] = a;
 }
 
 // First pass of a two-pass slab reduction: part p of P sums slabs
@@ -670,38 +559,6 @@ __global__ void __launch_bounds__(1024) reduce_rows_kernel(const float *__restri
         __syncthreads();
     }
     if (t == 0) out[blockIdx.x] = sh[0];
-}
-
-// per-slab channel sums of dZ (bias gradient), partial[c][slab] (rows for reduce_rows_kernel).  256 threads
-// per slab: thread t < R*C (R = 256 / C rows at a time) owns channel t % C and
-// rows t / C, t / C + R, ... of the slab, so each pass reads 256 consecutive
-// values; the R row-partials of a channel are then added in row order.
-__global__ void __launch_bounds__(256) chan_sum_kernel(const bf16 *__restrict__ dZ, int C, int npts, int slab,
-                                                       float *__restrict__ partial) {
-    __shared__ float red[256];
-    const int s = blockIdx.x, t = threadIdx.x;
-    const int R = 256 / C;  // C <= 256
-    const int pbeg = s * slab, pend = min(npts, pbeg + slab);
-    float a = 0.f;
-    if (t < R * C) {
-        const int c = t % C;
-        int p = pbeg + t / C;
-        for (; p + 7 * R < pend; p += 8 * R) {  // eight loads in flight, adds in row order
-            float v[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) v[j] = bf2f(dZ[(size_t)(p + j * R) * C + c]);
-#pragma unroll
-            for (int j = 0; j < 8; ++j) a += v[j];
-        }
-        for (; p < pend; p += R) a += bf2f(dZ[(size_t)p * C + c]);
-    }
-    red[t] = a;
-    __syncthreads();
-    if (t < C) {
-        float v = 0.f;
-        for (int r = 0; r < R; ++r) v += red[r * C + t];
-        partial[(size_t)t * gridDim.x + s] = v;
-    }
 }
 
 // --------------------------------------------------------- elementwise ----
@@ -911,24 +768,24 @@ __global__ void adam_kernel(float *__restrict__ w, const float *__restrict__ g, 
 
 // FP32 master conv weights [Cout][Cin_real][27] -> forward layout [Cout][Kp] (k = tap*Cin + ci)
 // and backward-data layout [Cin][Kp_t] (k = tap'*Cout + co, tap' = 26 - tap), BF16
-__global__ void pack_weights_kernel(const float *__restrict__ w, int Cout, int Cin_real, int Cin, int Kp,
-                                    int Kp_t, bf16 *__restrict__ Wf, bf16 *__restrict__ Wt) {
+// (the padding beyond 27 Cin and 27 Cout was cleared when the arrays were made); every layer in one
+// launch, layer blockIdx.y
+constexpr int kNConv = 10;
+struct PackTable {
+    struct Layer {
+        const float *w;
+        bf16 *Wf, *Wt;
+        int Cout, Cin_real, Cin, Kp, Kp_t;
+    } layer[kNConv];
+};
+__global__ void pack_weights_kernel(PackTable T) {
+    const PackTable::Layer &L = T.layer[blockIdx.y];
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const int total = Cout * Cin * 27;
-    if (i >= total) return;
-    const int tap = i % 27, ci = (i / 27) % Cin, co = i / (27 * Cin);
-    const float v = ci < Cin_real ? w[((size_t)co * Cin_real + ci) * 27 + tap] : 0.f;
-    Wf[(size_t)co * Kp + tap * Cin + ci] = f2bf(v);
-    if (Wt) Wt[(size_t)ci * Kp_t + (26 - tap) * Cout + co] = f2bf(v);
-}
-
-// weight-gradient layout [Cout][Kp] (k = tap*Cin + ci) -> master order [Cout][Cin_real][27]
-__global__ void unpack_wgrad_kernel(const float *__restrict__ gk, int Cout, int Cin_real, int Cin, int Kp,
-                                    float *__restrict__ g) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= Cout * Cin_real * 27) return;
-    const int tap = i % 27, ci = (i / 27) % Cin_real, co = i / (27 * Cin_real);
-    g[i] = gk[(size_t)co * Kp + tap * Cin + ci];
+    if (i >= L.Cout * L.Cin * 27) return;
+    const int tap = i % 27, ci = (i / 27) % L.Cin, co = i / (27 * L.Cin);
+    const float v = ci < L.Cin_real ? L.w[((size_t)co * L.Cin_real + ci) * 27 + tap] : 0.f;
+    L.Wf[(size_t)co * L.Kp + tap * L.Cin + ci] = f2bf(v);
+    if (L.Wt) L.Wt[(size_t)ci * L.Kp_t + (26 - tap) * L.Cout + co] = f2bf(v);
 }
 
 }  // namespace unet
@@ -943,7 +800,6 @@ namespace {
 struct ConvSpec {
     int cin_real, cin, cout, level;
 };
-constexpr int kNConv = 10;
 constexpr ConvSpec kConv[kNConv] = {
     {2, 8, 16, 0},   {16, 16, 16, 0},  // encoder level 1 (input padded to 8 channels)
     {16, 16, 32, 1}, {32, 32, 32, 1},  // encoder level 2
@@ -963,6 +819,26 @@ size_t param_count() {
     return c + kHeadIn + 1;
 }
 
+// Blocks of 64 points of a layer's weight gradient, and the workgroups that share them: up to 512, two
+// a CU.  Fewer leave CUs idle (the deep levels had 4 to 32 when a workgroup took 4096 points), more write
+// and re-read more partials than they save.  Training steps, ms, for 128 / 256 / 512 / 1024 / 2048
+// workgroups: 4 x 64^3 3.75, 2.76, 2.59, 2.63, 2.95; 8 x 36^3 2.08, 1.71, 1.64, 1.65, 1.84; 16 x 12^3
+// 0.80, 0.70, 0.71, 0.71, 0.71 (4096 points each: 4.19 at 4 x 64^3).
+WgradShape wgrad_shape(int n, int batch, int *nslab) {
+    WgradShape S;
+    S.n = n;
+    S.w8 = n >= 64 ? 64 : (n + 7) / 8 * 8;
+    S.rows = 64 / S.w8;
+    S.nyb = (n + S.rows - 1) / S.rows;
+    S.nseg = (n + 63) / 64;
+    S.nblk = batch * n * S.nyb * S.nseg;
+    S.inv_pairs = 1.0f / (float)(S.w8 / 2 + 1);
+    const int most = 512;
+    S.per_slab = (S.nblk + most - 1) / most;
+    *nslab = (S.nblk + S.per_slab - 1) / S.per_slab;
+    return S;
+}
+
 inline dim3 blocks_for(size_t count, int threads = 256) { return dim3((unsigned)((count + threads - 1) / threads)); }
 
 }  // namespace
@@ -977,11 +853,8 @@ struct cfm_unet {
     size_t woff[kNConv], boff[kNConv], head_off = 0;
     bf16 *Wf[kNConv] = {}, *Wt[kNConv] = {};
     int Kp[kNConv], Kpt[kNConv];
-    float *gk = nullptr;  // weight gradient in kernel layout (largest layer)
     float *rtmp = nullptr;  // two-pass slab reduction: [kReduceParts][largest layer]
     float *partial = nullptr;
-    size_t partial_cap = 0;
-    int slab = 4096;
     // activations
     bf16 *X0 = nullptr, *A0 = nullptr, *S1 = nullptr, *Q1 = nullptr, *A2 = nullptr, *S2 = nullptr, *Q2 = nullptr,
          *A4 = nullptr, *A5 = nullptr, *U2 = nullptr, *A6 = nullptr, *A7 = nullptr, *U1 = nullptr, *A8 = nullptr,
@@ -1056,14 +929,13 @@ extern "C" cfm_status cfm_unet_create(int n, int batch, cfm_unet **out) {
     for (int i = 0; i < kNConv; ++i) {
         A(&u->Wf[i], 2 * (size_t)kConv[i].cout * u->Kp[i]);
         if (i > 0) A(&u->Wt[i], 2 * (size_t)kConv[i].cin * u->Kpt[i]);
-        max_wk = std::max(max_wk, (size_t)kConv[i].cout * u->Kp[i]);
-        const size_t nslab = (u->P[kConv[i].level] + u->slab - 1) / u->slab;
-        max_partial = std::max(max_partial, nslab * kConv[i].cout * u->Kp[i]);
+        max_wk = std::max(max_wk, (size_t)kConv[i].cout * (u->Kp[i] + 1));
+        int nslab;
+        wgrad_shape(n >> kConv[i].level, batch, &nslab);
+        max_partial = std::max(max_partial, (size_t)nslab * kConv[i].cout * (u->Kp[i] + 1));
     }
-    A(&u->gk, 4 * max_wk);
     A(&u->rtmp, 4 * kReduceParts * max_wk);
     A(&u->partial, 4 * max_partial);
-    u->partial_cap = max_partial;
     const size_t P1 = u->P[0], P2 = u->P[1], P3 = u->P[2];
     A(&u->X0, 2 * P1 * 8);
     A(&u->A0, 2 * P1 * 16);
@@ -1090,6 +962,10 @@ extern "C" cfm_status cfm_unet_create(int n, int batch, cfm_unet **out) {
     for (bf16 **g : {&u->g2a, &u->g2b, &u->g2c}) A(g, 2 * P2 * 96);
     for (bf16 **g : {&u->g3a, &u->g3b}) A(g, 2 * P3 * 64);
     if (st != CFM_OK) return fail(st);
+    for (int i = 0; i < kNConv; ++i)  // the packed weights' padding stays zero
+        if (hipMemset(u->Wf[i], 0, 2 * (size_t)kConv[i].cout * u->Kp[i]) != hipSuccess ||
+            (i > 0 && hipMemset(u->Wt[i], 0, 2 * (size_t)kConv[i].cin * u->Kpt[i]) != hipSuccess))
+            return fail(CFM_EDEVICE);
     if (hipMemset(u->master, 0, 4 * u->nparam) != hipSuccess || hipMemset(u->adam_m, 0, 4 * u->nparam) != hipSuccess ||
         hipMemset(u->adam_v, 0, 4 * u->nparam) != hipSuccess)
         return fail(CFM_EDEVICE);
@@ -1098,15 +974,15 @@ extern "C" cfm_status cfm_unet_create(int n, int batch, cfm_unet **out) {
 }
 
 static cfm_status pack_all_weights(cfm_unet *u) {
+    PackTable T;
+    int most = 0;
     for (int i = 0; i < kNConv; ++i) {
         const ConvSpec &s = kConv[i];
-        CFM_HIP(hipMemsetAsync(u->Wf[i], 0, 2 * (size_t)s.cout * u->Kp[i], u->stream));
-        if (u->Wt[i]) CFM_HIP(hipMemsetAsync(u->Wt[i], 0, 2 * (size_t)s.cin * u->Kpt[i], u->stream));
-        const int total = s.cout * s.cin * 27;
-        hipLaunchKernelGGL(pack_weights_kernel, blocks_for(total), dim3(256), 0, u->stream, u->master + u->woff[i],
-                           s.cout, s.cin_real, s.cin, u->Kp[i], u->Kpt[i], u->Wf[i], u->Wt[i]);
-        CFM_HIP(hipGetLastError());
+        T.layer[i] = {u->master + u->woff[i], u->Wf[i], u->Wt[i], s.cout, s.cin_real, s.cin, u->Kp[i], u->Kpt[i]};
+        most = std::max(most, s.cout * s.cin * 27);
     }
+    hipLaunchKernelGGL(pack_weights_kernel, dim3((unsigned)((most + 255) / 256), kNConv), dim3(256), 0, u->stream, T);
+    CFM_HIP(hipGetLastError());
     return CFM_OK;
 }
 
@@ -1282,34 +1158,27 @@ extern "C" cfm_status cfm_unet_forward(cfm_unet *u, const float *input, float *o
     return CFM_OK;
 }
 
-// weight and bias gradients of conv I from its input X and output gradient dZ
-// the LDS-staged weight gradient for the network's (input, output) channel pairs
-// with 16-multiple input channels; the first layer (8 padded input channels)
-// keeps the gather kernel
 template <int CIN, int COUT, int WROWS, int KS = 1>
-static void launch_wgrad_rows(int nslab, hipStream_t st, const bf16 *X, const bf16 *dZ, int kp, float *partial, int n,
-                              int npts, int slab) {
+static void launch_wgrad_rows(int nslab, hipStream_t st, const bf16 *X, const bf16 *dZ, int kp, float *partial,
+                              const WgradShape &S) {
     constexpr int CINP = CIN / KS < 16 ? 16 : CIN / KS;
-    const int R = 64 / n;
-    const size_t lds = sizeof(bf16) * ((size_t)COUT * 72 + (size_t)3 * (R + 2) * CINP * (n + 8));
-    // (the largest staging, 48 input channels at n = 64, is just above 64 KiB)
+    const size_t lds = sizeof(bf16) * ((size_t)COUT * 72 + (size_t)3 * (S.rows + 2) * CINP * (S.w8 + 8));
+    // (the largest staging, 48 input channels and rows of 64 points, is just above 64 KiB)
     static const bool big_lds_ok =
         hipFuncSetAttribute((const void *)conv3_wgrad_rows_kernel<CIN, COUT, WROWS, KS>,
                             hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) == hipSuccess;
     (void)big_lds_ok;
     hipLaunchKernelGGL((conv3_wgrad_rows_kernel<CIN, COUT, WROWS, KS>), dim3(nslab, KS), dim3(64 * 9 / WROWS), lds,
-                       st, X, dZ, kp, partial, n, npts, slab);
+                       st, X, dZ, kp, partial, S);
 }
 
-// every tap in one workgroup (whole x rows per 64-point block): n = 16, 32, 64 and slabs of
-// whole blocks; three (dz, dy) rows per wavefront up to 4 channel-tile pairs, else one
+// three (dz, dy) rows per wavefront up to 4 channel-tile pairs, else one
 static bool wgrad_rows(int cin, int cout, int nslab, hipStream_t st, const bf16 *X, const bf16 *dZ, int kp,
-                       float *partial, int n, int npts, int slab) {
-    if ((n != 16 && n != 32 && n != 64) || slab % 64 != 0 || npts % 64 != 0) return false;
-#define CFM_WGRAD_ROWS(C, O, WR, KS)                                                    \
-    if (cin == C && cout == O) {                                                        \
-        launch_wgrad_rows<C, O, WR, KS>(nslab, st, X, dZ, kp, partial, n, npts, slab);  \
-        return true;                                                                    \
+                       float *partial, const WgradShape &S) {
+#define CFM_WGRAD_ROWS(C, O, WR, KS)                                         \
+    if (cin == C && cout == O) {                                             \
+        launch_wgrad_rows<C, O, WR, KS>(nslab, st, X, dZ, kp, partial, S);   \
+        return true;                                                         \
     }
     CFM_WGRAD_ROWS(8, 16, 3, 1)
     CFM_WGRAD_ROWS(16, 16, 3, 1)
@@ -1323,61 +1192,25 @@ static bool wgrad_rows(int cin, int cout, int nslab, hipStream_t st, const bf16 
     return false;
 }
 
-static bool wgrad_lds(int cin, int cout, int nslab, hipStream_t st, const bf16 *X, const bf16 *dZ, int kp,
-                      float *partial, int n, int npts, int slab) {
-    if (wgrad_rows(cin, cout, nslab, st, X, dZ, kp, partial, n, npts, slab)) return true;
-    const dim3 grid(27, nslab);
-#define CFM_WGRAD_LDS(C, O)                                                                              \
-    if (cin == C && cout == O) {                                                                         \
-        hipLaunchKernelGGL((conv3_wgrad_lds_kernel<C, O>), grid, dim3(256), 0, st, X, dZ, kp, partial, n, \
-                           npts, slab);                                                                  \
-        return true;                                                                                     \
-    }
-    CFM_WGRAD_LDS(16, 16)
-    CFM_WGRAD_LDS(16, 32)
-    CFM_WGRAD_LDS(32, 32)
-    CFM_WGRAD_LDS(32, 64)
-    CFM_WGRAD_LDS(64, 64)
-    CFM_WGRAD_LDS(96, 32)
-    CFM_WGRAD_LDS(48, 16)
-#undef CFM_WGRAD_LDS
-    return false;
-}
-
-// out[i] = sum over the nslab slab partials of u->partial (count values each), in two passes
-static void reduce_slabs(cfm_unet *u, int nslab, size_t count, float *out) {
-    if (nslab < 4 * kReduceParts) {
-        hipLaunchKernelGGL(reduce_slabs_kernel, blocks_for(count), dim3(256), 0, u->stream, u->partial, nslab, count,
-                           out);
-        return;
-    }
-    const dim3 grid((unsigned)((count + 255) / 256), kReduceParts);
-    hipLaunchKernelGGL(reduce_slab_parts_kernel, grid, dim3(256), 0, u->stream, u->partial, nslab, count, kReduceParts,
-                       u->rtmp);
-    hipLaunchKernelGGL(reduce_slabs_kernel, blocks_for(count), dim3(256), 0, u->stream, u->rtmp, kReduceParts, count,
-                       out);
-}
-
+// gradients of conv I's weights and biases from its input X and output gradient dZ
 static cfm_status conv_wgrad(cfm_unet *u, int I, const bf16 *X, const bf16 *dZ) {
     const ConvSpec &s = kConv[I];
-    const int level = s.level, n = u->n >> level;
-    const size_t npts = u->P[level];
-    const size_t slab = u->slab;  // fixed 4096-point slabs measured fastest (more wavefronts)
-    const int nslab = (int)((npts + slab - 1) / slab);
-    const int ntile_k = u->Kp[I] / 16;
-    const int ntile = (s.cout / 16) * ntile_k;
-    const size_t count = (size_t)s.cout * u->Kp[I];
-    if (!wgrad_lds(s.cin, s.cout, nslab, u->stream, X, dZ, u->Kp[I], u->partial, n, (int)npts, (int)slab))
-        hipLaunchKernelGGL(conv3_wgrad_kernel, dim3((ntile + 3) / 4, nslab), dim3(256), 0, u->stream, X, s.cin, dZ,
-                           s.cout, u->Kp[I], u->partial, n, (int)npts, (int)slab, ntile_k);
+    const int Kp = u->Kp[I], count = s.cout * (Kp + 1);
+    int nslab;
+    const WgradShape S = wgrad_shape(u->n >> s.level, u->batch, &nslab);
+    if (!wgrad_rows(s.cin, s.cout, nslab, u->stream, X, dZ, Kp, u->partial, S))
+        return CFM_FAIL(CFM_EINVAL, "unet: no weight-gradient kernel for %d -> %d channels", s.cin, s.cout);
     CFM_HIP(hipGetLastError());
-    reduce_slabs(u, nslab, count, u->gk);
-    hipLaunchKernelGGL(unpack_wgrad_kernel, blocks_for((size_t)s.cout * s.cin_real * 27), dim3(256), 0, u->stream,
-                       u->gk, s.cout, s.cin_real, s.cin, u->Kp[I], u->grad + u->woff[I]);
-    hipLaunchKernelGGL(chan_sum_kernel, dim3(nslab), dim3(256), 0, u->stream, dZ, s.cout, (int)npts, (int)slab,
-                       u->partial);
-    hipLaunchKernelGGL(reduce_rows_kernel, dim3(s.cout), dim3(1024), 0, u->stream, u->partial, nslab,
-                       u->grad + u->boff[I]);
+    const float *part = u->partial;
+    if (nslab >= 4 * kReduceParts) {
+        const dim3 grid((unsigned)((count + 255) / 256), kReduceParts);
+        hipLaunchKernelGGL(reduce_slab_parts_kernel, grid, dim3(256), 0, u->stream, u->partial, nslab, (size_t)count,
+                           kReduceParts, u->rtmp);
+        part = u->rtmp;
+        nslab = kReduceParts;
+    }
+    hipLaunchKernelGGL(reduce_slabs_kernel, blocks_for(count), dim3(256), 0, u->stream, part, nslab, s.cout,
+                       s.cin_real, s.cin, Kp, u->grad + u->woff[I], u->grad + u->boff[I]);
     CFM_HIP(hipGetLastError());
     return CFM_OK;
 }

@@ -90,3 +90,19 @@ def test_params_roundtrip(cfm, gpu):
     p = cfm.unet_init_params(9)
     with cfm.UNet(8, 1, params=p) as net:
         assert np.array_equal(net.params(), p)
+
+
+# rows that are not whole 8-point groups, that leave a 64-point block part empty, and that take two segments
+@pytest.mark.parametrize("n,batch", [(20, 2), (36, 1), (68, 1)])
+def test_gradient_of_ragged_rows(cfm, gpu, n, batch):
+    params, inp, target = _case(50 + n, n, batch)
+    with cfm.UNet(n, batch, params=params) as net:
+        loss, g = net.gradient(inp, target)
+    rl, rg, _ = uo.loss_and_grad(params.astype(np.float64), inp, target, n, rounding=True)
+    assert loss == pytest.approx(rl, rel=5e-3)
+    off = 0
+    for li, (ci, co) in enumerate(uo.CONVS):
+        for name, cnt in (("W", co * ci * 27), ("b", co)):
+            e = _rel(g[off: off + cnt], rg[off: off + cnt])
+            assert e < 3e-2, f"conv {li} {name}: rel err {e:.3g}"
+            off += cnt
