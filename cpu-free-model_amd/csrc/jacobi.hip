@@ -2551,7 +2551,7 @@ cfm_status cfm::jacobi_configure(const cfm_jacobi_params *p, JacobiConfig *c) {
     // the defaults (nothing about the kernel asked for) may go to the register tiles
     if (p->variant == CFM_JACOBI_PERSISTENT && p->time_block == 0 && p->tile_rows <= 0 && p->block_threads <= 0 &&
         p->grid_blocks <= 0 && p->chunks <= 0)
-        c->tile = jacobi_tile_configure(*p, c);
+        c->tile = is3d ? jacobi_pipe_configure(*p, c) : jacobi_tile_configure(*p, c);
     int rate_khz = 0;
     if (hipDeviceGetAttribute(&rate_khz, hipDeviceAttributeWallClockRate, c->dev.device) ==
             hipSuccess &&
@@ -2659,6 +2659,12 @@ int cfm::jacobi_passes(const cfm_jacobi_params &p, const JacobiConfig &c) {
 
 int cfm::jacobi_swaps(const cfm_jacobi_params &p, const JacobiConfig &c) {
     if (!c.tile) return jacobi_passes(p, c);
+    if (c.pipe) {
+        int turns = 0;
+        for (int k = 0; k < p.niter; ++turns)
+            k += jacobi_pipe_steps(k, p.niter, c.depth, p.norm_every, p.bc == CFM_BC_PERIODIC);
+        return turns;
+    }
     // periodic rows: the first sweep is a pass of its own
     const int first = p.bc == CFM_BC_PERIODIC ? std::min(p.niter, 1) : 0;
     return first + (p.niter - first + c.depth - 1) / c.depth;

@@ -39,7 +39,8 @@ struct JacobiConfig {
     KernelFn kernel = nullptr;
     bool t2 = false;  // more than one sweep per pass (the two-/three-/four-sweep kernels)
     int sweeps_per_pass = 1;
-    bool tile = false;  // the register-tile kernels (jacobi_tile.hip)
+    bool tile = false;  // the register-tile and pipeline kernels (jacobi_tile.hip, jacobi_pipe.hip)
+    bool pipe = false;  // the latter
     int tile_sx = 0, tile_sy = 0, tile_hx = 0, tile_hy = 0, depth = 0;
     int grid = 0;
     int norm_grid = 0;  // the streaming kernel's grid, which the no-allocation entry point's limit goes by
@@ -49,8 +50,16 @@ struct JacobiConfig {
 
 // Validates p and fills c for the current device.
 cfm_status jacobi_configure(const cfm_jacobi_params *p, JacobiConfig *c);
+// Sweeps of the pipeline kernels' pass that starts with sweep k: a sweep whose update norm is wanted
+// is the first of its pass, and with periodic planes the run's first sweep is a pass of its own.
+__host__ __device__ inline int jacobi_pipe_steps(int k, int niter, int depth, int norm_every, bool periodic) {
+    int steps = niter - k < depth ? niter - k : depth;
+    if (norm_every > 0 && norm_every - k % norm_every < steps) steps = norm_every - k % norm_every;
+    return periodic && k == 0 ? 1 : steps;
+}
 // Takes c to a register-tile kernel where that is the faster one; false leaves it as it is.
-bool jacobi_tile_configure(const cfm_jacobi_params &p, JacobiConfig *c);
+bool jacobi_tile_configure(const cfm_jacobi_params &p, JacobiConfig *c);  // 2D
+bool jacobi_pipe_configure(const cfm_jacobi_params &p, JacobiConfig *c);  // 3D
 // Enqueues one run of p.niter sweeps on `stream` (barrier reset, then the
 // persistent launch or one launch per sweep) over b0 (current field) and b1;
 // timers (may be null): per-workgroup phase ticks; *coop as launch_persistent

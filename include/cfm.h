@@ -80,8 +80,9 @@ typedef struct {
     int block_threads;/* 0 = one workgroup per CU (size set by the tile shape), or 256 */
     int time_block;   /* sweeps per HBM pass of the persistent kernels: 0 = auto (2D with nothing else
                          set: register tiles, whose passes are as deep as pays; 2D otherwise: Dirichlet 4,
-                         or 3 with 1024-thread workgroups, periodic y 2; 3D: 2, Dirichlet or periodic z (periodic:
-                         512-thread workgroups; nx > 512: x tiles, which need 16-byte aligned rows, a
+                         or 3 with 1024-thread workgroups, periodic y 2; 3D with nothing else set: a register
+                         pipeline of 4 sweeps a pass, where norms are not too frequent for it; 3D
+                         otherwise: 2, Dirichlet or periodic z (periodic: 512-thread workgroups; nx > 512: x tiles, which need 16-byte aligned rows, a
                          field below 2 GiB and 512-thread workgroups); with the default tile shape,
                          else 1), 1, 2, or 3 and 4 (2D Dirichlet only; 4 in 512-thread workgroups) */
     int phase_timers; /* nonzero: every workgroup of the persistent kernel records the time it spends
@@ -96,8 +97,9 @@ typedef struct {
     int block_threads;  /* threads per workgroup */
     int iterations;     /* sweeps (Jacobi) or CG iterations (summed inner for IR) */
     int outer_iterations; /* Jacobi: passes over the field in HBM as time_block counts them (auto in 2D:
-                             Dirichlet 4 sweeps each, periodic y 2; the register tiles may make
-                             several such passes between two trips through memory); IR: refinements */
+                             Dirichlet 4 sweeps each, periodic y 2; in 3D 2, or 1; the register tiles and
+                             the register pipeline may make several such passes between two trips
+                             through memory); IR: refinements */
     int cooperative;    /* persistent kernel launch: 1 = cooperative (co-residency guaranteed),
                            0 = ordinary launch because another process held ROCm's one-process
                            cooperative grant (co-residency expected, not guaranteed; the barrier
