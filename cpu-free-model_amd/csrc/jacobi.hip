@@ -2721,9 +2721,7 @@ static cfm_status jacobi_run(cfm_jacobi_plan *pl, double *norms, int norm_cap, i
         std::vector<double> part((size_t)c.norm_slots * c.grid);
         CFM_HIP(hipMemcpy(part.data(), pl->norm_part, sizeof(double) * part.size(), hipMemcpyDeviceToHost));
         for (int s = 0; s < c.norm_slots; ++s) {
-            double acc = 0.0;
-            for (int b = 0; b < c.grid; ++b) acc += part[(size_t)s * c.grid + b];
-            if (norms && s < norm_cap) norms[s] = std::sqrt(acc);
+            if (norms && s < norm_cap) norms[s] = std::sqrt(jacobi_norm_sum(part.data() + (size_t)s * c.grid, c.grid));
         }
         produced = c.norm_slots;
     }

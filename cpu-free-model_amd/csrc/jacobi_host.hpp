@@ -57,6 +57,18 @@ __host__ __device__ inline int jacobi_pipe_steps(int k, int niter, int depth, in
     if (norm_every > 0 && norm_every - k % norm_every < steps) steps = norm_every - k % norm_every;
     return periodic && k == 0 ? 1 : steps;
 }
+// The workgroups' partial sums of squares in workgroup order, with what each addition rounds off kept
+// and added last: more workgroups share a field in the tile kernels than in the streaming ones, and
+// their norms are as accurate for it.
+__host__ __device__ inline double jacobi_norm_sum(const double *part, int n) {
+    double sum = 0.0, lost = 0.0;
+    for (int b = 0; b < n; ++b) {
+        const double next = sum + part[b], from_part = next - sum;
+        lost += (sum - (next - from_part)) + (part[b] - from_part);
+        sum = next;
+    }
+    return lost == lost ? sum + lost : sum;  // (an infinite sum has no meaningful rest)
+}
 // Takes c to a register-tile kernel where that is the faster one; false leaves it as it is.
 bool jacobi_tile_configure(const cfm_jacobi_params &p, JacobiConfig *c);  // 2D
 bool jacobi_pipe_configure(const cfm_jacobi_params &p, JacobiConfig *c);  // 3D

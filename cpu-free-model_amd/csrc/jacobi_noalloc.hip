@@ -45,14 +45,12 @@ cfm_status scratch_ptr(int device, unsigned char **out) {
     return CFM_OK;
 }
 
-// sums[s] = part[s][0] + part[s][1] + ... in workgroup order, the order the
-// plan path adds them on the host (so the square roots are the same bits).
+// sums[s] = the sum of part[s][...] as the plan path forms it on the host (so the
+// square roots are the same bits).
 __global__ void norm_slot_sums_kernel(const double *part, int slots, int grid, double *sums) {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= slots) return;
-    double acc = 0.0;
-    for (int b = 0; b < grid; ++b) acc += part[(size_t)s * grid + b];
-    sums[s] = acc;
+    sums[s] = jacobi_norm_sum(part + (size_t)s * grid, grid);
 }
 
 }  // namespace
