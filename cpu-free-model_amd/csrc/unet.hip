@@ -304,34 +304,43 @@ __global__ void __launch_bounds__(64 * NW) conv3_fwd_xacc_kernel(const bf16 *__r
 // dx = -1 is the first, dx = +1 the dwords 1..4, dx = 0 a 2-byte byte-align of
 // the pair.  Input channels below 16 are padded with zero rows (the first layer's
 // 8).  The bias gradient is one more product, with a B fragment of ones.
-// KS > 1 splits the input channels over KS workgroups per slab (blockIdx.y):
-// each stages and computes CIN / KS of them, which keeps the accumulators of
-// the wide layers in registers.  Bound by staging (loads and transposing LDS stores) with
-// two workgroups a CU to overlap it; other row lengths than 16, 32 and 64 went through a kernel
-// that staged the input anew for each of the 27 taps.
+// blockIdx.y: the group of 16 input channels that the workgroup stages and computes.
+// Bound by latency and by the vector instructions of the staging: blocks follow one another along y,
+// the rows that the last block had stay in LDS, the new ones and the next dZ are loaded while a block is
+// multiplied, and where an item comes from and goes to is worked out once.  At 4 x 64^3, 48 -> 16:
+// 447 us with every block staged on its own, 261 with the rows kept, 161 us with the channels split and the items
+// kept; 16 -> 16 102, 72 and 52.  Other row lengths than 16, 32 and 64 went through a kernel that
+// staged the input anew for each of the 27 taps.
+constexpr int kWgradRow = 72;  // a staged input row: 64 points, one at each end, and padding that keeps fragments 16-byte aligned
+constexpr int kWgradRows16 = 16 * (kWgradRow + 1);  // and that of 16 channels
 struct WgradShape {
     int n, nblk, per_slab;  // points along an edge; blocks, and blocks a workgroup takes
     int w8, rows, nyb, nseg;  // a row's padded points, rows of a block, blocks along y and x
     float inv_pairs;          // 1 / (w8 / 2 + 1)
 };
 
-template <int CIN, int COUT, int WROWS, int KS = 1>
-__global__ void __launch_bounds__(64 * 9 / WROWS) conv3_wgrad_rows_kernel(const bf16 *__restrict__ Xg,
+template <int CIN, int COUT>
+__global__ void __launch_bounds__(192) conv3_wgrad_rows_kernel(const bf16 *__restrict__ Xg,
                                                                         const bf16 *__restrict__ dZ, int Kp,
                                                                         float *__restrict__ partial, WgradShape S) {
-    constexpr int CINX = CIN;            // channels per point of the input tensor
-    constexpr int CW = CIN / KS;         // input channels of this workgroup
-    constexpr int CINP = CW < 16 ? 16 : CW;
-    constexpr int MT = COUT / 16, KT = CINP / 16, NWAVE = 9 / WROWS, NTH = 64 * NWAVE;
-    static_assert(CIN % KS == 0 && (KS == 1 || CW % 16 == 0), "channel split");
+    constexpr int CINX = CIN;                // channels per point of the input tensor
+    constexpr int CW = CIN < 16 ? CIN : 16;  // input channels of this workgroup
+    constexpr int CINP = 16;                 // and as many rows as a fragment has
+    constexpr int MT = COUT / 16, KT = 1, WROWS = 3, NTH = 192;
+    static_assert(CIN % CW == 0, "channel split");
     const int ci0 = blockIdx.y * CW;
     const bf16 *X = Xg + ci0;
     constexpr int DS = 72;  // dZ row stride (64 points + 8: spreads the 16 rows of a fragment over the banks)
-    static_assert(CINP % 16 == 0 && COUT % 16 == 0 && CW % 8 == 0 && 9 % WROWS == 0, "shape");
+    static_assert(COUT % 16 == 0 && CW % 8 == 0, "shape");
     extern __shared__ __attribute__((aligned(16))) bf16 wg_lds[];
-    const int n = S.n, W8 = S.w8, R = S.rows, W = W8 + 8, ROWS = 3 * (R + 2);
+    const int n = S.n, W8 = S.w8, R = S.rows;
     bf16 *dzT = wg_lds;                 // [COUT][DS]
-    bf16 *xT = wg_lds + COUT * DS;      // [ROWS][CINP][W], x stored at column x - x0 + 1
+    // [3 planes][R + 2 rows][16 channels][W], x stored at column x - x0 + 1, with 8 elements more after
+    // every 8 channels: the column pairs of the two groups, which one store writes together, then lie on
+    // different banks
+    bf16 *xT = wg_lds + COUT * DS;
+    constexpr int W = kWgradRow, RSTR = CINP * (W + 1);
+    static_assert(RSTR == kWgradRows16, "as the launch counts it");
     const int s = blockIdx.x;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int nl = lane & 15, g = lane >> 4;
@@ -340,9 +349,9 @@ __global__ void __launch_bounds__(64 * 9 / WROWS) conv3_wgrad_rows_kernel(const 
     const bf16x8 one8 = {(bf16)1.0f, (bf16)1.0f, (bf16)1.0f, (bf16)1.0f,
                          (bf16)1.0f, (bf16)1.0f, (bf16)1.0f, (bf16)1.0f};
     if (CW < CINP) {  // padded input channels: zero once, never overwritten
-        for (int v = threadIdx.x; v < ROWS * (CINP - CW) * W; v += NTH) {
+        for (int v = threadIdx.x; v < 3 * (R + 2) * (CINP - CW) * W; v += NTH) {
             const int c = CW + (v / W) % (CINP - CW), r = v / (W * (CINP - CW));
-            xT[((size_t)r * CINP + c) * W + v % W] = (bf16)0.0f;
+            xT[r * RSTR + c * W + (c >> 3) * 8 + v % W] = (bf16)0.0f;
         }
     }
     f32x4 acc[WROWS][3][MT][KT], accb[MT];
@@ -366,51 +375,113 @@ __global__ void __launch_bounds__(64 * 9 / WROWS) conv3_wgrad_rows_kernel(const 
         xg[h] = q - rq[h] * W8;
         if (rq[h] >= R) rq[h] = 0;
     }
+    // Two neighbouring points' 8 channels, transposed into LDS: each 4-byte store writes one channel's pair.
+    struct Pair {
+        u16x8 p[2];
+    };
+    const auto put = [](bf16 *to, int stride, const Pair &v) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            *reinterpret_cast<unsigned *>(to + i * stride) = (unsigned)v.p[0][i] | ((unsigned)v.p[1][i] << 16);
+    };
+    // 8 channels of a point that lies `off` bytes from `p`; zeros if it is not there
+    const auto get = [](const bf16 *p, int bytes, int off, bool there) {
+        const auto r = __builtin_amdgcn_make_buffer_rsrc((void *)p, (short)0, bytes, 0x00020000);
+        return __builtin_bit_cast(u16x8, __builtin_amdgcn_raw_buffer_load_b128(r, there ? off : -16, 0, 0));
+    };
+    // dZ of a block: a pair of points of 8 channels an item
+    constexpr int ZITEMS = 32 * (COUT / 8), NZ = (ZITEMS + NTH - 1) / NTH;
+    struct ZItem {
+        int lds, off, row, x;  // where it goes; where it comes from, from point (x0, y0) on; which point it is
+    } zi[NZ];
+#pragma unroll
+    for (int i = 0; i < NZ; ++i) {
+        const int v = threadIdx.x + i * NTH, j = 2 * (v / (COUT / 8)), c8 = v % (COUT / 8);
+        const int row = j / W8, x = j - row * W8;
+        zi[i] = {8 * c8 * DS + j, ((row * n + x) * COUT + 8 * c8) * 2, v < ZITEMS && row < R ? row : n, x};
+    }
+    const auto get_dz = [&](const ZItem &t, int x0, int y0, int z, int b) {
+        const bf16 *from = dZ + ((((size_t)b * n + z) * n + y0) * n + x0) * COUT;
+        const bool row = y0 + t.row < n;
+        Pair o;
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+            o.p[e] = get(from, 64 * n * COUT * 2, t.off + e * COUT * 2, row && x0 + t.x + e < n);
+        return o;
+    };
+    const auto put_dz = [&](int i, const Pair &o) {
+        if ((int)threadIdx.x + i * NTH < ZITEMS) put(dzT + zi[i].lds, DS, o);
+    };
+    // Input rows, 8 channels of a pair of columns an item.  Row y is kept at y + 1 modulo R + 2 of its
+    // plane's rows, so a block needs only the R rows that the block before it did not have.
+    const int pairs = W8 / 2 + 1;
+    struct XItem {
+        int lds, off, plane, row, x;  // as above, from (x0, first row, z) on; the plane's offset -1, 0, 1
+    };
+    const auto x_item = [&](int v, int rows) {
+        const int c8 = v % (CW / 8), pr = v / (CW / 8);
+        const int r = (int)(((float)pr + 0.5f) * S.inv_pairs);  // pr / pairs, exact below 2^20
+        const int xj = 2 * (pr - r * pairs), dz = r >= 2 * rows ? 2 : r >= rows ? 1 : 0, row = r - dz * rows;
+        return XItem{dz * (R + 2) * RSTR + c8 * (8 * W + 8) + xj, ((row * n + xj - 1) * CINX + 8 * c8) * 2,
+                     v < 3 * rows * pairs * (CW / 8) ? dz - 1 : n + 1, row, xj - 1};
+    };
+    const auto get_x = [&](const XItem &t, int x0, int y, int z, int b) {
+        const bool there = z + t.plane >= 0 && z + t.plane < n && y + t.row >= 0 && y + t.row < n;
+        // (an offset below zero, the column before x0, is within the tensor wherever it is read)
+        const bf16 *from = X + ((((size_t)b * n + z) * n + y) * n + x0 - 1) * CINX - n * n * CINX;
+        const unsigned off = (unsigned)t.off + CINX * 2 + (unsigned)(t.plane + 1) * (unsigned)(n * n * CINX * 2);
+        Pair o;
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+            o.p[e] = get(from, 0x7fffffff, (int)(off + e * CINX * 2), there && x0 + t.x + e >= 0 && x0 + t.x + e < n);
+        return o;
+    };
+    const auto put_x = [&](const XItem &t, int base, const Pair &o) {
+        const int slot = base + t.row >= R + 2 ? base + t.row - (R + 2) : base + t.row;
+        if (t.plane <= 1) put(xT + t.lds + slot * RSTR, W, o);
+    };
+    // the next block's new rows and dZ wait in registers while this block is multiplied: R <= 8 rows of
+    // R (W8 / 2 + 1) <= 40 pairs
+    constexpr int NX = (3 * 40 * (CW / 8) + NTH - 1) / NTH;
+    XItem xi[NX];
+#pragma unroll
+    for (int i = 0; i < NX; ++i) xi[i] = x_item(threadIdx.x + i * NTH, R);
+    Pair pz[NZ], px[NX];
     const int blk_end = min(S.nblk, (s + 1) * S.per_slab);
+    bool fresh = true;  // nothing of the block's rows is staged yet
     for (int blk = s * S.per_slab; blk < blk_end; ++blk) {
         int u = blk;
+        const int yb = u % S.nyb, y0 = yb * R;
+        u /= S.nyb;
         const int x0 = (u % S.nseg) * 64;
         u /= S.nseg;
-        const int y0 = (u % S.nyb) * R;
-        u /= S.nyb;
         const int z = u % n, b = u / n;
-        // stage dZ of the block, transposed: two points per thread, so each LDS store
-        // writes one channel's pair of neighbouring points (4 bytes)
-        for (int v = threadIdx.x; v < 32 * (COUT / 8); v += NTH) {
-            const int j = 2 * (v / (COUT / 8)), c8 = v % (COUT / 8);
-            const int rr = j / W8, x = x0 + j - rr * W8, y = y0 + rr;
-            const bool row = rr < R && y < n;
-            const bf16 *p = dZ + ((((size_t)b * n + z) * n + y) * n + x) * COUT + 8 * c8;
-            u16x8 a0 = __builtin_bit_cast(u16x8, zero8), a1 = a0;
-            if (row && x < n) a0 = *reinterpret_cast<const u16x8 *>(p);
-            if (row && x + 1 < n) a1 = *reinterpret_cast<const u16x8 *>(p + COUT);
+        const int base = y0 % (R + 2);  // where row y0 - 1 is kept
+        if (fresh) {
 #pragma unroll
-            for (int i = 0; i < 8; ++i)
-                *reinterpret_cast<unsigned *>(&dzT[(8 * c8 + i) * DS + j]) = (unsigned)a0[i] | ((unsigned)a1[i] << 16);
-        }
-        // stage the 3 x (R+2) input rows around the block, transposed, x0 - 1 .. x0 + W8 (two
-        // columns per thread as above)
-        for (int v = threadIdx.x; v < ROWS * (W8 / 2 + 1) * (CW / 8); v += NTH) {
-            const int c8 = v % (CW / 8), pr = v / (CW / 8);
-            const int r = (int)(((float)pr + 0.5f) * S.inv_pairs);  // pr / (W8/2 + 1), exact below 2^20
-            const int xj = 2 * (pr - r * (W8 / 2 + 1));
-            const int rz = r >= 2 * (R + 2) ? 2 : r >= R + 2 ? 1 : 0;
-            const int zz = z + rz - 1, yy = y0 + r - rz * (R + 2) - 1;
-            u16x8 a[2];
+            for (int i = 0; i < NZ; ++i) put_dz(i, get_dz(zi[i], x0, y0, z, b));
+            constexpr int U = 4;  // loads of four items in flight
+            for (int v = threadIdx.x; v < 3 * (R + 2) * pairs * (CW / 8); v += U * NTH) {
+                XItem t[U];
+                Pair p[U];
 #pragma unroll
-            for (int e = 0; e < 2; ++e) {
-                const int xx = x0 + xj + e - 1;
-                bf16x8 val = zero8;
-                if (xx >= 0 && xx < n && yy >= 0 && yy < n && zz >= 0 && zz < n)
-                    val = *reinterpret_cast<const bf16x8 *>(X + ((((size_t)b * n + zz) * n + yy) * n + xx) * CINX + 8 * c8);
-                a[e] = __builtin_bit_cast(u16x8, val);
+                for (int i = 0; i < U; ++i) {
+                    t[i] = x_item(v + i * NTH, R + 2);
+                    p[i] = get_x(t[i], x0, y0 - 1, z, b);
+                }
+#pragma unroll
+                for (int i = 0; i < U; ++i) put_x(t[i], base, p[i]);
             }
-#pragma unroll
-            for (int i = 0; i < 8; ++i)
-                *reinterpret_cast<unsigned *>(&xT[((size_t)r * CINP + 8 * c8 + i) * W + xj]) =
-                    (unsigned)a[0][i] | ((unsigned)a[1][i] << 16);
         }
         __syncthreads();
+        fresh = yb + 1 == S.nyb;
+        const bool more = !fresh && blk + 1 < blk_end;
+        if (more) {
+#pragma unroll
+            for (int i = 0; i < NZ; ++i) pz[i] = get_dz(zi[i], x0, y0 + R, z, b);
+#pragma unroll
+            for (int i = 0; i < NX; ++i) px[i] = get_x(xi[i], x0, y0 + R + 1, z, b);
+        }
 #pragma unroll
         for (int h = 0; h < 2; ++h) {  // two K steps of 32 points
             const int q = 32 * h + 8 * g;  // this lane's first point in the block
@@ -426,10 +497,11 @@ __global__ void __launch_bounds__(64 * 9 / WROWS) conv3_wgrad_rows_kernel(const 
             for (int a = 0; a < WROWS; ++a) {
                 const int rw = w * WROWS + a;  // (dz, dy) row index 0..8
                 const int dz = rw / 3, dy = rw % 3;  // offsets + 1
-                const int r = dz * (R + 2) + rq[h] + dy;
+                int slot = base + rq[h] + dy;
+                if (slot >= R + 2) slot -= R + 2;
 #pragma unroll
                 for (int k = 0; k < KT; ++k) {
-                    const bf16 *src = &xT[((size_t)r * CINP + k * 16 + nl) * W + xg[h]];
+                    const bf16 *src = xT + (dz * (R + 2) + slot) * RSTR + (k * 16 + nl) * W + (2 * k + (nl >> 3)) * 8 + xg[h];
                     const bf16x8 lo = *reinterpret_cast<const bf16x8 *>(src);
                     const bf16x8 hi = *reinterpret_cast<const bf16x8 *>(src + 8);
                     typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
@@ -450,6 +522,13 @@ __global__ void __launch_bounds__(64 * 9 / WROWS) conv3_wgrad_rows_kernel(const 
             }
         }
         __syncthreads();  // the staged rows are rewritten next
+        if (more) {
+#pragma unroll
+            for (int i = 0; i < NZ; ++i) put_dz(i, pz[i]);
+            // (row y0 + R + 1 is row R + 2 from y0 - 1 on: kept where that was)
+#pragma unroll
+            for (int i = 0; i < NX; ++i) put_x(xi[i], base, px[i]);
+        }
     }
     // D[4g+i][nl] = dW[m*16 + 4g + i][tap*CIN + k*16 + nl], tap = 9 dz + 3 dy + dx (offsets + 1)
     float *out = partial + (size_t)s * COUT * (Kp + 1);
@@ -819,12 +898,12 @@ size_t param_count() {
     return c + kHeadIn + 1;
 }
 
-// Blocks of 64 points of a layer's weight gradient, and the workgroups that share them: up to 512, two
-// a CU.  Fewer leave CUs idle (the deep levels had 4 to 32 when a workgroup took 4096 points), more write
-// and re-read more partials than they save.  Training steps, ms, for 128 / 256 / 512 / 1024 / 2048
-// workgroups: 4 x 64^3 3.75, 2.76, 2.59, 2.63, 2.95; 8 x 36^3 2.08, 1.71, 1.64, 1.65, 1.84; 16 x 12^3
-// 0.80, 0.70, 0.71, 0.71, 0.71 (4096 points each: 4.19 at 4 x 64^3).
-WgradShape wgrad_shape(int n, int batch, int *nslab) {
+// Blocks of 64 points of a layer's weight gradient, and the workgroups that share them: 512, two a CU, with
+// the groups of 16 input channels counted (a workgroup that goes on to the next rows stages a third of
+// them anew, and more workgroups write and re-read more partials), or up to 1024 where 512 would take
+// fewer than 8 blocks each.  Training steps, ms, for 512 / 1024 / 2048 workgroups: 4 x 64^3 2.15, 2.23, 2.28;
+// 8 x 36^3 1.47, 1.50, 1.55; 16 x 12^3 0.80, 0.73, 0.73.
+WgradShape wgrad_shape(int n, int batch, int cin, int *nslab) {
     WgradShape S;
     S.n = n;
     S.w8 = n >= 64 ? 64 : (n + 7) / 8 * 8;
@@ -833,7 +912,8 @@ WgradShape wgrad_shape(int n, int batch, int *nslab) {
     S.nseg = (n + 63) / 64;
     S.nblk = batch * n * S.nyb * S.nseg;
     S.inv_pairs = 1.0f / (float)(S.w8 / 2 + 1);
-    const int most = 512;
+    const int groups = (cin + 15) / 16;
+    const int most = std::max(1, (S.nblk * (long long)groups >= 8 * 512 ? 512 : 1024) / groups);
     S.per_slab = (S.nblk + most - 1) / most;
     *nslab = (S.nblk + S.per_slab - 1) / S.per_slab;
     return S;
@@ -931,7 +1011,7 @@ extern "C" cfm_status cfm_unet_create(int n, int batch, cfm_unet **out) {
         if (i > 0) A(&u->Wt[i], 2 * (size_t)kConv[i].cin * u->Kpt[i]);
         max_wk = std::max(max_wk, (size_t)kConv[i].cout * (u->Kp[i] + 1));
         int nslab;
-        wgrad_shape(n >> kConv[i].level, batch, &nslab);
+        wgrad_shape(n >> kConv[i].level, batch, kConv[i].cin, &nslab);
         max_partial = std::max(max_partial, (size_t)nslab * kConv[i].cout * (u->Kp[i] + 1));
     }
     A(&u->rtmp, 4 * kReduceParts * max_wk);
@@ -1158,36 +1238,33 @@ extern "C" cfm_status cfm_unet_forward(cfm_unet *u, const float *input, float *o
     return CFM_OK;
 }
 
-template <int CIN, int COUT, int WROWS, int KS = 1>
+template <int CIN, int COUT>
 static void launch_wgrad_rows(int nslab, hipStream_t st, const bf16 *X, const bf16 *dZ, int kp, float *partial,
                               const WgradShape &S) {
-    constexpr int CINP = CIN / KS < 16 ? 16 : CIN / KS;
-    const size_t lds = sizeof(bf16) * ((size_t)COUT * 72 + (size_t)3 * (S.rows + 2) * CINP * (S.w8 + 8));
-    // (the largest staging, 48 input channels and rows of 64 points, is just above 64 KiB)
-    static const bool big_lds_ok =
-        hipFuncSetAttribute((const void *)conv3_wgrad_rows_kernel<CIN, COUT, WROWS, KS>,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) == hipSuccess;
+    const size_t lds = sizeof(bf16) * ((size_t)COUT * 72 + (size_t)3 * (S.rows + 2) * kWgradRows16);
+    // (short rows, eight to a block, take more than 64 KiB)
+    static const bool big_lds_ok = hipFuncSetAttribute((const void *)conv3_wgrad_rows_kernel<CIN, COUT>,
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) == hipSuccess;
     (void)big_lds_ok;
-    hipLaunchKernelGGL((conv3_wgrad_rows_kernel<CIN, COUT, WROWS, KS>), dim3(nslab, KS), dim3(64 * 9 / WROWS), lds,
-                       st, X, dZ, kp, partial, S);
+    hipLaunchKernelGGL((conv3_wgrad_rows_kernel<CIN, COUT>), dim3(nslab, (CIN + 15) / 16), dim3(192), lds, st, X, dZ, kp,
+                       partial, S);
 }
 
-// three (dz, dy) rows per wavefront up to 4 channel-tile pairs, else one
 static bool wgrad_rows(int cin, int cout, int nslab, hipStream_t st, const bf16 *X, const bf16 *dZ, int kp,
                        float *partial, const WgradShape &S) {
-#define CFM_WGRAD_ROWS(C, O, WR, KS)                                         \
-    if (cin == C && cout == O) {                                             \
-        launch_wgrad_rows<C, O, WR, KS>(nslab, st, X, dZ, kp, partial, S);   \
-        return true;                                                         \
+#define CFM_WGRAD_ROWS(C, O)                                             \
+    if (cin == C && cout == O) {                                         \
+        launch_wgrad_rows<C, O>(nslab, st, X, dZ, kp, partial, S);       \
+        return true;                                                     \
     }
-    CFM_WGRAD_ROWS(8, 16, 3, 1)
-    CFM_WGRAD_ROWS(16, 16, 3, 1)
-    CFM_WGRAD_ROWS(16, 32, 3, 1)
-    CFM_WGRAD_ROWS(32, 32, 3, 1)
-    CFM_WGRAD_ROWS(48, 16, 3, 1)
-    CFM_WGRAD_ROWS(32, 64, 1, 1)
-    CFM_WGRAD_ROWS(64, 64, 1, 2)  // (the input channels split over two workgroups: the accumulators
-    CFM_WGRAD_ROWS(96, 32, 1, 2)  //  of all of them do not fit in registers)
+    CFM_WGRAD_ROWS(8, 16)
+    CFM_WGRAD_ROWS(16, 16)
+    CFM_WGRAD_ROWS(16, 32)
+    CFM_WGRAD_ROWS(32, 32)
+    CFM_WGRAD_ROWS(48, 16)
+    CFM_WGRAD_ROWS(32, 64)
+    CFM_WGRAD_ROWS(64, 64)
+    CFM_WGRAD_ROWS(96, 32)
 #undef CFM_WGRAD_ROWS
     return false;
 }
@@ -1197,7 +1274,7 @@ static cfm_status conv_wgrad(cfm_unet *u, int I, const bf16 *X, const bf16 *dZ) 
     const ConvSpec &s = kConv[I];
     const int Kp = u->Kp[I], count = s.cout * (Kp + 1);
     int nslab;
-    const WgradShape S = wgrad_shape(u->n >> s.level, u->batch, &nslab);
+    const WgradShape S = wgrad_shape(u->n >> s.level, u->batch, s.cin, &nslab);
     if (!wgrad_rows(s.cin, s.cout, nslab, u->stream, X, dZ, Kp, u->partial, S))
         return CFM_FAIL(CFM_EINVAL, "unet: no weight-gradient kernel for %d -> %d channels", s.cin, s.cout);
     CFM_HIP(hipGetLastError());
