@@ -38,6 +38,23 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ float bf2f(bf16 v) { return (float)v; }
 __device__ __forceinline__ bf16 f2bf(float v) { return (bf16)v; }  // round to nearest even
 
+// The decoder's convolutions (48 and 96 input channels) read the concatenation of an upsampled
+// tensor and a skip connection; it is not stored: the channels below upsampled_channels(CIN) come from the
+// points of a grid of half the edge (nearest upsampling), the others from the skip connection's tensor.
+constexpr __host__ __device__ int upsampled_channels(int cin) { return cin == 48 ? 32 : cin == 96 ? 64 : 0; }
+
+// channels 8 cv .. 8 cv + 7 of point (x, y, z) of batch element b
+template <int CIN>
+__device__ __forceinline__ bf16x8 input8(const bf16 *__restrict__ X, const bf16 *__restrict__ Xup, int n, int b, int z,
+                                         int y, int x, int cv) {
+    constexpr int UP = upsampled_channels(CIN), OWN = CIN - UP;
+    if (UP > 0 && cv < UP / 8) {
+        const int m = n / 2;
+        return *reinterpret_cast<const bf16x8 *>(Xup + ((((size_t)b * m + z / 2) * m + y / 2) * m + x / 2) * UP + cv * 8);
+    }
+    return *reinterpret_cast<const bf16x8 *>(X + ((((size_t)b * n + z) * n + y) * n + x) * OWN + (cv - UP / 8) * 8);
+}
+
 // ------------------------------------------------------------- conv fwd ---
 // Y = conv3x3x3(X) + bias, optional ReLU.  W is [Cout][Kp] BF16 (k = tap*Cin+ci,
 // zero padded to Kp, a multiple of 32).
@@ -52,7 +69,8 @@ __device__ __forceinline__ bf16 f2bf(float v) { return (bf16)v; }  // round to n
 // The four accumulators of a lane (output channels 4g..4g+3 of one point) are
 // biased, rectified, rounded to BF16 and written as one 8-byte store.
 template <int MT, int CIN, int TY, int TZ>
-__global__ void __launch_bounds__(256) conv3_fwd_lds_kernel(const bf16 *__restrict__ X, const bf16 *__restrict__ W,
+__global__ void __launch_bounds__(256) conv3_fwd_lds_kernel(const bf16 *__restrict__ X, const bf16 *__restrict__ Xup,
+                                                            const bf16 *__restrict__ W,
                                                             int Kp, const float *__restrict__ bias,
                                                             bf16 *__restrict__ Y, int n, int nbx, int nby, int nbz,
                                                             int relu, const bf16 *__restrict__ mask) {
@@ -79,7 +97,7 @@ __global__ void __launch_bounds__(256) conv3_fwd_lds_kernel(const bf16 *__restri
         const int gx = x0 - 1 + cx, gy = y0 - 1 + cy, gz = z0 - 1 + cz;
         bf16x8 val = zero8;
         if (gx >= 0 && gx < n && gy >= 0 && gy < n && gz >= 0 && gz < n)
-            val = *reinterpret_cast<const bf16x8 *>(X + ((((size_t)b * n + gz) * n + gy) * n + gx) * CIN + cv * 8);
+            val = input8<CIN>(X, Xup, n, b, gz, gy, gx, cv);
         blk[v] = val;
     }
     __syncthreads();
@@ -162,6 +180,7 @@ __global__ void __launch_bounds__(256) conv3_fwd_lds_kernel(const bf16 *__restri
 // k loop unrolled by KU.
 template <int MT, int CIN, int TY, int TZ, int NXT, int NW, int KU>
 __global__ void __launch_bounds__(64 * NW) conv3_fwd_xacc_kernel(const bf16 *__restrict__ X,
+                                                                 const bf16 *__restrict__ Xup,
                                                                  const bf16 *__restrict__ W, int Kp,
                                                                  const float *__restrict__ bias,
                                                                  bf16 *__restrict__ Y, int n, int nby, int nbz,
@@ -188,7 +207,7 @@ __global__ void __launch_bounds__(64 * NW) conv3_fwd_xacc_kernel(const bf16 *__r
         const int gy = y0 - 1 + cy, gz = z0 - 1 + cz;
         bf16x8 val = zero8;
         if (cx < n && gy >= 0 && gy < n && gz >= 0 && gz < n)
-            val = *reinterpret_cast<const bf16x8 *>(X + ((((size_t)b * n + gz) * n + gy) * n + cx) * CIN + cv * 8);
+            val = input8<CIN>(X, Xup, n, b, gz, gy, cx, cv);
         blk[v] = val;
     }
     __syncthreads();
@@ -321,15 +340,17 @@ struct WgradShape {
 
 template <int CIN, int COUT>
 __global__ void __launch_bounds__(192) conv3_wgrad_rows_kernel(const bf16 *__restrict__ Xg,
+                                                                        const bf16 *__restrict__ Xup,
                                                                         const bf16 *__restrict__ dZ, int Kp,
                                                                         float *__restrict__ partial, WgradShape S) {
-    constexpr int CINX = CIN;                // channels per point of the input tensor
+    constexpr int UP = upsampled_channels(CIN), CINX = CIN - UP;  // channels per point of the input tensor(s)
     constexpr int CW = CIN < 16 ? CIN : 16;  // input channels of this workgroup
     constexpr int CINP = 16;                 // and as many rows as a fragment has
     constexpr int MT = COUT / 16, KT = 1, WROWS = 3, NTH = 192;
     static_assert(CIN % CW == 0, "channel split");
     const int ci0 = blockIdx.y * CW;
-    const bf16 *X = Xg + ci0;
+    const bool up = ci0 < UP;  // (uniform; UP is a multiple of 16)
+    const bf16 *X = up ? Xup + ci0 : Xg + (ci0 - UP);
     constexpr int DS = 72;  // dZ row stride (64 points + 8: spreads the 16 rows of a fragment over the banks)
     static_assert(COUT % 16 == 0 && CW % 8 == 0, "shape");
     extern __shared__ __attribute__((aligned(16))) bf16 wg_lds[];
@@ -344,8 +365,6 @@ __global__ void __launch_bounds__(192) conv3_wgrad_rows_kernel(const bf16 *__res
     const int s = blockIdx.x;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int nl = lane & 15, g = lane >> 4;
-    const bf16x8 zero8 = {(bf16)0.0f, (bf16)0.0f, (bf16)0.0f, (bf16)0.0f,
-                          (bf16)0.0f, (bf16)0.0f, (bf16)0.0f, (bf16)0.0f};
     const bf16x8 one8 = {(bf16)1.0f, (bf16)1.0f, (bf16)1.0f, (bf16)1.0f,
                          (bf16)1.0f, (bf16)1.0f, (bf16)1.0f, (bf16)1.0f};
     if (CW < CINP) {  // padded input channels: zero once, never overwritten
@@ -416,21 +435,31 @@ __global__ void __launch_bounds__(192) conv3_wgrad_rows_kernel(const bf16 *__res
     // plane's rows, so a block needs only the R rows that the block before it did not have.
     const int pairs = W8 / 2 + 1;
     struct XItem {
-        int lds, off, plane, row, x;  // as above, from (x0, first row, z) on; the plane's offset -1, 0, 1
+        int lds, off, plane, row, x, c;  // as above, from (x0, first row, z) on; the plane's offset -1, 0, 1
     };
     const auto x_item = [&](int v, int rows) {
         const int c8 = v % (CW / 8), pr = v / (CW / 8);
         const int r = (int)(((float)pr + 0.5f) * S.inv_pairs);  // pr / pairs, exact below 2^20
         const int xj = 2 * (pr - r * pairs), dz = r >= 2 * rows ? 2 : r >= rows ? 1 : 0, row = r - dz * rows;
         return XItem{dz * (R + 2) * RSTR + c8 * (8 * W + 8) + xj, ((row * n + xj - 1) * CINX + 8 * c8) * 2,
-                     v < 3 * rows * pairs * (CW / 8) ? dz - 1 : n + 1, row, xj - 1};
+                     v < 3 * rows * pairs * (CW / 8) ? dz - 1 : n + 1, row, xj - 1, 8 * c8};
     };
     const auto get_x = [&](const XItem &t, int x0, int y, int z, int b) {
         const bool there = z + t.plane >= 0 && z + t.plane < n && y + t.row >= 0 && y + t.row < n;
+        Pair o;
+        if (UP > 0 && up) {
+            const int m = n / 2;
+            const unsigned line = (unsigned)((b * m + ((z + t.plane) >> 1)) * m + ((y + t.row) >> 1)) * m;
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                const int x = x0 + t.x + e;
+                o.p[e] = get(X, 0x7fffffff, (int)(((line + (x >> 1)) * UP + t.c) * 2), there && x >= 0 && x < n);
+            }
+            return o;
+        }
         // (an offset below zero, the column before x0, is within the tensor wherever it is read)
         const bf16 *from = X + ((((size_t)b * n + z) * n + y) * n + x0 - 1) * CINX - n * n * CINX;
         const unsigned off = (unsigned)t.off + CINX * 2 + (unsigned)(t.plane + 1) * (unsigned)(n * n * CINX * 2);
-        Pair o;
 #pragma unroll
         for (int e = 0; e < 2; ++e)
             o.p[e] = get(from, 0x7fffffff, (int)(off + e * CINX * 2), there && x0 + t.x + e >= 0 && x0 + t.x + e < n);
@@ -698,17 +727,6 @@ __global__ void pool_bwd_kernel(const bf16 *__restrict__ dY, bf16 *__restrict__ 
     st8(dX + (size_t)q * C + 8 * cv, o);
 }
 
-// nearest upsampling m -> 2m, written into channels [off, off+C) of a buffer with Ct channels
-__global__ void up_fwd_kernel(const bf16 *__restrict__ X, bf16 *__restrict__ Y, int C, int Ct, int off, int m,
-                              int nb) {
-    const unsigned n = 2 * m, V = C / 8, um = m;
-    const unsigned i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (unsigned)nb * n * n * n * V) return;
-    const unsigned cv = i % V, q = i / V;
-    const unsigned x = q % n, y = (q / n) % n, z = (q / (n * n)) % n, b = q / (n * n * n);
-    st8(Y + (size_t)q * Ct + off + 8 * cv, ld8(X + ((((size_t)b * um + z / 2) * um + y / 2) * um + x / 2) * C + 8 * cv));
-}
-
 // gradient of nearest upsampling: sum of the 8 children (from channels [off, off+C) of dY), then
 // (mask != null) the ReLU backward of the layer that produced the upsampled tensor
 __global__ void up_bwd_kernel(const bf16 *__restrict__ dY, bf16 *__restrict__ dX, int C, int Ct, int off, int m,
@@ -737,16 +755,6 @@ __global__ void up_bwd_kernel(const bf16 *__restrict__ dY, bf16 *__restrict__ dX
             if (!(bf2f(mk[j]) > 0.f)) o[j] = (bf16)0.0f;
     }
     st8(dX + (size_t)q * C + 8 * cv, o);
-}
-
-// copy C channels between buffers with different channel counts / offsets
-__global__ void chan_copy_kernel(const bf16 *__restrict__ src, int Cs, int offs, bf16 *__restrict__ dst, int Cd,
-                                 int offd, int C, size_t npts) {
-    const unsigned V = C / 8;
-    const unsigned i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (unsigned)npts * V) return;
-    const unsigned p = i / V, cv = i % V;
-    st8(dst + (size_t)p * Cd + offd + 8 * cv, ld8(src + (size_t)p * Cs + offs + 8 * cv));
 }
 
 // input packing: host-order float planes [b][2][n^3] -> NDHWC BF16 with 8 channels (2 used)
@@ -937,7 +945,7 @@ struct cfm_unet {
     float *partial = nullptr;
     // activations
     bf16 *X0 = nullptr, *A0 = nullptr, *S1 = nullptr, *Q1 = nullptr, *A2 = nullptr, *S2 = nullptr, *Q2 = nullptr,
-         *A4 = nullptr, *A5 = nullptr, *U2 = nullptr, *A6 = nullptr, *A7 = nullptr, *U1 = nullptr, *A8 = nullptr,
+         *A4 = nullptr, *A5 = nullptr, *A6 = nullptr, *A7 = nullptr, *A8 = nullptr,
          *A9 = nullptr;
     float *pred = nullptr, *target = nullptr, *dpred = nullptr, *in_f = nullptr;
     double *lpart = nullptr;
@@ -1026,10 +1034,8 @@ extern "C" cfm_status cfm_unet_create(int n, int batch, cfm_unet **out) {
     A(&u->Q2, 2 * P3 * 32);
     A(&u->A4, 2 * P3 * 64);
     A(&u->A5, 2 * P3 * 64);
-    A(&u->U2, 2 * P2 * 96);
     A(&u->A6, 2 * P2 * 32);
     A(&u->A7, 2 * P2 * 32);
-    A(&u->U1, 2 * P1 * 48);
     A(&u->A8, 2 * P1 * 16);
     A(&u->A9, 2 * P1 * 16);
     A(&u->pred, 4 * P1);
@@ -1085,7 +1091,7 @@ extern "C" cfm_status cfm_unet_get_params(cfm_unet *u, float *params) {
 }
 
 template <int MT, int CIN>
-static bool launch_conv_lds(int n, int batch, hipStream_t st, const bf16 *X, const bf16 *W, int kp,
+static bool launch_conv_lds(int n, int batch, hipStream_t st, const bf16 *X, const bf16 *Xup, const bf16 *W, int kp,
                             const float *bias, bf16 *Y, int relu, const bf16 *mask) {
     if (kp != (27 * CIN + 31) / 32 * 32) return false;
     // tile 16 x TY x TZ points, the staged block at most 80 KiB of LDS (two workgroups per CU): up
@@ -1096,7 +1102,7 @@ static bool launch_conv_lds(int n, int batch, hipStream_t st, const bf16 *X, con
     static_assert((TZ + 2) * (TY + 2) * 18 * CIN * 2 <= 80 * 1024, "staged block above 80 KiB");
     const int nbx = (n + 15) / 16, nby = (n + TY - 1) / TY, nbz = (n + TZ - 1) / TZ;
     const dim3 grid((unsigned)(nbx * nby * nbz * batch));
-    hipLaunchKernelGGL((conv3_fwd_lds_kernel<MT, CIN, TY, TZ>), grid, dim3(256), 0, st, X, W, kp, bias, Y, n, nbx, nby,
+    hipLaunchKernelGGL((conv3_fwd_lds_kernel<MT, CIN, TY, TZ>), grid, dim3(256), 0, st, X, Xup, W, kp, bias, Y, n, nbx, nby,
                        nbz, relu, mask);
     return true;
 }
@@ -1110,7 +1116,7 @@ static bool launch_conv_lds(int n, int batch, hipStream_t st, const bf16 *X, con
 // wavefront; eight wavefronts (one row each) when the eight-row block is too large for two
 // workgroups per CU.
 template <int MT, int CIN, int NXT>
-static void launch_conv_xacc(int n, int batch, hipStream_t st, const bf16 *X, const bf16 *W, int kp,
+static void launch_conv_xacc(int n, int batch, hipStream_t st, const bf16 *X, const bf16 *Xup, const bf16 *W, int kp,
                              const float *bias, bf16 *Y, int relu, const bf16 *mask) {
     constexpr bool two = MT * NXT <= 4;
     constexpr int lds8 = NXT * 16 * 6 * 4 * CIN * 2;
@@ -1119,7 +1125,7 @@ static void launch_conv_xacc(int n, int batch, hipStream_t st, const bf16 *X, co
     static_assert(NXT * 16 * (TY + 2) * (TZ + 2) * CIN * 2 <= 144 * 1024, "staged block above 144 KiB");
     const int nby = (n + TY - 1) / TY, nbz = (n + TZ - 1) / TZ;
     hipLaunchKernelGGL((conv3_fwd_xacc_kernel<MT, CIN, TY, TZ, NXT, NW, 2>), dim3((unsigned)(nby * nbz * batch)),
-                       dim3(64 * NW), 0, st, X, W, kp, bias, Y, n, nby, nbz, relu, mask);
+                       dim3(64 * NW), 0, st, X, Xup, W, kp, bias, Y, n, nby, nbz, relu, mask);
 }
 
 // The x-accumulator kernel where it measured faster than the per-tap one: the wide inputs of
@@ -1128,13 +1134,13 @@ static void launch_conv_xacc(int n, int batch, hipStream_t st, const bf16 *X, co
 // staged block keeps 3 to 7 workgroups per CU against 1 to 3 and won (16 -> 16: 0.33 vs 0.41
 // ms), and the 16 -> 48 and 32 -> 96 data gradients need 3 x 3 and 3 x 6 accumulator tiles per
 // row: one wavefront per SIMD, twice the time.
-static bool conv_xacc(int cin, int mt, int n, int batch, hipStream_t st, const bf16 *X, const bf16 *W, int kp,
+static bool conv_xacc(int cin, int mt, int n, int batch, hipStream_t st, const bf16 *X, const bf16 *Xup, const bf16 *W, int kp,
                       const float *bias, bf16 *Y, int relu, const bf16 *mask) {
     if (!CFM_UNET_XACC || n > 64 || kp < 27 * cin) return false;
     const int nxt = n <= 16 ? 1 : n <= 32 ? 2 : 4;
 #define CFM_CONV_XACC(C, M, T)                                               \
     if (cin == C && mt == M && nxt == T) {                                   \
-        launch_conv_xacc<M, C, T>(n, batch, st, X, W, kp, bias, Y, relu, mask); \
+        launch_conv_xacc<M, C, T>(n, batch, st, X, Xup, W, kp, bias, Y, relu, mask); \
         return true;                                                         \
     }
     CFM_CONV_XACC(48, 1, 4)
@@ -1147,11 +1153,11 @@ static bool conv_xacc(int cin, int mt, int n, int batch, hipStream_t st, const b
 }
 
 // the (input channels, output channel tiles) pairs of the network's forward and data-gradient convs
-static bool conv_lds(int cin, int mt, int n, int batch, hipStream_t st, const bf16 *X, const bf16 *W, int kp,
+static bool conv_lds(int cin, int mt, int n, int batch, hipStream_t st, const bf16 *X, const bf16 *Xup, const bf16 *W, int kp,
                      const float *bias, bf16 *Y, int relu, const bf16 *mask) {
 #define CFM_CONV_LDS(C, M)                                                  \
     if (cin == C && mt == M) {                                              \
-        return launch_conv_lds<M, C>(n, batch, st, X, W, kp, bias, Y, relu, mask); \
+        return launch_conv_lds<M, C>(n, batch, st, X, Xup, W, kp, bias, Y, relu, mask); \
     }
     CFM_CONV_LDS(8, 1)
     CFM_CONV_LDS(16, 1)
@@ -1172,11 +1178,11 @@ static bool conv_lds(int cin, int mt, int n, int batch, hipStream_t st, const bf
 // Y = conv(X) for the (input channels, output channels) pairs of the network
 // mask (may be null): the data gradient of a ReLU layer, zero where mask (the layer's forward
 // output, [points][cout]) is not positive
-static cfm_status conv_fwd(cfm_unet *u, const bf16 *X, int cin, const bf16 *W, int kp, const float *bias, bf16 *Y,
+static cfm_status conv_fwd(cfm_unet *u, const bf16 *X, const bf16 *Xup, int cin, const bf16 *W, int kp, const float *bias, bf16 *Y,
                            int cout, int level, int relu, const bf16 *mask = nullptr) {
     const int n = u->n >> level;
-    if (cout % 16 != 0 || !(conv_xacc(cin, cout / 16, n, u->batch, u->stream, X, W, kp, bias, Y, relu, mask) ||
-                            conv_lds(cin, cout / 16, n, u->batch, u->stream, X, W, kp, bias, Y, relu, mask)))
+    if (cout % 16 != 0 || !(conv_xacc(cin, cout / 16, n, u->batch, u->stream, X, Xup, W, kp, bias, Y, relu, mask) ||
+                            conv_lds(cin, cout / 16, n, u->batch, u->stream, X, Xup, W, kp, bias, Y, relu, mask)))
         return CFM_FAIL(CFM_EINVAL, "unet: no convolution kernel for %d -> %d channels", cin, cout);
     CFM_HIP(hipGetLastError());
     return CFM_OK;
@@ -1190,8 +1196,9 @@ static cfm_status run_forward_dev(cfm_unet *u, const float *d_in) {
     const float *b[kNConv];
     for (int i = 0; i < kNConv; ++i) b[i] = u->master + u->boff[i];
     cfm_status st;
-#define CONV(I, X, Y) \
-    if ((st = conv_fwd(u, X, kConv[I].cin, u->Wf[I], u->Kp[I], b[I], Y, kConv[I].cout, kConv[I].level, 1)) != CFM_OK) return st
+#define CONV(I, X, Y) CONV2(I, X, nullptr, Y)
+#define CONV2(I, X, XUP, Y) \
+    if ((st = conv_fwd(u, X, XUP, kConv[I].cin, u->Wf[I], u->Kp[I], b[I], Y, kConv[I].cout, kConv[I].level, 1)) != CFM_OK) return st
     CONV(0, u->X0, u->A0);
     CONV(1, u->A0, u->S1);
     hipLaunchKernelGGL(pool_fwd_kernel, blocks_for(P2 * 16 / 8), dim3(256), 0, u->stream, u->S1, u->Q1, 16, n, u->batch);
@@ -1200,15 +1207,12 @@ static cfm_status run_forward_dev(cfm_unet *u, const float *d_in) {
     hipLaunchKernelGGL(pool_fwd_kernel, blocks_for(u->P[2] * 32 / 8), dim3(256), 0, u->stream, u->S2, u->Q2, 32, n / 2, u->batch);
     CONV(4, u->Q2, u->A4);
     CONV(5, u->A4, u->A5);
-    hipLaunchKernelGGL(up_fwd_kernel, blocks_for(P2 * 64 / 8), dim3(256), 0, u->stream, u->A5, u->U2, 64, 96, 0, n / 4, u->batch);
-    hipLaunchKernelGGL(chan_copy_kernel, blocks_for(P2 * 32 / 8), dim3(256), 0, u->stream, u->S2, 32, 0, u->U2, 96, 64, 32, P2);
-    CONV(6, u->U2, u->A6);
+    CONV2(6, u->S2, u->A5, u->A6);
     CONV(7, u->A6, u->A7);
-    hipLaunchKernelGGL(up_fwd_kernel, blocks_for(P1 * 32 / 8), dim3(256), 0, u->stream, u->A7, u->U1, 32, 48, 0, n / 2, u->batch);
-    hipLaunchKernelGGL(chan_copy_kernel, blocks_for(P1 * 16 / 8), dim3(256), 0, u->stream, u->S1, 16, 0, u->U1, 48, 32, 16, P1);
-    CONV(8, u->U1, u->A8);
+    CONV2(8, u->S1, u->A7, u->A8);
     CONV(9, u->A8, u->A9);
 #undef CONV
+#undef CONV2
     hipLaunchKernelGGL(head_fwd_kernel, blocks_for(P1), dim3(256), 0, u->stream, u->A9, u->master + u->head_off,
                        u->pred, P1);
     CFM_HIP(hipGetLastError());
@@ -1239,22 +1243,22 @@ extern "C" cfm_status cfm_unet_forward(cfm_unet *u, const float *input, float *o
 }
 
 template <int CIN, int COUT>
-static void launch_wgrad_rows(int nslab, hipStream_t st, const bf16 *X, const bf16 *dZ, int kp, float *partial,
+static void launch_wgrad_rows(int nslab, hipStream_t st, const bf16 *X, const bf16 *Xup, const bf16 *dZ, int kp, float *partial,
                               const WgradShape &S) {
     const size_t lds = sizeof(bf16) * ((size_t)COUT * 72 + (size_t)3 * (S.rows + 2) * kWgradRows16);
     // (short rows, eight to a block, take more than 64 KiB)
     static const bool big_lds_ok = hipFuncSetAttribute((const void *)conv3_wgrad_rows_kernel<CIN, COUT>,
                                                        hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) == hipSuccess;
     (void)big_lds_ok;
-    hipLaunchKernelGGL((conv3_wgrad_rows_kernel<CIN, COUT>), dim3(nslab, (CIN + 15) / 16), dim3(192), lds, st, X, dZ, kp,
-                       partial, S);
+    hipLaunchKernelGGL((conv3_wgrad_rows_kernel<CIN, COUT>), dim3(nslab, (CIN + 15) / 16), dim3(192), lds, st, X, Xup,
+                       dZ, kp, partial, S);
 }
 
-static bool wgrad_rows(int cin, int cout, int nslab, hipStream_t st, const bf16 *X, const bf16 *dZ, int kp,
+static bool wgrad_rows(int cin, int cout, int nslab, hipStream_t st, const bf16 *X, const bf16 *Xup, const bf16 *dZ, int kp,
                        float *partial, const WgradShape &S) {
 #define CFM_WGRAD_ROWS(C, O)                                             \
     if (cin == C && cout == O) {                                         \
-        launch_wgrad_rows<C, O>(nslab, st, X, dZ, kp, partial, S);       \
+        launch_wgrad_rows<C, O>(nslab, st, X, Xup, dZ, kp, partial, S);  \
         return true;                                                     \
     }
     CFM_WGRAD_ROWS(8, 16)
@@ -1270,12 +1274,12 @@ static bool wgrad_rows(int cin, int cout, int nslab, hipStream_t st, const bf16 
 }
 
 // gradients of conv I's weights and biases from its input X and output gradient dZ
-static cfm_status conv_wgrad(cfm_unet *u, int I, const bf16 *X, const bf16 *dZ) {
+static cfm_status conv_wgrad(cfm_unet *u, int I, const bf16 *X, const bf16 *dZ, const bf16 *Xup = nullptr) {
     const ConvSpec &s = kConv[I];
     const int Kp = u->Kp[I], count = s.cout * (Kp + 1);
     int nslab;
     const WgradShape S = wgrad_shape(u->n >> s.level, u->batch, s.cin, &nslab);
-    if (!wgrad_rows(s.cin, s.cout, nslab, u->stream, X, dZ, Kp, u->partial, S))
+    if (!wgrad_rows(s.cin, s.cout, nslab, u->stream, X, Xup, dZ, Kp, u->partial, S))
         return CFM_FAIL(CFM_EINVAL, "unet: no weight-gradient kernel for %d -> %d channels", s.cin, s.cout);
     CFM_HIP(hipGetLastError());
     const float *part = u->partial;
@@ -1296,7 +1300,7 @@ static cfm_status conv_wgrad(cfm_unet *u, int I, const bf16 *X, const bf16 *dZ) 
 // forward output of the ReLU layer feeding conv I), the gradient before that ReLU
 static cfm_status conv_dgrad(cfm_unet *u, int I, const bf16 *dZ, bf16 *dX, const bf16 *mask = nullptr) {
     const ConvSpec &s = kConv[I];
-    return conv_fwd(u, dZ, s.cout, u->Wt[I], u->Kpt[I], nullptr, dX, s.cin, s.level, 0, mask);
+    return conv_fwd(u, dZ, nullptr, s.cout, u->Wt[I], u->Kpt[I], nullptr, dX, s.cin, s.level, 0, mask);
 }
 
 static cfm_status run_backward(cfm_unet *u, const float *target_host, double *loss) {
@@ -1322,14 +1326,14 @@ static cfm_status run_backward(cfm_unet *u, const float *target_host, double *lo
     // decoder level 1
     CK(conv_wgrad(u, 9, u->A8, u->g1b));
     CK(conv_dgrad(u, 9, u->g1b, u->g1a, u->A8));       // dZ8
-    CK(conv_wgrad(u, 8, u->U1, u->g1a));
+    CK(conv_wgrad(u, 8, u->S1, u->g1a, u->A7));
     CK(conv_dgrad(u, 8, u->g1a, u->g1c));               // dU1 [P1][48]
     hipLaunchKernelGGL(up_bwd_kernel, blocks_for(P2 * 32 / 8), dim3(256), 0, u->stream, u->g1c, u->g2b, 32, 48, 0,
                        n / 2, u->batch, u->A7);          // dZ7
     // decoder level 2
     CK(conv_wgrad(u, 7, u->A6, u->g2b));
     CK(conv_dgrad(u, 7, u->g2b, u->g2a, u->A6));       // dZ6
-    CK(conv_wgrad(u, 6, u->U2, u->g2a));
+    CK(conv_wgrad(u, 6, u->S2, u->g2a, u->A5));
     CK(conv_dgrad(u, 6, u->g2a, u->g2c));               // dU2 [P2][96]
     hipLaunchKernelGGL(up_bwd_kernel, blocks_for(P3 * 64 / 8), dim3(256), 0, u->stream, u->g2c, u->g3b, 64, 96, 0,
                        n / 4, u->batch, u->A5);          // dZ5
