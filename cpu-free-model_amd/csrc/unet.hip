@@ -88,17 +88,26 @@ __global__ void __launch_bounds__(256) conv3_fwd_lds_kernel(const bf16 *__restri
     const int x0 = bx * 16, y0 = by * TY, z0 = bz * TZ;
     const bf16x8 zero8 = {(bf16)0.0f, (bf16)0.0f, (bf16)0.0f, (bf16)0.0f,
                           (bf16)0.0f, (bf16)0.0f, (bf16)0.0f, (bf16)0.0f};
-    for (int v = threadIdx.x; v < HZ * HY * HX * NV; v += 256) {
-        const int cv = v % NV;
-        int r = v / NV;
-        const int cx = r % HX;
-        r /= HX;
-        const int cy = r % HY, cz = r / HY;
-        const int gx = x0 - 1 + cx, gy = y0 - 1 + cy, gz = z0 - 1 + cz;
-        bf16x8 val = zero8;
-        if (gx >= 0 && gx < n && gy >= 0 && gy < n && gz >= 0 && gz < n)
-            val = input8<CIN>(X, Xup, n, b, gz, gy, gx, cv);
-        blk[v] = val;
+    // (the loads of U vectors go out before the first of them is stored: one after the other they would
+    // each wait out the latency of the memory)
+    constexpr int TOTAL = HZ * HY * HX * NV, TURNS = (TOTAL + 255) / 256, U = TURNS < 6 ? TURNS : 6;
+#pragma unroll
+    for (int i0 = 0; i0 < TURNS; i0 += U) {
+        bf16x8 val[U];
+#pragma unroll
+        for (int i = 0; i < U; ++i) {
+            const int v = threadIdx.x + (i0 + i) * 256;
+            const int cv = v % NV, cx = v / NV % HX, cy = v / (NV * HX) % HY, cz = v / (NV * HX * HY);
+            const int gx = x0 - 1 + cx, gy = y0 - 1 + cy, gz = z0 - 1 + cz;
+            val[i] = zero8;
+            if (v < TOTAL && gx >= 0 && gx < n && gy >= 0 && gy < n && gz >= 0 && gz < n)
+                val[i] = input8<CIN>(X, Xup, n, b, gz, gy, gx, cv);
+        }
+#pragma unroll
+        for (int i = 0; i < U; ++i) {
+            const int v = threadIdx.x + (i0 + i) * 256;
+            if (v < TOTAL) blk[v] = val[i];
+        }
     }
     __syncthreads();
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -198,17 +207,24 @@ __global__ void __launch_bounds__(64 * NW) conv3_fwd_xacc_kernel(const bf16 *__r
     const int y0 = by * TY, z0 = bz * TZ;
     const bf16x8 zero8 = {(bf16)0.0f, (bf16)0.0f, (bf16)0.0f, (bf16)0.0f,
                           (bf16)0.0f, (bf16)0.0f, (bf16)0.0f, (bf16)0.0f};
-    for (int v = threadIdx.x; v < HZ * HY * XW * NV; v += 64 * NW) {
-        const int cv = v % NV;
-        int r = v / NV;
-        const int cx = r % XW;
-        r /= XW;
-        const int cy = r % HY, cz = r / HY;
-        const int gy = y0 - 1 + cy, gz = z0 - 1 + cz;
-        bf16x8 val = zero8;
-        if (cx < n && gy >= 0 && gy < n && gz >= 0 && gz < n)
-            val = input8<CIN>(X, Xup, n, b, gz, gy, cx, cv);
-        blk[v] = val;
+    constexpr int TOTAL = HZ * HY * XW * NV, TURNS = (TOTAL + 64 * NW - 1) / (64 * NW), U = TURNS < 6 ? TURNS : 6;
+#pragma unroll
+    for (int i0 = 0; i0 < TURNS; i0 += U) {  // (U loads in flight)
+        bf16x8 val[U];
+#pragma unroll
+        for (int i = 0; i < U; ++i) {
+            const int v = threadIdx.x + (i0 + i) * 64 * NW;
+            const int cv = v % NV, cx = v / NV % XW, cy = v / (NV * XW) % HY, cz = v / (NV * XW * HY);
+            const int gy = y0 - 1 + cy, gz = z0 - 1 + cz;
+            val[i] = zero8;
+            if (v < TOTAL && cx < n && gy >= 0 && gy < n && gz >= 0 && gz < n)
+                val[i] = input8<CIN>(X, Xup, n, b, gz, gy, cx, cv);
+        }
+#pragma unroll
+        for (int i = 0; i < U; ++i) {
+            const int v = threadIdx.x + (i0 + i) * 64 * NW;
+            if (v < TOTAL) blk[v] = val[i];
+        }
     }
     __syncthreads();
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
