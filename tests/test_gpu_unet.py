@@ -60,6 +60,19 @@ def test_gradient_matches_oracle(cfm, gpu, n, batch):
     assert _rel(g[off:], rg[off:]) < 1e-2
 
 
+def test_forward_in_parts(cfm, gpu):
+    """A batch large enough to be launched in two (here uneven) parts gives each sample what it gets alone."""
+    n, batch = 64, 3
+    params, inp, _ = _case(60, n, batch)
+    with cfm.UNet(n, batch, params=params) as net:
+        out = net.forward(inp)
+        again = net.forward(inp[::-1].copy())
+    assert np.array_equal(again[::-1], out)
+    with cfm.UNet(n, 1, params=params) as one:
+        for i in range(batch):
+            assert np.array_equal(one.forward(inp[i:i + 1])[0], out[i])
+
+
 def test_gradient_is_deterministic(cfm, gpu):
     params, inp, target = _case(31, 16, 2)
     with cfm.UNet(16, 2, params=params) as net:
