@@ -998,7 +998,7 @@ extern "C" size_t cfm_unet_param_count(void) { return param_count(); }
 extern "C" cfm_status cfm_unet_create(int n, int batch, cfm_unet **out) {
     if (!out) return CFM_EINVAL;
     *out = nullptr;
-    // batch * n^3 <= 2^27 keeps the weight-gradient slab count (points / 4096) within a grid's y extent
+    // batch * n^3 <= 2^27 keeps the elementwise kernels' and the weight gradients' offsets within 32 bits
     if (n < 4 || n % 4 != 0 || batch < 1 || (long long)batch * n * n * n > (1LL << 27)) return CFM_EINVAL;
     int ndev = 0;
     if (hipGetDeviceCount(&ndev) != hipSuccess || ndev < 1) return CFM_EDEVICE;
