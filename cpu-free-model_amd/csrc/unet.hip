@@ -1249,14 +1249,19 @@ static cfm_status run_forward_dev(cfm_unet *u, const float *d_in, int b0, int nb
 
 // Parts of the batch that the forward pass is launched in.  In two, the first part's kernels run while
 // the host copies the second part in (and, for an output, the second part's while the first is
-// copied out): 8 x 64^3 1.64 ms against 1.96 in one.  Parts of fewer points than these would leave the
-// deep levels' kernels few workgroups, for a copy that is over sooner than they are.
-static int forward_parts(const cfm_unet *u) { return u->batch >= 2 && u->P[0] >= ((size_t)1 << 19) ? 2 : 1; }
+// copied out): 8 x 64^3 1.61 ms against 1.96 in one.  Parts of fewer points than these would leave the
+// deep levels' kernels few workgroups, for a copy that is over sooner than they are (2 x 64^3 648 us in
+// two parts, 619 before; 12 x 36^3 799 and 781).
+static int forward_parts(const cfm_unet *u) { return u->batch >= 2 && u->P[0] >= ((size_t)1 << 20) ? 2 : 1; }
 
-// Copies the input in and enqueues the forward pass; done[p] is recorded after part p.
+// Copies the input in and enqueues the forward pass; with several parts, done[p] is recorded after part p.
 static cfm_status run_forward(cfm_unet *u, const float *input_host) {
     const int parts = forward_parts(u);
     const size_t each = 2 * (u->P[0] / u->batch);
+    if (parts == 1) {  // (nothing to run beside: a second stream would only add its waits, 17 us of a small pass's 233)
+        CFM_HIP(hipMemcpyAsync(u->in_f, input_host, 4 * each * u->batch, hipMemcpyHostToDevice, u->stream));
+        return run_forward_dev(u, u->in_f, 0, u->batch);
+    }
     for (int p = 0; p < parts; ++p) {
         const int b0 = u->batch * p / parts, nb = u->batch * (p + 1) / parts - b0;
         CFM_HIP(hipMemcpyAsync(u->in_f + each * b0, input_host + each * b0, 4 * each * nb, hipMemcpyHostToDevice, u->copies));
@@ -1284,6 +1289,11 @@ extern "C" cfm_status cfm_unet_forward(cfm_unet *u, const float *input, float *o
     if (st != CFM_OK) return st;
     const int parts = forward_parts(u);
     const size_t each = u->P[0] / u->batch;
+    if (parts == 1) {
+        CFM_HIP(hipMemcpyAsync(output, u->pred, 4 * u->P[0], hipMemcpyDeviceToHost, u->stream));
+        CFM_HIP(hipStreamSynchronize(u->stream));
+        return CFM_OK;
+    }
     for (int p = 0; p < parts; ++p) {
         const int b0 = u->batch * p / parts, nb = u->batch * (p + 1) / parts - b0;
         CFM_HIP(hipStreamWaitEvent(u->copies, u->done[p], 0));
@@ -1358,10 +1368,13 @@ static cfm_status conv_dgrad(cfm_unet *u, int I, const bf16 *dZ, bf16 *dX, const
 static cfm_status run_backward(cfm_unet *u, const float *target_host, double *loss) {
     const size_t P1 = u->P[0], P2 = u->P[1], P3 = u->P[2];
     const int n = u->n;
-    // (on the copies' stream: the forward pass still runs)
-    CFM_HIP(hipMemcpyAsync(u->target, target_host, 4 * P1, hipMemcpyHostToDevice, u->copies));
-    CFM_HIP(hipEventRecord(u->copied, u->copies));
-    CFM_HIP(hipStreamWaitEvent(u->stream, u->copied, 0));
+    if (forward_parts(u) > 1) {  // beside the forward pass, which still runs
+        CFM_HIP(hipMemcpyAsync(u->target, target_host, 4 * P1, hipMemcpyHostToDevice, u->copies));
+        CFM_HIP(hipEventRecord(u->copied, u->copies));
+        CFM_HIP(hipStreamWaitEvent(u->stream, u->copied, 0));
+    } else {
+        CFM_HIP(hipMemcpyAsync(u->target, target_host, 4 * P1, hipMemcpyHostToDevice, u->stream));
+    }
     const unsigned nb1 = (unsigned)((P1 + 255) / 256);
     hipLaunchKernelGGL(mse_kernel, dim3(nb1), dim3(256), 0, u->stream, u->pred, u->target, u->dpred, u->lpart, P1);
     const float *hw = u->master + u->head_off;

@@ -62,7 +62,7 @@ def test_gradient_matches_oracle(cfm, gpu, n, batch):
 
 def test_forward_in_parts(cfm, gpu):
     """A batch large enough to be launched in two (here uneven) parts gives each sample what it gets alone."""
-    n, batch = 64, 3
+    n, batch = 64, 5
     params, inp, _ = _case(60, n, batch)
     with cfm.UNet(n, batch, params=params) as net:
         out = net.forward(inp)
