@@ -31,7 +31,7 @@ struct VecAt {
 };
 
 // A lane's N elements at row[x .. x+N), and one of them.  THROUGH: past the L2 (scope bit sc1), for
-// grid_barrier_through; rows are then shorter than 2 GiB.
+// grid_barrier_through; offsets are 32-bit, so jacobi_tile_configure declines rows of 2 GiB and more.
 constexpr int kSc1 = 16;  // buffer instructions' cache policy bit
 template <bool THROUGH, typename T, int N>
 __device__ __forceinline__ typename VecAt<T, N>::type load_at(const T *row, int x) {
@@ -401,8 +401,9 @@ double pass_us(const cfm_jacobi_params &p, const Shape2D &s, int depth, int cus)
 }  // namespace
 
 bool jacobi_tile_configure(const cfm_jacobi_params &p, JacobiConfig *c) {
-    if (p.nz >= 3) return false;
     const bool f64 = p.prec == CFM_F64;
+    // a row's byte offsets are 32-bit, and a buffer's range check drops what lies beyond 2 GiB
+    if (p.nz >= 3 || (double)p.nx * (f64 ? 8 : 4) > 0x7fffffff) return false;
     // 16-wavefront shapes for fields of few tiles (short rows of work per wavefront, one
     // workgroup per CU); 14 (FP32: 13, 14 spills when timed) rows in 8 wavefronts, two workgroups per CU that hide each other's
     // loads, for fields of many (16384^2 FP64 x 48 sweeps: 5.3 ms against 5.7 for 8 x 16).
