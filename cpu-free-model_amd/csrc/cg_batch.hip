@@ -548,14 +548,13 @@ static cfm_status batch_use_resident(cfm_cg_batch_plan *pl) {
     return CFM_OK;
 }
 
-// The resident kernel's schedule, for SELL-64 plans whose systems each fit the chip.  With rounds a
-// workgroup may wait for members still at their previous systems, so a short watchdog keeps one round.
+// The resident kernel's schedule, for SELL-64 plans whose systems each fit the chip.
 static cfm_status batch_plan_resident(cfm_cg_batch_plan *pl, int max_width) {
     int grid = 0, rounds = 0;
     const BatchResidentFn fn = batch_resident_kernel(max_width, pl->dev, &grid);
     if (!fn) return CFM_OK;
     const std::vector<TeamSlot> slots = batch_resident_schedule(pl->h_chunk0, grid, &rounds);
-    if (slots.empty() || (rounds > 1 && pl->p.spin_limit_us > 0)) return CFM_OK;
+    if (slots.empty()) return CFM_OK;
     CFM_HIP(hipMalloc((void **)&pl->res_slots, sizeof(TeamSlot) * slots.size()));
     CFM_HIP(hipMalloc((void **)&pl->team, sizeof(TeamSync)));
     CFM_HIP(hipMemcpy(pl->res_slots, slots.data(), sizeof(TeamSlot) * slots.size(), hipMemcpyHostToDevice));

@@ -39,31 +39,51 @@ struct Team {
     unsigned long long epoch;
 };
 
+// The sum of the launch's arrival words.  They only grow, and a workgroup that iterates passes a barrier
+// in every iteration: as long as any does, the sum grows.
+__device__ __forceinline__ unsigned long long arrivals(const TeamSync *s) {
+    unsigned long long sum = 0;
+    for (int b = 0; b < (int)gridDim.x; ++b)
+        sum += __hip_atomic_load(&s->arrive[b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return sum;
+}
+
 // grid_barrier_through for one team: arrivals to its first workgroup, which releases every member on a
 // line of its own (a line that only that member reads: no release of an earlier team can be late).
+// At the first barrier of a later round members may still be at their previous systems, for as long as
+// those take: that wait's clock starts anew while the launch makes progress.  (All others wait for at
+// most an iteration.)
 __device__ __forceinline__ bool team_barrier(Team &T) {
     __shared__ int s_abort;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     const unsigned long long e = ++T.epoch;
-    if (T.size == 1) return true;
     TeamSync *s = T.s;
-    const unsigned long long limit = s->spin_limit_ticks;
-    int ab = 0;
-    if (threadIdx.x == 0) {
-        s_abort = 0;
+    if (threadIdx.x == 0)
         __hip_atomic_store(&s->arrive[T.me], e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
+    if (T.size == 1) return true;
+    const unsigned long long limit = s->spin_limit_ticks;
+    const bool patient = (unsigned)e == 1 && (e >> 32) > 1;
+    int ab = 0;
+    if (threadIdx.x == 0) s_abort = 0;
     const bool gather = T.me == T.base;
     if (gather) __syncthreads();
     if (gather || threadIdx.x == 0) {
-        const unsigned long long t0 = __builtin_amdgcn_s_memrealtime();
+        unsigned long long t0 = __builtin_amdgcn_s_memrealtime(), seen = 0;
         const unsigned long long *first = gather ? &s->arrive[T.base + threadIdx.x] : &s->go[16 * T.me];
         const int count = gather ? T.size - (int)threadIdx.x : 1;
         for (int b = 0; b < count && !ab; b += blockDim.x) {
             while (__hip_atomic_load(first + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < e) {
-                if (__hip_atomic_load(&s->abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ||
-                    spin_expired(t0, limit)) {
+                const bool late = spin_expired(t0, limit);
+                if (late && patient) {
+                    const unsigned long long now = arrivals(s);
+                    if (now != seen) {
+                        seen = now;
+                        t0 = __builtin_amdgcn_s_memrealtime();
+                        continue;
+                    }
+                }
+                if (late || __hip_atomic_load(&s->abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
                     __hip_atomic_store(&s->abort, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                     ab = 1;
                     break;

@@ -57,3 +57,34 @@ def test_batch_resident_largest_system(gpu, orc):
 def test_batch_resident_guard(gpu, orc, tol, max_iter):
     systems = [gpu.poisson3d(10, 11, 12), gpu.poisson3d(20, 9, 14), gpu.tridiag(4000, 9)]
     _check(gpu, orc, systems, tol=tol, max_iter=max_iter, guard=1, bad=(1,))
+
+
+def _line(n):
+    """The 1D Laplacian (about n iterations to converge)."""
+    col = (np.arange(n)[:, None] + np.arange(-1, 2)).astype(np.int32)
+    ok = (col >= 0) & (col < n)
+    rp = np.zeros(n + 1, dtype=np.int32)
+    rp[1:] = np.cumsum(ok.sum(1))
+    return rp, col[ok], np.broadcast_to([-1.0, 2.0, -1.0], col.shape)[ok]
+
+
+def test_batch_resident_waits_for_longer_systems(gpu):
+    """A team of the second round whose members come from a system of the first round that ends at once and from one
+    that iterates for many times the watchdog's limit waits for the latter, and solves its system as a solve alone does."""
+    chunks = (260, 250, 240, 230, 225)  # rounds {260, 250, 240} and {230, 225}; the last spans the first two
+    max_iter, limit_us = 3000, 2000
+    systems = [_line(1024 * c) for c in chunks]
+    srp, rp, col, val = gpu.block_diag(systems)
+    b = gpu.uniform(8, 0, int(srp[-1])) - 0.5
+    b[srp[1]:srp[4]] = 0.0  # solved by x0 = 0
+    p = gpu.cg_params(method=gpu.CG_PIPELINED, tol=1e-8, max_iter=max_iter, spin_limit_us=limit_us)
+    with gpu.CgBatchPlan(srp, rp, col, val, p) as plan:
+        plan.set_rhs(b)
+        plan.set_x0(None)
+        st, iters, stat, _, t = plan.solve()
+        x = plan.x()
+    assert t["block_threads"] == 256 and t["kernel_ms"] > 5e-3 * limit_us
+    assert st == gpu.ENOTCONV and list(iters) == [max_iter, 0, 0, 0, max_iter]
+    for s in (0, 4):
+        alone = gpu.cg(*systems[s], b[srp[s]:srp[s + 1]], method=gpu.CG_PIPELINED, tol=1e-8, max_iter=max_iter)
+        assert alone[0] == gpu.ENOTCONV and np.array_equal(x[srp[s]:srp[s + 1]], alone[1])
