@@ -338,7 +338,8 @@ __global__ void __launch_bounds__(64 * NW) conv3_fwd_xacc_kernel(const bf16 *__r
 // one input channel, shifted by dx) comes from two aligned 16-byte LDS reads:
 // dx = -1 is the first, dx = +1 the dwords 1..4, dx = 0 a 2-byte byte-align of
 // the pair.  Input channels below 16 are padded with zero rows (the first layer's
-// 8).  The bias gradient is one more product, with a B fragment of ones.
+// 8).  The bias gradient is one more product, with a B fragment of ones; every kBiasBlocks blocks its
+// sums go to FP64 ones in LDS.
 // blockIdx.y: the group of 16 input channels that the workgroup stages and computes.
 // Bound by latency and by the vector instructions of the staging: blocks follow one another along y,
 // the rows that the last block had stay in LDS, the new ones and the next dZ are loaded while a block is
@@ -348,6 +349,7 @@ __global__ void __launch_bounds__(64 * NW) conv3_fwd_xacc_kernel(const bf16 *__r
 // staged the input anew for each of the 27 taps.
 constexpr int kWgradRow = 72;  // a staged input row: 64 points, one at each end, and padding that keeps fragments 16-byte aligned
 constexpr int kWgradRows16 = 16 * (kWgradRow + 1);  // and that of 16 channels
+constexpr int kBiasBlocks = 8;
 struct WgradShape {
     int n, nblk, per_slab;  // points along an edge; blocks, and blocks a workgroup takes
     int w8, rows, nyb, nseg;  // a row's padded points, rows of a block, blocks along y and x
@@ -355,7 +357,7 @@ struct WgradShape {
 };
 
 template <int CIN, int COUT>
-__global__ void __launch_bounds__(192) conv3_wgrad_rows_kernel(const bf16 *__restrict__ Xg,
+__global__ void __launch_bounds__(192, COUT == 16 ? 3 : 1) conv3_wgrad_rows_kernel(const bf16 *__restrict__ Xg,
                                                                         const bf16 *__restrict__ Xup,
                                                                         const bf16 *__restrict__ dZ, int Kp,
                                                                         float *__restrict__ partial, WgradShape S) {
@@ -378,6 +380,7 @@ __global__ void __launch_bounds__(192) conv3_wgrad_rows_kernel(const bf16 *__res
     bf16 *xT = wg_lds + COUT * DS;
     constexpr int W = kWgradRow, RSTR = CINP * (W + 1);
     static_assert(RSTR == kWgradRows16, "as the launch counts it");
+    double *biasT = reinterpret_cast<double *>(xT + 3 * (R + 2) * RSTR);  // [COUT], a lane's own each
     const int s = blockIdx.x;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int nl = lane & 15, g = lane >> 4;
@@ -400,6 +403,12 @@ __global__ void __launch_bounds__(192) conv3_wgrad_rows_kernel(const bf16 *__res
                 for (int k = 0; k < KT; ++k) acc[a][d][m][k] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int m = 0; m < MT; ++m) accb[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const bool bias = w == 0 && blockIdx.y == 0;  // (uniform over the wavefront)
+    if (bias && nl == 0)
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) biasT[m * 16 + 4 * g + i] = 0.0;
     // this lane's first point in each of the two K steps: its row in the block and its column (a
     // group beyond the last row multiplies zeros of dZ with any staged row)
     int rq[2], xg[2];
@@ -533,7 +542,7 @@ __global__ void __launch_bounds__(192) conv3_wgrad_rows_kernel(const bf16 *__res
             bf16x8 av[MT];
 #pragma unroll
             for (int m = 0; m < MT; ++m) av[m] = *reinterpret_cast<const bf16x8 *>(&dzT[(m * 16 + nl) * DS + q]);
-            if (w == 0) {
+            if (bias) {
 #pragma unroll
                 for (int m = 0; m < MT; ++m)
                     accb[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[m], one8, accb[m], 0, 0, 0);
@@ -566,6 +575,15 @@ __global__ void __launch_bounds__(192) conv3_wgrad_rows_kernel(const bf16 *__res
                 }
             }
         }
+        if (bias && ((blk - s * S.per_slab) % kBiasBlocks == kBiasBlocks - 1 || blk + 1 == blk_end)) {
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
+                if (nl == 0)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) biasT[m * 16 + 4 * g + i] += (double)accb[m][i];
+                accb[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+            }
+        }
         __syncthreads();  // the staged rows are rewritten next
         if (more) {
 #pragma unroll
@@ -596,19 +614,22 @@ __global__ void __launch_bounds__(192) conv3_wgrad_rows_kernel(const bf16 *__res
         }
     }
     // (the K tail [27 CIN, Kp) is left as it is: nothing reads it)
-    if (w == 0 && blockIdx.y == 0 && nl == 0) {
+    if (bias && nl == 0) {
 #pragma unroll
         for (int m = 0; m < MT; ++m)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) out[(size_t)COUT * Kp + m * 16 + 4 * g + i] = accb[m][i];
+            for (int i = 0; i < 4; ++i)
+                out[(size_t)COUT * Kp + m * 16 + 4 * g + i] = (float)biasT[m * 16 + 4 * g + i];
     }
 }
 
 // The slabs' sums, part[s][i] in the fixed order s = 0, 1, ..., for i < COUT (Kp + 1), taken
 // from the kernel layout (co, k = tap*Cin + ci; then the bias) to the master order [Cout][Cin_real][27]
-// and [Cout].  Eight loads are issued before their eight in-order adds, so the memory latency is
+// and [Cout].  In FP64: there may be thousands of slabs, and the sums are bound by the loads.  Eight
+// loads are issued before their eight in-order adds, so the memory latency is
 // paid once per eight slabs instead of once per slab.
-__global__ void reduce_slabs_kernel(const float *__restrict__ part, int nslab, int Cout, int Cin_real, int Cin, int Kp,
+template <typename T>
+__global__ void reduce_slabs_kernel(const T *__restrict__ part, int nslab, int Cout, int Cin_real, int Cin, int Kp,
                                     float *__restrict__ g, float *__restrict__ gb) {
     const int count = Cout * (Kp + 1);
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -617,20 +638,20 @@ __global__ void reduce_slabs_kernel(const float *__restrict__ part, int nslab, i
     const int co = i / Kp, k = i - co * Kp;
     const int tap = k / Cin, ci = k - tap * Cin;
     if (!bias && (tap >= 27 || ci >= Cin_real)) return;  // the K tail, padded input channels
-    float a = 0.f;
+    double a = 0.0;
     int s = 0;
     for (; s + 8 <= nslab; s += 8) {
-        float v[8];
+        T v[8];
 #pragma unroll
         for (int j = 0; j < 8; ++j) v[j] = part[(size_t)(s + j) * count + i];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) a += v[j];
+        for (int j = 0; j < 8; ++j) a += (double)v[j];
     }
-    for (; s < nslab; ++s) a += part[(size_t)s * count + i];
+    for (; s < nslab; ++s) a += (double)part[(size_t)s * count + i];
     if (bias)
-        gb[i - Cout * Kp] = a;
+        gb[i - Cout * Kp] = (float)a;
     else
-        g[((size_t)co * Cin_real + ci) * 27 + tap] = a;
+        g[((size_t)co * Cin_real + ci) * 27 + tap] = (float)a;
 }
 
 // First pass of a two-pass slab reduction: part p of P sums slabs
@@ -638,21 +659,21 @@ __global__ void reduce_slabs_kernel(const float *__restrict__ part, int nslab, i
 // share the reads; reduce_slabs_kernel then adds the P parts in order (a fixed
 // tree: the same bits on every call).
 __global__ void reduce_slab_parts_kernel(const float *__restrict__ partial, int nslab, size_t count, int nparts,
-                                         float *__restrict__ tmp) {
+                                         double *__restrict__ tmp) {
     const size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
     const int part = blockIdx.y;
     if (i >= count) return;
     const int s0 = (int)((long long)nslab * part / nparts), s1 = (int)((long long)nslab * (part + 1) / nparts);
-    float a = 0.f;
+    double a = 0.0;
     int s = s0;
     for (; s + 8 <= s1; s += 8) {
         float v[8];
 #pragma unroll
         for (int j = 0; j < 8; ++j) v[j] = partial[(size_t)(s + j) * count + i];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) a += v[j];
+        for (int j = 0; j < 8; ++j) a += (double)v[j];
     }
-    for (; s < s1; ++s) a += partial[(size_t)s * count + i];
+    for (; s < s1; ++s) a += (double)partial[(size_t)s * count + i];
     tmp[(size_t)part * count + i] = a;
 }
 
@@ -915,6 +936,11 @@ constexpr int kHeadIn = 16;
 inline int pad32(int k) { return (k + 31) / 32 * 32; }
 
 constexpr int kReduceParts = 16;  // parts of the first pass of the slab reductions
+// Blocks of 64 points that a weight gradient's workgroup adds up in FP32; the workgroups' sums are added
+// in FP64.  Against the FP64 mean of single samples' gradients (rms, relative, the worst layer): 4 x 64^3
+// 6.5e-8, 32 x 64^3 5.5e-8, 128 x 64^3 5.1e-8; with 512 workgroups at any batch and FP32 throughout
+// 1.8e-7, 2.7e-7 and 8.6e-7.  Training steps 2.16 -> 2.15, 13.0 -> 12.2 ms at 4 and 32 x 64^3.
+constexpr int kSlabBlocks = 64;
 
 size_t param_count() {
     size_t c = 0;
@@ -926,7 +952,8 @@ size_t param_count() {
 // the groups of 16 input channels counted (a workgroup that goes on to the next rows stages a third of
 // them anew, and more workgroups write and re-read more partials), or up to 1024 where 512 would take
 // fewer than 8 blocks each.  Training steps, ms, for 512 / 1024 / 2048 workgroups: 4 x 64^3 2.15, 2.23, 2.28;
-// 8 x 36^3 1.47, 1.50, 1.55; 16 x 12^3 0.80, 0.73, 0.73.
+// 8 x 36^3 1.47, 1.50, 1.55; 16 x 12^3 0.80, 0.73, 0.73.  A workgroup adds up at most kSlabBlocks blocks in
+// FP32, for the sums' precision; larger layers take a multiple of 512 workgroups.
 WgradShape wgrad_shape(int n, int batch, int cin, int *nslab) {
     WgradShape S;
     S.n = n;
@@ -937,8 +964,10 @@ WgradShape wgrad_shape(int n, int batch, int cin, int *nslab) {
     S.nblk = batch * n * S.nyb * S.nseg;
     S.inv_pairs = 1.0f / (float)(S.w8 / 2 + 1);
     const int groups = (cin + 15) / 16;
-    const int most = std::max(1, (S.nblk * (long long)groups >= 8 * 512 ? 512 : 1024) / groups);
-    S.per_slab = (S.nblk + most - 1) / most;
+    const long long work = S.nblk * (long long)groups;
+    const long long turns = (work + 512 * kSlabBlocks - 1) / (512 * kSlabBlocks);
+    const int most = std::max(1, (int)((work >= 8 * 512 ? 512 * turns : 1024) / groups));
+    S.per_slab = std::min((S.nblk + most - 1) / most, kSlabBlocks);
     *nslab = (S.nblk + S.per_slab - 1) / S.per_slab;
     return S;
 }
@@ -958,7 +987,7 @@ struct cfm_unet {
     size_t woff[kNConv], boff[kNConv], head_off = 0;
     bf16 *Wf[kNConv] = {}, *Wt[kNConv] = {};
     int Kp[kNConv], Kpt[kNConv];
-    float *rtmp = nullptr;  // two-pass slab reduction: [kReduceParts][largest layer]
+    double *rtmp = nullptr;  // two-pass slab reduction: [kReduceParts][largest layer]
     float *partial = nullptr;
     // activations
     bf16 *X0 = nullptr, *A0 = nullptr, *S1 = nullptr, *Q1 = nullptr, *A2 = nullptr, *S2 = nullptr, *Q2 = nullptr,
@@ -1045,7 +1074,7 @@ extern "C" cfm_status cfm_unet_create(int n, int batch, cfm_unet **out) {
         wgrad_shape(n >> kConv[i].level, batch, kConv[i].cin, &nslab);
         max_partial = std::max(max_partial, (size_t)nslab * kConv[i].cout * (u->Kp[i] + 1));
     }
-    A(&u->rtmp, 4 * kReduceParts * max_wk);
+    A(&u->rtmp, 8 * kReduceParts * max_wk);
     A(&u->partial, 4 * max_partial);
     const size_t P1 = u->P[0], P2 = u->P[1], P3 = u->P[2];
     A(&u->X0, 2 * P1 * 8);
@@ -1307,7 +1336,7 @@ extern "C" cfm_status cfm_unet_forward(cfm_unet *u, const float *input, float *o
 template <int CIN, int COUT>
 static void launch_wgrad_rows(int nslab, hipStream_t st, const bf16 *X, const bf16 *Xup, const bf16 *dZ, int kp, float *partial,
                               const WgradShape &S) {
-    const size_t lds = sizeof(bf16) * ((size_t)COUT * 72 + (size_t)3 * (S.rows + 2) * kWgradRows16);
+    const size_t lds = sizeof(bf16) * ((size_t)COUT * 72 + (size_t)3 * (S.rows + 2) * kWgradRows16) + sizeof(double) * COUT;
     // (short rows, eight to a block, take more than 64 KiB)
     static const bool big_lds_ok = hipFuncSetAttribute((const void *)conv3_wgrad_rows_kernel<CIN, COUT>,
                                                        hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) == hipSuccess;
@@ -1344,16 +1373,16 @@ static cfm_status conv_wgrad(cfm_unet *u, int I, const bf16 *X, const bf16 *dZ, 
     if (!wgrad_rows(s.cin, s.cout, nslab, u->stream, X, Xup, dZ, Kp, u->partial, S))
         return CFM_FAIL(CFM_EINVAL, "unet: no weight-gradient kernel for %d -> %d channels", s.cin, s.cout);
     CFM_HIP(hipGetLastError());
-    const float *part = u->partial;
     if (nslab >= 4 * kReduceParts) {
         const dim3 grid((unsigned)((count + 255) / 256), kReduceParts);
         hipLaunchKernelGGL(reduce_slab_parts_kernel, grid, dim3(256), 0, u->stream, u->partial, nslab, (size_t)count,
                            kReduceParts, u->rtmp);
-        part = u->rtmp;
-        nslab = kReduceParts;
+        hipLaunchKernelGGL(reduce_slabs_kernel<double>, blocks_for(count), dim3(256), 0, u->stream, u->rtmp, kReduceParts,
+                           s.cout, s.cin_real, s.cin, Kp, u->grad + u->woff[I], u->grad + u->boff[I]);
+    } else {
+        hipLaunchKernelGGL(reduce_slabs_kernel<float>, blocks_for(count), dim3(256), 0, u->stream, u->partial, nslab,
+                           s.cout, s.cin_real, s.cin, Kp, u->grad + u->woff[I], u->grad + u->boff[I]);
     }
-    hipLaunchKernelGGL(reduce_slabs_kernel, blocks_for(count), dim3(256), 0, u->stream, part, nslab, s.cout,
-                       s.cin_real, s.cin, Kp, u->grad + u->woff[I], u->grad + u->boff[I]);
     CFM_HIP(hipGetLastError());
     return CFM_OK;
 }

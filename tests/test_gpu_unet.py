@@ -119,3 +119,29 @@ def test_gradient_of_ragged_rows(cfm, gpu, n, batch):
             e = _rel(g[off: off + cnt], rg[off: off + cnt])
             assert e < 3e-2, f"conv {li} {name}: rel err {e:.3g}"
             off += cnt
+
+
+def test_gradient_sums_of_a_large_batch(cfm, gpu):
+    """The weight gradients' FP32 sums do not get longer with the batch: a batch's gradient against the FP64 mean of
+    its samples' gradients.  Adding up m terms of either sign in FP32 leaves about half a rounding (2^-25) of the
+    running sum at each addition, sqrt(m/2) 2^-25 of the result in all; 128 additions in a row (64 blocks of two K
+    steps) are 2.4e-7, half as much again for the samples' own gradients and the spread between layers."""
+    n, batch = 64, 128
+    params = cfm.unet_init_params(12)
+    rng = np.random.default_rng(12)
+    inp = rng.standard_normal((batch, 2, n, n, n), dtype=np.float32)
+    target = rng.standard_normal((batch, n, n, n), dtype=np.float32)
+    ref = np.zeros(cfm.unet_param_count())
+    with cfm.UNet(n, 1, params=params) as net:
+        for i in range(batch):
+            ref += net.gradient(inp[i:i + 1], target[i:i + 1])[1]
+    ref /= batch
+    with cfm.UNet(n, batch, params=params) as net:
+        g = net.gradient(inp, target)[1]
+    off = 0
+    for li, (ci, co) in enumerate(uo.CONVS):
+        for name, cnt in (("W", co * ci * 27), ("b", co)):
+            d = g[off:off + cnt] - ref[off:off + cnt]
+            e = np.sqrt(np.mean(d * d) / np.mean(ref[off:off + cnt] ** 2))
+            assert e < 3.6e-7, f"conv {li} {name}: rms relative error {e:.3g}"
+            off += cnt
