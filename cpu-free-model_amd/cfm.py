@@ -41,7 +41,7 @@ EXPORTS = (
     "cfm_unet_get_params", "cfm_unet_forward", "cfm_unet_gradient", "cfm_unet_train_step",
     "cfm_cg_batch_x0_rejected", "cfm_cg_batch_load_features", "cfm_cg_batch_warm_start", "cfm_gen_varcoef3d_coef",
     "cfm_cg_batch_smooth_x0", "cfm_gen_tridiag", "cfm_mm_read", "cfm_host_free", "cfm_jacobi_plan_phase_times",
-    "cfm_cg_plan_phase_times", "cfm_jacobi_run_noalloc",
+    "cfm_cg_plan_phase_times", "cfm_jacobi_run_noalloc", "cfm_cg_batch_resident",
 )
 PHASES = ("spmv", "update", "reduce", "barrier", "other")
 
@@ -161,6 +161,8 @@ def _load():
     L.cfm_cg_batch_tune.argtypes = [_vp, ctypes.c_int, ctypes.c_char_p, _ip, _ip]
     L.cfm_cg_batch_matrix_format.argtypes = [_vp]
     L.cfm_cg_batch_matrix_format.restype = ctypes.c_int
+    L.cfm_cg_batch_resident.argtypes = [_vp]
+    L.cfm_cg_batch_resident.restype = ctypes.c_int
     L.cfm_cg_batch_plan_destroy.argtypes = [_vp]
     L.cfm_cg_batch_plan_destroy.restype = None
     _fp = ctypes.POINTER(ctypes.c_float)
@@ -708,6 +710,10 @@ class CgBatchPlan:
     def matrix_format(self):
         """Storage of the next solve: "sell" or "dia"."""
         return {1: "sell", 2: "dia"}[lib.cfm_cg_batch_matrix_format(self._h)]
+
+    def resident(self):
+        """Whether the next solve uses the resident kernel."""
+        return lib.cfm_cg_batch_resident(self._h) == 1
 
     def close(self):
         if self._h:

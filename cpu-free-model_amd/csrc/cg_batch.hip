@@ -932,8 +932,10 @@ extern "C" cfm_status cfm_cg_batch_solve(cfm_cg_batch_plan *pl, int *iters, int 
 // from the current x0) of the kTuneFinalists fastest and keep the fastest solve: the
 // first iterations, where every system is active, do not show the tail, where the
 // few systems still iterating leave most of the grid waiting at barriers.  With a
-// cache file the winner is stored under a key of device, system count, row count and
-// tolerance, and looked up first.
+// cache file the winner is stored under a key of device, system count, row count,
+// tolerance and what it was chosen among (the storages and the resident kernel's rounds),
+// and looked up first.  (Keys without the last part are of files from before there was a
+// resident kernel: their winners were not timed against it.)
 constexpr int kTuneFinalists = 3;
 constexpr int kTuneResident = 0;  // in place of a sub-block count: the resident kernel
 
@@ -941,8 +943,9 @@ extern "C" cfm_status cfm_cg_batch_tune(cfm_cg_batch_plan *pl, int trial_iters, 
                                         int *best_block, int *best_grid) {
     if (!pl || trial_iters < 1) return CFM_EINVAL;
     char key[512];
-    std::snprintf(key, sizeof(key), "cg_batch|%s|cus=%d|nsys=%d|rows=%lld|chunks=%d|tol=%.3g", pl->dev.name,
-                  pl->dev.cus, pl->nsys, pl->total_rows, pl->total_chunks, pl->p.tol);
+    std::snprintf(key, sizeof(key), "cg_batch|%s|cus=%d|nsys=%d|rows=%lld|chunks=%d|tol=%.3g|format=%d|diag=%d|rounds=%d",
+                  pl->dev.name, pl->dev.cus, pl->nsys, pl->total_rows, pl->total_chunks, pl->p.tol, pl->p.matrix_format,
+                  pl->dmax, pl->res_rounds);
     for (char *q = key; *q; ++q)  // the cache line is whitespace-separated
         if (*q == ' ' || *q == '\t') *q = '_';
     const bool have_sell = pl->p.matrix_format != 2, have_dia = pl->dmax > 0;
@@ -1036,6 +1039,11 @@ extern "C" cfm_status cfm_cg_batch_tune(cfm_cg_batch_plan *pl, int trial_iters, 
 extern "C" int cfm_cg_batch_matrix_format(const cfm_cg_batch_plan *pl) {
     if (!pl) return -1;
     return pl->dia_on ? 2 : 1;
+}
+
+extern "C" int cfm_cg_batch_resident(const cfm_cg_batch_plan *pl) {
+    if (!pl) return -1;
+    return pl->resident ? 1 : 0;
 }
 
 extern "C" cfm_status cfm_cg_batch_x0_rejected(cfm_cg_batch_plan *pl, int *flags) {

@@ -284,15 +284,20 @@ cfm_status cfm_cg_batch_get_x(cfm_cg_batch_plan *plan, double *x);
 /* Autotuner: times trial_iters fixed iterations for each workgroup shape
  * (256/512/1024 threads), grid size (1..occupancy workgroups per CU) and
  * storage the plan holds (SELL-64; DIA too for an auto plan whose systems are
- * all banded), then times full solves (the plan's tol and max_iter, from the
+ * all banded), and the resident kernel where the plan has it, then times full solves (the plan's tol and max_iter, from the
  * current x0) of the three fastest and keeps the fastest solve; cache_path
  * (may be NULL) stores/looks up the winner per (device, system count, row
- * count, tolerance).  The reference has no tuner: its launch shapes are
+ * count, tolerance, storages, resident kernel's rounds).  A resident winner is
+ * reported with its own launch (256 threads, its grid); asking for that shape
+ * in a plan's parameters gives the general kernel.  The reference has no tuner: its launch shapes are
  * fixed per binary (CG/src/single-stream/pipelined.cu). */
 cfm_status cfm_cg_batch_tune(cfm_cg_batch_plan *plan, int trial_iters, const char *cache_path,
                              int *best_block, int *best_grid);
 /* Storage the next solve uses: 1 = SELL-64, 2 = DIA (-1 for a NULL plan). */
 int cfm_cg_batch_matrix_format(const cfm_cg_batch_plan *plan);
+/* Kernel the next solve uses: 1 = resident (each system in the registers of its
+ * own workgroups while it is solved), 0 = general (-1 for a NULL plan). */
+int cfm_cg_batch_resident(const cfm_cg_batch_plan *plan);
 void cfm_cg_batch_plan_destroy(cfm_cg_batch_plan *plan);
 /* After a solve with x0_guard set: flags[s] = 1 where system s was restarted
  * from x0 = 0 because its initial guess was worse than zero. */

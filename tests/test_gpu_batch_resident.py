@@ -88,3 +88,31 @@ def test_batch_resident_waits_for_longer_systems(gpu):
     for s in (0, 4):
         alone = gpu.cg(*systems[s], b[srp[s]:srp[s + 1]], method=gpu.CG_PIPELINED, tol=1e-8, max_iter=max_iter)
         assert alone[0] == gpu.ENOTCONV and np.array_equal(x[srp[s]:srp[s + 1]], alone[1])
+
+
+def test_batch_tune_cache_names_the_candidates(gpu, tmp_path):
+    """A winner is only looked up by plans that choose among the same candidates: not one from a plan that has no
+    resident kernel, nor one of a file from before there was one."""
+    systems = [gpu.poisson3d(8, 9, 10), gpu.poisson3d(20, 9, 14)]
+    srp, rp, col, val = gpu.block_diag(systems)
+    b = gpu.uniform(5, 0, int(srp[-1]))
+    cache = tmp_path / "tune.txt"
+
+    def tune(**kw):
+        p = gpu.cg_params(method=gpu.CG_PIPELINED, tol=1e-8, max_iter=500, **kw)
+        with gpu.CgBatchPlan(srp, rp, col, val, p) as plan:
+            plan.set_rhs(b)
+            plan.set_x0(None)
+            first = plan.resident()
+            won = plan.tune(trial_iters=5, cache_path=str(cache))
+            return first, won, plan.resident(), len(cache.read_text().splitlines())
+
+    first, won, resident, lines = tune(block_threads=1024)
+    assert not first and not resident and lines == 1
+    first, won, resident, lines = tune()
+    assert first and lines == 2
+    assert tune() == (True, won, resident, 2)  # its own line is found again
+    # a line as it was written before there was a resident kernel
+    old = cache.read_text().splitlines()[1].split()[0].split("|format=")[0]
+    cache.write_text(f"{old} 4 256 0\n")
+    assert tune()[3] == 2
