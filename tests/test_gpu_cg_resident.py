@@ -73,3 +73,30 @@ def _banded(n, half, seed):
 def test_resident_row_widths(gpu, orc, half, method):
     """1, 5, 7 and 9 entries a row (the last too wide for the registers)."""
     _check(gpu, orc, *_banded(2500, half, half), method, 9)
+
+
+def _nine_diagonals(n):
+    """Nine full diagonals but for the pair of entries (10, 11) and (11, 10), which a diagonal's storage holds as zeros."""
+    offs = np.array([-900, -3, -2, -1, 0, 1, 2, 3, 900])
+    col = (np.arange(n)[:, None] + offs).astype(np.int32)
+    ok = (col >= 0) & (col < n)
+    ok[10, 5] = ok[11, 3] = False
+    rp = np.zeros(n + 1, dtype=np.int32)
+    rp[1:] = np.cumsum(ok.sum(1))
+    return rp, col[ok], np.broadcast_to(np.where(offs == 0, 10.0, -1.0), col.shape)[ok]
+
+
+@pytest.mark.parametrize("method", ["standard", "pipelined"])
+def test_nine_diagonals_below_2_20_rows_keep_sell(gpu, orc, method):
+    """Stored by rows, an infinite guess reaches only the rows that hold its column: <r, r> is infinite, not NaN (an
+    infinity times a diagonal's stored zero)."""
+    rp, col, val = _nine_diagonals(700000)
+    b = gpu.uniform(3, 0, 700000) - 0.5
+    x0 = np.zeros(700000)
+    x0[11] = np.inf
+    A = orc.Csr(rp, col, val)
+    ost, ox, ohist, oit = orc.cg(A, b, x0=x0, tol=1e-8, max_iter=3, variant=method)
+    st, x, hist, it, t = gpu.cg(rp, col, val, b, x0=x0, method=METHODS[method], tol=1e-8, max_iter=3)
+    assert np.isinf(ohist[0]) and np.isinf(hist[0])
+    assert (st, it) == (ost, oit) and np.array_equal(x, ox)
+    _check(gpu, orc, rp, col, val, method, 3)
