@@ -498,10 +498,15 @@ struct Stream {
     }
     // sell_row's chain for one row (its slice, this lane); live: the row's chunk is the system's (both
     // uniform over the wavefront).  kOff moves an offset out of every buffer.
+    // GUESS: x is the caller's and may hold infinities.  What is read for entries that the row does not
+    // have (a diagonal's zeros, x[0] beyond a SELL-64 slice's width) is then left out, so that they reach
+    // only the rows that have their columns.
+    template <bool GUESS = false>
     __device__ __forceinline__ T row(const T *x, int row, int slice, int lane, bool live) const {
         constexpr int kOff = (int)0x80000000u;
         const auto rx = __builtin_amdgcn_make_buffer_rsrc((void *)x, (short)0, n * (int)sizeof(T), 0x00020000);
         T v[kStreamWidth], g[kStreamWidth], acc = T(0);
+        bool there[kStreamWidth];
         // (opaque: hoisted out of the solve's loop, every entry's offset of every row would hold a register)
         asm volatile("" : "+v"(row), "+v"(lane));
         if constexpr (DIA) {
@@ -511,6 +516,7 @@ struct Stream {
                 const int e = min(d, S.ndiag - 1);
                 v[d] = buffer_at<T>(val, row * (int)sizeof(T) | out, e * S.npad * (int)sizeof(T));
                 g[d] = buffer_at<T>(rx, (row + S.doff[e]) * (int)sizeof(T) | out, 0);
+                there[d] = v[d] != T(0);
             }
         } else {
             const int beg = S.slice_ptr[live ? slice : 0];
@@ -523,10 +529,13 @@ struct Stream {
                 v[j] = buffer_at<T>(val, lane * (int)sizeof(T) | out, (beg + 64 * j) * (int)sizeof(T));
             }
 #pragma unroll
-            for (int j = 0; j < kStreamWidth; ++j) g[j] = buffer_at<T>(rx, c[j] * (int)sizeof(T), 0);
+            for (int j = 0; j < kStreamWidth; ++j) {
+                g[j] = buffer_at<T>(rx, c[j] * (int)sizeof(T), 0);
+                there[j] = j < width;
+            }
         }
 #pragma unroll
-        for (int j = 0; j < kStreamWidth; ++j) acc = fma(v[j], g[j], acc);
+        for (int j = 0; j < kStreamWidth; ++j) acc = GUESS && !there[j] ? acc : fma(v[j], g[j], acc);
         asm volatile("" : "+v"(acc));  // (the next row's loads come after it)
         return acc;
     }
@@ -651,7 +660,7 @@ __global__ void __launch_bounds__(256 * kSub) cg_standard_streamed(CgArgs A) {
 #pragma unroll
     for (int e = 0; e < 2 * NCH; ++e) two[e] = 0.0;
     CFM_FOR_RESIDENT_ROWS({
-        const double ax = M.row(A.x0, row, slice, P.t & 63, live);
+        const double ax = M.template row<true>(A.x0, row, slice, P.t & 63, live);
         const double bi = own(A, A.b, row);
         x.set(q, i, own(A, A.x0, row));
         p[q][i] = r[q][i] = fma(-1.0, ax, bi);
@@ -749,7 +758,7 @@ __global__ void __launch_bounds__(256 * kSub) cg_pipelined_streamed(CgArgs A) {
 #pragma unroll
     for (int q = 0; q < NCH; ++q) one[q] = 0.0;
     CFM_FOR_RESIDENT_ROWS({
-        const double ax = M.row(A.x0, row, slice, P.t & 63, live);
+        const double ax = M.template row<true>(A.x0, row, slice, P.t & 63, live);
         const double bi = own(A, A.b, row);
         if (X_MEM)
             put(A, A.x, row, own(A, A.x0, row));
@@ -868,7 +877,7 @@ __global__ void __launch_bounds__(256 * kSub) cg_ir_streamed(CgArgs A) {
 #pragma unroll
         for (int e = 0; e < 3 * NCH; ++e) three[e] = 0.0;
         CFM_FOR_RESIDENT_ROWS({
-            const double ax = M.row(first ? A.x0 : A.x, row, slice, P.t & 63, live);
+            const double ax = M.template row<true>(first ? A.x0 : A.x, row, slice, P.t & 63, live);
             const double bi = own(A, A.b, row);
             const double ri = fma(-1.0, ax, bi);
             if (first) put(A, A.x, row, own(A, A.x0, row));

@@ -100,3 +100,44 @@ def test_nine_diagonals_below_2_20_rows_keep_sell(gpu, orc, method):
     assert np.isinf(ohist[0]) and np.isinf(hist[0])
     assert (st, it) == (ost, oit) and np.array_equal(x, ox)
     _check(gpu, orc, rp, col, val, method, 3)
+
+
+def _pairs(n, seed):
+    """Rows of up to 4 entries at random columns (no diagonals to store them by)."""
+    rng = np.random.default_rng(seed)
+    rows = [np.arange(n)]
+    cols = [np.arange(n)]
+    for _ in range(3):
+        p = rng.permutation(n)[: n // 2 * 2].reshape(-1, 2)
+        rows += [p[:, 0], p[:, 1]]
+        cols += [p[:, 1], p[:, 0]]
+    r, c = np.concatenate(rows), np.concatenate(cols)
+    key = np.unique(r * np.int64(n) + c)
+    r, c = key // n, key % n
+    rp = np.zeros(n + 1, dtype=np.int32)
+    rp[1:] = np.cumsum(np.bincount(r, minlength=n))
+    return rp, c.astype(np.int32), np.where(r == c, 4.0, -1.0)
+
+
+@pytest.mark.parametrize("method", list(METHODS))
+@pytest.mark.parametrize("matrix", ["poisson", "pairs"])
+def test_streamed_infinite_guess(gpu, orc, matrix, method):
+    """An infinity in the guess reaches the rows that hold its column and no others, as in the oracle: <r, r> is
+    infinite, not NaN."""
+    rp, col, val = gpu.poisson3d(96, 96, 60) if matrix == "poisson" else _pairs(540000, 5)
+    n = rp.size - 1
+    assert n > 2 ** 19
+    b = gpu.uniform(3, 0, n) - 0.5
+    for at in (0, 95):
+        x0 = np.zeros(n)
+        x0[at] = np.inf
+        A = orc.Csr(rp, col, val)
+        if method == "ir":
+            ost, ox, ohist, _, oit = orc.cg_ir(A, b, x0=x0, tol=1e-9, inner_max=5, max_outer=2, inner_tol=1e-3)
+            kw = dict(tol=1e-9, max_iter=5, max_outer=2, inner_tol=1e-3)
+        else:
+            ost, ox, ohist, oit = orc.cg(A, b, x0=x0, tol=1e-8, max_iter=3, variant=method)
+            kw = dict(tol=1e-8, max_iter=3)
+        st, x, hist, it, _ = gpu.cg(rp, col, val, b, x0=x0, method=METHODS[method], **kw)
+        assert np.isinf(ohist[0]) and np.isinf(hist[0])
+        assert (st, it) == (ost, oit) and np.array_equal(x, ox, equal_nan=True)
