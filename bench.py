@@ -216,7 +216,7 @@ def jacobi_f32_figures(cfm, shape, niter):
             _, t = plan.run()
             fields[name] = plan.download()
         res[name] = {"glups": round(interior * niter / t.kernel_ms / 1e6, 1), "ms": round(t.kernel_ms, 2),
-                     "passes": t.outer_iterations}
+                     "passes": cfm.jacobi_route(p)["passes"]}
     d = fields["f32"].astype(np.float64) - fields["f64"]
     res["f32"]["max_abs_err_vs_f64"] = float(f"{np.abs(d).max():.3e}")
     res["f32"]["rel_l2_err_vs_f64"] = float(f"{np.linalg.norm(d) / np.linalg.norm(fields['f64']):.3e}")
@@ -389,10 +389,9 @@ def main():
 
     interior = (n - 2) ** 3
     lups = interior * niter * args.steps
-    # passes over the field in HBM per launch: with nothing about the kernel asked for, the register
-    # pipeline's four sweeps each; else as the plan counts them (two sweeps each when time-blocked)
-    pipe = not any(v > 0 for v in (args.tile_rows, args.grid, args.chunks, args.time_block, args.block))
-    passes = -(-niter // 4) if pipe else t.outer_iterations
+    # passes over the field in HBM per launch: the register pipeline's four sweeps each, unless a kernel is asked for
+    route = cfm.jacobi_route(p)
+    pipe, passes = route["kernel"] == "register pipeline", route["passes"]
     value = lups / wall / 1e9
     mean_kernel_s = sum(kernel_ms) / len(kernel_ms) / 1e3
     achieved = BYTES_PER_LUP_F64 * interior * passes / mean_kernel_s / 1e9

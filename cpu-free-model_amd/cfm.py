@@ -42,6 +42,7 @@ EXPORTS = (
     "cfm_cg_batch_x0_rejected", "cfm_cg_batch_load_features", "cfm_cg_batch_warm_start", "cfm_gen_varcoef3d_coef",
     "cfm_cg_batch_smooth_x0", "cfm_gen_tridiag", "cfm_mm_read", "cfm_host_free", "cfm_jacobi_plan_phase_times",
     "cfm_cg_plan_phase_times", "cfm_jacobi_run_noalloc", "cfm_cg_batch_resident",
+    "cfm_jacobi_describe",
 )
 PHASES = ("spmv", "update", "reduce", "barrier", "other")
 
@@ -75,6 +76,10 @@ class CgParams(ctypes.Structure):
                 ("inner_tol", ctypes.c_double), ("grid_blocks", ctypes.c_int),
                 ("spin_limit_us", ctypes.c_int), ("block_threads", ctypes.c_int), ("x0_guard", ctypes.c_int),
                 ("matrix_format", ctypes.c_int), ("phase_timers", ctypes.c_int)]
+
+
+class JacobiRoute(ctypes.Structure):
+    _fields_ = [(n, ctypes.c_int) for n in ("kernel", "passes", "sweeps_per_pass")]
 
 
 class PhaseTimes(ctypes.Structure):
@@ -134,6 +139,7 @@ def _load():
     L.cfm_jacobi_run.argtypes = [ctypes.POINTER(JacobiParams), _vp, _vp, _dp, ctypes.c_int, _ip,
                                  ctypes.POINTER(Timing)]
     L.cfm_jacobi_init_field.argtypes = [ctypes.c_int] * 5 + [_vp]
+    L.cfm_jacobi_describe.argtypes = [ctypes.POINTER(JacobiParams), ctypes.POINTER(JacobiRoute)]
     L.cfm_jacobi_run_noalloc.argtypes = [ctypes.POINTER(JacobiParams), _vp, _vp, _vp, _dp, ctypes.c_int, _ip,
                                          ctypes.POINTER(Timing)]
     L.cfm_cg_plan_create.argtypes = [ctypes.c_int, ctypes.c_int, _vp, _vp, _vp, ctypes.c_int, ctypes.c_int,
@@ -338,6 +344,14 @@ def jacobi_params(nx, ny, nz=1, niter=1000, norm_every=0, prec=F64, bc=BC_DIRICH
                   time_block=0, phase_timers=0):
     return JacobiParams(nx, ny, nz, niter, norm_every, prec, bc, variant, tile_rows, grid_blocks, chunks,
                         spin_limit_us, block_threads, time_block, phase_timers)
+
+
+def jacobi_route(params):
+    """What a run of these parameters does: its kernel, its trips through memory and the sweeps of one at most."""
+    r = JacobiRoute()
+    _check(lib.cfm_jacobi_describe(ctypes.byref(params), ctypes.byref(r)), "cfm_jacobi_describe")
+    return {"kernel": ("streaming", "register tiles", "register pipeline")[r.kernel], "passes": r.passes,
+            "sweeps_per_pass": r.sweeps_per_pass}
 
 
 class JacobiPlan:

@@ -157,11 +157,13 @@ inline int run_jacobi(int argc, char **argv, int dims) {
                     ph.workgroups, ph.ms[CFM_PHASE_SPMV], ph.max_ms[CFM_PHASE_SPMV], ph.ms[CFM_PHASE_BARRIER],
                     ph.max_ms[CFM_PHASE_BARRIER], ph.total_ms);
     if (json) {
+        cfm_jacobi_route route{};
+        (void)cfm_jacobi_describe(&p, &route);
         const double lups = (double)(p.nx - 2) * (p.ny - 2) * (dims == 2 ? 1 : p.nz - 2) * p.niter;
         std::printf("{\"version\": \"%s\", \"kernel_ms\": %.4f, \"glups\": %.3f, \"gbs\": %.1f, \"grid\": %d, "
                     "\"block\": %d, \"passes\": %d, \"cooperative\": %d",
                     names[selection], t.kernel_ms, lups / (t.kernel_ms * 1e6),
-                    lups * 2 * esz / (t.kernel_ms * 1e6), t.grid_blocks, t.block_threads, t.outer_iterations,
+                    lups * 2 * esz / (t.kernel_ms * 1e6), t.grid_blocks, t.block_threads, route.passes,
                     t.cooperative);
         if (ph.workgroups > 0)
             std::printf(", \"phases\": {\"workgroups\": %d, \"sweeps_ms\": %.4f, \"sweeps_max_ms\": %.4f, "

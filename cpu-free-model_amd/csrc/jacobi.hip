@@ -2659,15 +2659,24 @@ int cfm::jacobi_passes(const cfm_jacobi_params &p, const JacobiConfig &c) {
 
 int cfm::jacobi_swaps(const cfm_jacobi_params &p, const JacobiConfig &c) {
     if (!c.tile) return jacobi_passes(p, c);
-    if (c.pipe) {
-        int turns = 0;
-        for (int k = 0; k < p.niter; ++turns)
-            k += jacobi_pipe_steps(k, p.niter, c.depth, p.norm_every, p.bc == CFM_BC_PERIODIC);
-        return turns;
-    }
-    // periodic rows: the first sweep is a pass of its own
+    const auto up = [&](int sweeps) { return (int)((sweeps + c.depth - 1LL) / c.depth); };
+    // periodic rows or planes: the first sweep is a pass of its own
     const int first = p.bc == CFM_BC_PERIODIC ? std::min(p.niter, 1) : 0;
-    return first + (p.niter - first + c.depth - 1) / c.depth;
+    if (!c.pipe || p.norm_every <= 0) return first + up(p.niter - first);
+    // the pipeline's passes start anew at each sweep whose norm is wanted (jacobi_pipe_steps)
+    const int head = std::min(p.niter, p.norm_every), rest = p.niter - head;
+    return first + up(head - first) + rest / p.norm_every * up(p.norm_every) + up(rest % p.norm_every);
+}
+
+extern "C" cfm_status cfm_jacobi_describe(const cfm_jacobi_params *p, cfm_jacobi_route *out) {
+    if (!out) return CFM_EINVAL;
+    JacobiConfig c;
+    const cfm_status st = jacobi_configure(p, &c);
+    if (st != CFM_OK) return st;
+    out->kernel = !c.tile ? CFM_JACOBI_STREAMING : c.pipe ? CFM_JACOBI_REGISTER_PIPELINE : CFM_JACOBI_REGISTER_TILES;
+    out->passes = p->variant == CFM_JACOBI_NO_COMPUTE ? 0 : jacobi_swaps(*p, c);
+    out->sweeps_per_pass = c.tile ? c.depth : c.sweeps_per_pass;
+    return CFM_OK;
 }
 
 void cfm::jacobi_fill_timing(cfm_timing *t, const cfm_jacobi_params &p, const JacobiConfig &c, float ms,

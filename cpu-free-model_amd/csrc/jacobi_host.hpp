@@ -50,7 +50,7 @@ struct JacobiConfig {
 
 // Validates p and fills c for the current device.
 cfm_status jacobi_configure(const cfm_jacobi_params *p, JacobiConfig *c);
-// Sweeps of the pipeline kernels' pass that starts with sweep k: a sweep whose update norm is wanted
+// Sweeps of the pipeline kernels' pass that starts with sweep k (jacobi_swaps counts the passes): a sweep whose update norm is wanted
 // is the first of its pass, and with periodic planes the run's first sweep is a pass of its own.
 __host__ __device__ inline int jacobi_pipe_steps(int k, int niter, int depth, int norm_every, bool periodic) {
     int steps = niter - k < depth ? niter - k : depth;

@@ -99,7 +99,7 @@ typedef struct {
     int outer_iterations; /* Jacobi: passes over the field in HBM as time_block counts them (auto in 2D:
                              Dirichlet 4 sweeps each, periodic y 2; in 3D 2, or 1; the register tiles and
                              the register pipeline may make several such passes between two trips
-                             through memory); IR: refinements */
+                             through memory, which cfm_jacobi_describe counts); IR: refinements */
     int cooperative;    /* persistent kernel launch: 1 = cooperative (co-residency guaranteed),
                            0 = ordinary launch because another process held ROCm's one-process
                            cooperative grant (co-residency expected, not guaranteed; the barrier
@@ -157,6 +157,15 @@ cfm_status cfm_bandwidth_probe_shape(size_t bytes, int reps, int kind, int grid,
                                      double *gbs, double *best_ms);
 
 /* ------------------------------------------------------------- Jacobi --- */
+/* What a run of these parameters does: its kernel and its trips through memory (each reads one of
+ * the two arrays and writes the other). */
+enum { CFM_JACOBI_STREAMING = 0, CFM_JACOBI_REGISTER_TILES = 1, CFM_JACOBI_REGISTER_PIPELINE = 2 };
+typedef struct {
+    int kernel;          /* one of the above */
+    int passes;          /* trips through memory of one run */
+    int sweeps_per_pass; /* sweeps of one trip at most */
+} cfm_jacobi_route;
+cfm_status cfm_jacobi_describe(const cfm_jacobi_params *p, cfm_jacobi_route *out);
 /* Replaces the allocate/initialise/launch/swap part of
  * SSMultiThreadedTwoBlockComm::init (Stencil/jacobi2D/src/single-stream/
  * multi-threaded-two-block-comm.cu:126-308, Stencil/jacobi3D/src/single-stream/

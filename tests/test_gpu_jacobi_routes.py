@@ -1,0 +1,57 @@
+"""Which kernel a Jacobi run takes, and what it says of its passes (cfm_jacobi_describe)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _route(gpu, shape, niter, norm_every=0, dtype=np.float64, bc=1, **kw):
+    nz, ny, nx = (1,) + shape if len(shape) == 2 else shape
+    prec = gpu.F64 if dtype == np.float64 else gpu.F32
+    return gpu.jacobi_route(gpu.jacobi_params(nx, ny, nz, niter, norm_every, prec, bc, **kw))
+
+
+def _pipeline_passes(niter, norm_every, bc):
+    """Passes of four sweeps; one starts at each sweep whose norm is wanted, and with periodic planes the first
+    sweep is one of its own."""
+    k = passes = 0
+    while k < niter:
+        steps = min(4, niter - k)
+        if norm_every:
+            steps = min(steps, norm_every - k % norm_every)
+        k += 1 if bc == 0 and k == 0 else steps
+        passes += 1
+    return passes
+
+
+@pytest.mark.parametrize("bc", [0, 1])
+def test_pipeline_passes(gpu, bc):
+    for niter in (0, 1, 2, 3, 4, 5, 9, 40, 41, 1000):
+        for norm_every in (0, 3, 4, 5, 6, 7, 10, 50, 2000):
+            r = _route(gpu, (64, 64, 64), niter, norm_every, bc=bc)
+            if r["kernel"] == "register pipeline":  # (norms that are too frequent go another way)
+                assert r["passes"] == _pipeline_passes(niter, norm_every, bc) and r["sweeps_per_pass"] == 4
+            else:
+                assert niter <= 2 or norm_every == 3
+
+
+def test_passes_that_are_made(gpu):
+    """The benchmark's fields: a quarter of the sweeps in 3D, deeper passes in 2D."""
+    assert _route(gpu, (512, 512, 512), 1000) == {"kernel": "register pipeline", "passes": 250, "sweeps_per_pass": 4}
+    r = _route(gpu, (16384, 16384), 1000)
+    assert r["kernel"] == "register tiles" and 4 < r["sweeps_per_pass"] <= 24
+    assert r["passes"] == -(-1000 // r["sweeps_per_pass"])
+    r = _route(gpu, (16384, 16384), 1000, bc=0)
+    assert r["passes"] == 1 + -(-999 // r["sweeps_per_pass"])
+    # one workgroup holds the field for the whole run
+    assert _route(gpu, (60, 100), 777) == {"kernel": "register tiles", "passes": 1, "sweeps_per_pass": 777}
+
+
+def test_passes_of_an_asked_kernel(gpu):
+    assert _route(gpu, (512, 512, 512), 7, time_block=2) == {"kernel": "streaming", "passes": 4, "sweeps_per_pass": 2}
+    assert _route(gpu, (512, 512, 512), 7, time_block=1)["passes"] == 7
+    assert _route(gpu, (1024, 1024), 7, time_block=4)["passes"] == 2
+    assert _route(gpu, (40, 40, 40), 7, variant=gpu.LAUNCH_PER_ITER)["passes"] == 7
+    assert _route(gpu, (40, 40, 40), 7, variant=gpu.NO_COMPUTE)["passes"] == 0
+    with pytest.raises(gpu.CfmError):
+        _route(gpu, (40, 40, 2), 7)
