@@ -482,18 +482,19 @@ __global__ void __launch_bounds__(64 * WAVES, R >= 4 && WAVES <= 8 ? 2 : 4) jaco
 }
 
 // A shape and what it measured: microseconds of a step with one workgroup on a CU and with as many as
-// fit, and the rate at which it moves fields (each pass reads one array and writes the other) that
-// the 256 MB of memory-side cache do not hold.
+// fit, the rate at which it moves fields (each pass reads one array and writes the other) that
+// the 256 MB of memory-side cache do not hold, and how much longer the steps of a pass with a norm, and of
+// one of fewer than L sweeps, take than a plain pass's (both are masked throughout).
 struct Shape3D {
     int vx, r, waves, per_cu;
     bool through;
-    double step_us, full_us, tb_s;
+    double step_us, full_us, tb_s, norm, part;
     KernelFn fn[2];  // [timed]
 };
 
 template <typename T, int VX, int R, int WAVES, bool THROUGH>
-Shape3D shape3d(int per_cu, double step_us, double full_us, double tb_s) {
-    return {VX, R, WAVES, per_cu, THROUGH, step_us, full_us, tb_s,
+Shape3D shape3d(int per_cu, double step_us, double full_us, double tb_s, double norm, double part) {
+    return {VX, R, WAVES, per_cu, THROUGH, step_us, full_us, tb_s, norm, part,
             {(KernelFn)jacobi3d_pipe_kernel<T, VX, R, WAVES, THROUGH, false>,
              (KernelFn)jacobi3d_pipe_kernel<T, VX, R, WAVES, THROUGH, true>}};
 }
@@ -503,13 +504,49 @@ int tiles_along(int n, int span) { return n <= span ? 1 : (n - span + span - 2 *
 
 // Estimated microseconds of one pass: the chunk's planes and 2 L more to fill and empty the pipeline,
 // for each round of boxes; the device-wide barrier, the first loads and the last stores, 5 us.
-double pass_us(const cfm_jacobi_params &p, const Shape3D &s, int tiles, int chunks, int cus) {
+double pass_us(const cfm_jacobi_params &p, const Shape3D &s, int tiles, int chunks, int cus, double longer = 1.0) {
     const int len = (p.nz - 2 + chunks - 1) / chunks;
     const double units = (double)tiles * chunks;
     const double rounds = std::ceil(units / (cus * s.per_cu));
     const double moved = 2.0 * (p.prec == CFM_F64 ? 8 : 4) * p.nx * (double)p.ny * p.nz;
-    return 5.0 + std::max(rounds * (len + 2 * L) * (units > cus ? s.full_us : s.step_us),
+    return 5.0 + std::max(rounds * (len + 2 * L) * (units > cus ? s.full_us : s.step_us) * longer,
                           moved > 2.0e8 ? moved / (s.tb_s * 1e6) : 0.0);
+}
+
+// Estimated microseconds of `sweeps` sweeps from the start of a run.
+double run_us(const cfm_jacobi_params &p, const Shape3D &s, int tiles, int chunks, int cus, int sweeps) {
+    const double plain = pass_us(p, s, tiles, chunks, cus), norm = pass_us(p, s, tiles, chunks, cus, s.norm),
+                 part = pass_us(p, s, tiles, chunks, cus, s.part);
+    double us = 0.0;
+    for (int k = 0; k < sweeps;) {
+        const int steps = jacobi_pipe_steps(k, sweeps, L, p.norm_every, p.bc == CFM_BC_PERIODIC);
+        us += p.norm_every > 0 && k % p.norm_every == 0 ? norm : steps < L ? part : plain;
+        k += steps;
+    }
+    return us;
+}
+
+// The same of the streaming kernels (jacobi.hip), as configured in c: a step a plane and two more to warm
+// up, for each round of units; norms cost them nothing.  Microseconds of a step as measured, FP64 and FP32:
+// two sweeps a pass 1.75 and 2.1 (rows of whole vectors), 2.1 and 2.4 (x tiles), 2.55 and 5.9 (other rows),
+// 1.25, 1.6, 2.0 and 1.45, 1.7, 4.8 where a run's last pass has one; the one-sweep kernels 2.45 and 3.75
+// (FP32 rows that are not whole vectors: 7.3 a tile of 1024 columns).
+// At 512^3, 300^3, 128^3 and 317 x 251 x 190 FP64 this gives 473, 179, 40 and 130 us for two sweeps, measured 468,
+// 173, 41 and 125.
+double streaming_us(const cfm_jacobi_params &p, const JacobiConfig &c, int sweeps) {
+    const bool f64 = p.prec == CFM_F64, periodic = p.bc == CFM_BC_PERIODIC;
+    const bool aligned = (size_t)p.nx * c.elem_size % 16 == 0, tiles_x = c.ntx > 1;
+    const double units = (double)c.ntx * c.nty * c.chunks, rounds = std::ceil(units / c.grid);
+    const double steps = rounds * (c.chunk_len + 2), moved = 2.0 * c.elem_size * p.nx * (double)p.ny * p.nz;
+    if (!c.t2) {
+        const double step = f64 ? 2.45 : aligned ? 3.75 : 7.3 * std::min(1.0, p.nx / 1024.0);
+        return sweeps * (3.0 + std::max(steps * step, moved / 4.6e6));
+    }
+    const double slow = periodic ? 1.06 : 1.0;  // (the copies of the opposite planes)
+    const double two = slow * (!aligned ? (f64 ? 2.55 : 5.9) : tiles_x ? (f64 ? 2.1 : 2.4) : (f64 ? 1.75 : 2.1));
+    const double one = slow * (!aligned ? (f64 ? 2.0 : 4.8) : tiles_x ? (f64 ? 1.6 : 1.7) : (f64 ? 1.25 : 1.45));
+    return sweeps / 2 * ((periodic ? 12.0 : 5.0) + std::max(steps * two, moved / 4.6e6)) +
+           sweeps % 2 * ((sweeps > 1 ? 5.0 : 0.0) + std::hypot(steps * one, moved / 5.5e6));
 }
 
 }  // namespace
@@ -517,7 +554,7 @@ double pass_us(const cfm_jacobi_params &p, const Shape3D &s, int tiles, int chun
 bool jacobi_pipe_configure(const cfm_jacobi_params &p, JacobiConfig *c) {
     const bool f64 = p.prec == CFM_F64;
     // 32-bit offsets within a plane and a tile's rows beyond it, and a wavefront's rows beyond kNowhere
-    const double pitch = (double)p.nx * (f64 ? 8 : 4), points = pitch / (f64 ? 8 : 4) * p.ny * p.nz;
+    const double pitch = (double)p.nx * (f64 ? 8 : 4);
     if (p.nz < 3 || pitch * p.ny >= 2.0e9 || pitch >= 1.6e7) return false;
     // Few rows a wavefront for small fields (a step is then shorter, and more boxes share the field),
     // many for large ones (less halo).  FP64: 16-byte lanes move a large field faster than 8-byte
@@ -525,14 +562,14 @@ bool jacobi_pipe_configure(const cfm_jacobi_params &p, JacobiConfig *c) {
     // rows at a pitch of 4096 bytes fall on few of the caches' channels), but waste half their
     // columns on rows of up to 64 points.  Going past the L2 costs nothing where a field's boxes are read once a
     // pass, and the barrier is then 3.6 us shorter.
-    static const Shape3D s64[] = {shape3d<double, 1, 2, 8, true>(2, 0.83, 1.22, 3.1),
-                                  shape3d<double, 1, 4, 8, true>(1, 1.22, 1.22, 3.8),
-                                  shape3d<double, 1, 8, 8, false>(1, 2.2, 2.2, 3.1),
-                                  shape3d<double, 2, 4, 8, false>(1, 2.2, 2.2, 4.1)};
-    static const Shape3D s32[] = {shape3d<float, 1, 2, 8, true>(3, 0.6, 1.05, 3.1),
-                                  shape3d<float, 2, 2, 8, true>(2, 0.8, 1.23, 3.1),
-                                  shape3d<float, 2, 4, 8, true>(1, 1.2, 1.2, 3.3),
-                                  shape3d<float, 2, 8, 8, false>(1, 2.4, 2.4, 3.4)};
+    static const Shape3D s64[] = {shape3d<double, 1, 2, 8, true>(2, 0.83, 1.22, 3.1, 1.3, 1.0),
+                                  shape3d<double, 1, 4, 8, true>(1, 1.22, 1.22, 3.8, 1.3, 1.0),
+                                  shape3d<double, 1, 8, 8, false>(1, 2.2, 2.2, 3.1, 1.3, 1.0),
+                                  shape3d<double, 2, 4, 8, false>(1, 2.2, 2.2, 4.1, 1.15, 1.15)};
+    static const Shape3D s32[] = {shape3d<float, 1, 2, 8, true>(3, 0.6, 1.05, 3.1, 1.65, 1.0),
+                                  shape3d<float, 2, 2, 8, true>(2, 0.8, 1.23, 3.1, 1.65, 1.0),
+                                  shape3d<float, 2, 4, 8, true>(1, 1.2, 1.2, 3.3, 1.65, 1.0),
+                                  shape3d<float, 2, 8, 8, false>(1, 2.4, 2.4, 3.4, 1.65, 1.0)};
     const Shape3D *best = nullptr;
     int chunks = 0, ntx = 0, nty = 0;
     double best_us = 1e30;
@@ -546,13 +583,13 @@ bool jacobi_pipe_configure(const cfm_jacobi_params &p, JacobiConfig *c) {
         }
     }
     if (!best) return false;
-    // A sweep whose norm is wanted starts a pass, so passes are short where norms are frequent: with
-    // sweeps a pass on average, the streaming kernels (jacobi.hip), two sweeps a pass with or without
-    // norms, may be the faster ones.  They take at least 15 us a sweep and 1.6 ps a point
-    // (FP32: 0.8): 229 us measured at 512^3 FP64, 39 at 200^3, 21 at 24^3.
-    const int ne = p.norm_every;
-    const double sweeps = ne > 0 ? (double)ne / ((ne + L - 1) / L) : L;
-    if (best_us / sweeps > 15.0 + points * (f64 ? 1.6e-6 : 0.8e-6)) return false;
+    // The streaming kernels make two sweeps a pass whatever the run: they are the faster ones where a run is
+    // short, where norms are frequent (a sweep whose norm is wanted starts a pass) and where planes are
+    // few.  512^3 FP64, us, streaming / pipeline: 2 sweeps 542 / 657, 4 of periodic planes 1122 / 1305, 40 with a
+    // norm every 5 9416 / 9312, every 4 9368 / 6215; 3 x 512 x 512, 40 sweeps 251 / 181, with a norm every 3
+    // 255 / 277.  (Within the estimates' spread of 5 % the streaming kernels keep a run.)
+    const int sweeps = std::min(p.niter, 4096);
+    if (1.05 * run_us(p, *best, ntx * nty, chunks, c->dev.cus, sweeps) > streaming_us(p, *c, sweeps)) return false;
     KernelFn fn = best->fn[p.phase_timers != 0];
     const int block = 64 * best->waves;
     int per_cu = 0;

@@ -55,3 +55,19 @@ def test_passes_of_an_asked_kernel(gpu):
     assert _route(gpu, (40, 40, 40), 7, variant=gpu.NO_COMPUTE)["passes"] == 0
     with pytest.raises(gpu.CfmError):
         _route(gpu, (40, 40, 2), 7)
+
+
+# (shape, sweeps, norm_every, boundary) and whether the pipeline is the faster kernel there, as measured
+@pytest.mark.parametrize("shape,niter,norm_every,bc,dtype,pipeline", [
+    ((512, 512, 512), 40, 0, 1, np.float64, True), ((512, 512, 512), 2, 0, 1, np.float64, False),
+    ((512, 512, 512), 1, 0, 1, np.float64, False), ((512, 512, 512), 4, 0, 1, np.float64, True),
+    ((512, 512, 512), 4, 0, 0, np.float64, False), ((512, 512, 512), 5, 0, 0, np.float64, True),
+    ((512, 512, 512), 2, 0, 0, np.float32, False), ((512, 512, 512), 40, 4, 1, np.float64, True),
+    ((512, 512, 512), 40, 1, 1, np.float64, False), ((512, 512, 512), 40, 3, 1, np.float32, False),
+    ((300, 300, 300), 2, 0, 0, np.float64, False), ((300, 300, 300), 3, 0, 1, np.float64, True),
+    ((3, 512, 512), 2, 0, 1, np.float64, False), ((3, 512, 512), 40, 0, 1, np.float64, True),
+    ((3, 512, 512), 40, 2, 1, np.float64, False), ((64, 64, 64), 1, 0, 1, np.float64, True),
+    ((64, 64, 64), 40, 2, 0, np.float32, True)])
+def test_pipeline_where_it_is_faster(gpu, shape, niter, norm_every, bc, dtype, pipeline):
+    kernel = _route(gpu, shape, niter, norm_every, dtype, bc)["kernel"]
+    assert kernel == ("register pipeline" if pipeline else "streaming")
