@@ -398,6 +398,54 @@ double pass_us(const cfm_jacobi_params &p, const Shape2D &s, int depth, int cus)
            (pairs ? 0.05 * std::ceil(rounds / 2) : 0.2 * rounds) * depth + (pairs ? 0.5 : 0.75) * traffic;
 }
 
+// Estimated microseconds of `sweeps` sweeps from the start of a run: its passes, with what large, flat and
+// narrow fields and norms add to them (measured, too):
+//   * a pass that moves more than the caches hold takes at least its traffic at 4.2 TB/s;
+//   * each round of tiles beyond the first its loads and stores: 1.2 us, 2.2 for pairs of workgroups (16 and
+//     fewer rows of 2,000,000), 3 more where every tile has a face in x (8 to 64 columns);
+//   * a pass with a norm masks all its tiles, and each norm sums up every point.
+double run_us(const cfm_jacobi_params &p, const Shape2D &s, int depth, int cus, int sweeps) {
+    const Split2D o = split2d(p, s, depth);
+    const bool f64 = p.prec == CFM_F64, pairs = s.waves <= 8;
+    const double rounds = std::ceil((double)o.ntx * o.nty / cus), rows = rounds * (s.r * s.waves / 4);
+    const double moved = 2.0 * (f64 ? 8 : 4) * p.nx * (double)p.ny;
+    const double tiles = (rounds - 1) * ((pairs ? 2.2 : 1.2) + (o.ntx <= 2 ? 3.0 : 0.0));
+    const bool masked = rounds <= (pairs ? 2 : 1);  // (as in pass_us)
+    double us = 0.0;
+    for (int k = 0; k < sweeps;) {
+        const int steps = p.bc == CFM_BC_PERIODIC && k == 0 ? 1 : std::min(depth, sweeps - k);
+        const int ne = p.norm_every, norms = ne > 0 ? (k + steps + ne - 1) / ne - (k + ne - 1) / ne : 0;
+        double pass = pass_us(p, s, steps, cus) + tiles + norms * rows * (f64 ? 0.025 : 0.052);
+        if (norms > 0 && !masked) pass += 1.07 * rows * steps * (f64 ? 16 : 30) / 2400.0;
+        us += moved > 2.5e8 ? std::max(pass, moved / 4.2e6) : pass;
+        k += steps;
+    }
+    return us;
+}
+
+// The same of the streaming kernels (jacobi.hip), as configured in c: a row after another of a chunk, one and
+// two more at each end for every further sweep of the pass, for each round of wavefronts; norms cost them
+// nothing.  Microseconds of a row for 1 to 4 sweeps a pass, more the fuller the chip is (half as much again for FP32 rows that
+// are not whole vectors), and TB/s; 9 us between passes.  At 16384^2 and 1024^2 FP64 this gives 1202 and 156
+// us for four sweeps, 904 and 91 for two of periodic rows, measured 1124 and 144, 863 and 89.
+double streaming_us(const cfm_jacobi_params &p, const JacobiConfig &c, int sweeps) {
+    static const double row64[] = {0.85, 1.0, 1.5, 1.9}, row32[] = {1.0, 1.4, 1.6, 2.4}, periodic[] = {0.9, 1.15};
+    static const double tb64[] = {4.8, 4.8, 4.0, 3.6}, tb32[] = {4.6, 4.5, 4.0, 3.1};
+    const bool f64 = p.prec == CFM_F64, per = p.bc == CFM_BC_PERIODIC;
+    const bool ragged = !f64 && (size_t)p.nx * 4 % 16 != 0;
+    const double fill = (double)c.ntx * c.chunks / ((double)c.grid * (c.block / 64)), rounds = std::max(1.0, fill);
+    const double moved = 2.0 * c.elem_size * p.nx * (double)p.ny;
+    const auto pass = [&](int s) {
+        double row = (per ? periodic : f64 ? row64 : row32)[s - 1];
+        if (fill <= 1.0) row *= 1.0 + (s == 1 ? 0.7 : 0.3) * fill;
+        const double tb = per ? 4.8 : (f64 ? tb64 : tb32)[s - 1];
+        return (sweeps == 1 ? 2.0 : 9.0) +
+               std::max(rounds * (c.chunk_len + 2 * (s - 1)) * row * (ragged ? 1.5 : 1.0), moved / (tb * 1e6));
+    };
+    const int whole = c.sweeps_per_pass, rest = sweeps % whole;
+    return (sweeps / whole ? sweeps / whole * pass(whole) : 0.0) + (rest ? pass(rest) : 0.0);
+}
+
 }  // namespace
 
 bool jacobi_tile_configure(const cfm_jacobi_params &p, JacobiConfig *c) {
@@ -430,6 +478,13 @@ bool jacobi_tile_configure(const cfm_jacobi_params &p, JacobiConfig *c) {
         }
     }
     if (!best) return false;
+    // The streaming kernels walk the rows of a field of any shape at the memory's rate, with or without norms:
+    // they are the faster ones for a few sweeps of a large field, and for fields of few rows, most of
+    // which a tile's rows lie outside.  FP64, us, streaming / tiles: 16384^2 1 sweep 893 / 987, 2 of periodic rows 921 /
+    // 1977, 4 1331 / 923, 40 with every norm 11,614 / 9886; 4,000,000 x 5, 40 sweeps 1054 / 4365, 1,000,000 x 32
+    // 1643 / 1295.  (Within the estimates' spread of 8 % the streaming kernels keep a run.)
+    const int few = std::min(p.niter, 4096);
+    if (1.08 * run_us(p, *best, depth, c->dev.cus, few) > streaming_us(p, *c, few)) return false;
     KernelFn fn = best->fn[p.phase_timers != 0];
     const int block = 64 * best->waves;
     int per_cu = 0;

@@ -71,3 +71,24 @@ def test_passes_of_an_asked_kernel(gpu):
 def test_pipeline_where_it_is_faster(gpu, shape, niter, norm_every, bc, dtype, pipeline):
     kernel = _route(gpu, shape, niter, norm_every, dtype, bc)["kernel"]
     assert kernel == ("register pipeline" if pipeline else "streaming")
+
+
+@pytest.mark.parametrize("shape,niter,norm_every,bc,dtype,tiles", [
+    ((16384, 16384), 40, 0, 1, np.float64, True), ((16384, 16384), 1, 0, 1, np.float64, False),
+    ((16384, 16384), 2, 0, 1, np.float64, False), ((16384, 16384), 2, 0, 0, np.float64, False),
+    ((16384, 16384), 4, 0, 0, np.float64, False), ((16384, 16384), 8, 0, 0, np.float64, True),
+    ((16384, 16384), 40, 1, 1, np.float64, True), ((8192, 8192), 4, 1, 0, np.float32, False),
+    ((8192, 8192), 40, 10, 0, np.float32, True), ((1024, 1024), 1, 0, 1, np.float64, True),
+    ((1024, 1024), 1000, 1, 0, np.float32, True), ((5, 4000000), 40, 0, 1, np.float64, False),
+    ((3, 30000000), 40, 0, 0, np.float32, False), ((32, 1000000), 40, 0, 1, np.float64, True),
+    ((32, 1000000), 2, 0, 1, np.float64, False), ((3, 30000), 40, 0, 1, np.float64, True)])
+def test_tiles_where_they_are_faster(gpu, shape, niter, norm_every, bc, dtype, tiles):
+    kernel = _route(gpu, shape, niter, norm_every, dtype, bc)["kernel"]
+    assert kernel == ("register tiles" if tiles else "streaming")
+
+
+@pytest.mark.parametrize("dtype,limit", [(np.float64, 1 << 28), (np.float32, 1 << 29)])
+def test_rows_of_2gib_are_no_tiles(gpu, dtype, limit):
+    """(whatever the estimates say: their offsets are 32-bit)"""
+    assert _route(gpu, (3, limit), 40, 0, dtype)["kernel"] == "streaming"
+    assert _route(gpu, (3, limit - 4), 40, 0, dtype)["kernel"] in ("streaming", "register tiles")
