@@ -3,6 +3,8 @@
 // configuration of one parameter set, and the enqueue of one run.
 #pragma once
 
+#include <algorithm>
+
 #include "cfm_common.hpp"
 
 namespace cfm {
@@ -36,6 +38,7 @@ struct JacobiConfig {
     size_t elems = 0;
     size_t elem_size = 0;
     int norm_slots = 0;
+    size_t norm_doubles = 0;  // set before: what the workgroups' sums of all norms have to fit in (0: no limit)
     KernelFn kernel = nullptr;
     bool t2 = false;  // more than one sweep per pass (the two-/three-/four-sweep kernels)
     int sweeps_per_pass = 1;
@@ -68,6 +71,11 @@ __host__ __device__ inline double jacobi_norm_sum(const double *part, int n) {
         sum = next;
     }
     return lost == lost ? sum + lost : sum;  // (an infinite sum has no meaningful rest)
+}
+// Workgroups whose sums of the run's norms, and the norms themselves, fit.
+inline int jacobi_norm_workgroups(const JacobiConfig &c) {
+    if (c.norm_doubles == 0 || c.norm_slots == 0) return kMaxGrid;
+    return (int)std::min((size_t)kMaxGrid, std::max(c.norm_doubles / c.norm_slots, (size_t)2) - 1);
 }
 // Takes c to a register-tile kernel where that is the faster one; false leaves it as it is.
 bool jacobi_tile_configure(const cfm_jacobi_params &p, JacobiConfig *c);  // 2D

@@ -3,7 +3,8 @@
 // a file-scope device array (`scratch`) instead of plan buffers, so the call
 // makes no hipMalloc / hipFree and creates no stream or event.  Launch
 // configuration and kernels are the plan path's (jacobi_configure,
-// jacobi_enqueue), so results are the same bits.
+// jacobi_enqueue), so the field is the same bits, and so are the norms unless they are so many that
+// their sums fit the array for fewer workgroups than a plan would launch.
 #include <hip/hip_runtime.h>
 
 #include <chrono>
@@ -45,8 +46,7 @@ cfm_status scratch_ptr(int device, unsigned char **out) {
     return CFM_OK;
 }
 
-// sums[s] = the sum of part[s][...] as the plan path forms it on the host (so the
-// square roots are the same bits).
+// sums[s] = the sum of part[s][...] as the plan path forms it on the host.
 __global__ void norm_slot_sums_kernel(const double *part, int slots, int grid, double *sums) {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= slots) return;
@@ -65,6 +65,7 @@ extern "C" cfm_status cfm_jacobi_run_noalloc(const cfm_jacobi_params *p, void *f
     if (p->phase_timers) return CFM_FAIL(CFM_EINVAL, "jacobi_noalloc: phase timers need a plan");
     const auto w0 = std::chrono::steady_clock::now();
     JacobiConfig c;
+    c.norm_doubles = kScratchDoubles;
     cfm_status st = jacobi_configure(p, &c);
     if (st != CFM_OK) return st;
     const size_t slots = p->variant == CFM_JACOBI_NO_COMPUTE ? 0 : (size_t)c.norm_slots;
@@ -72,8 +73,6 @@ extern "C" cfm_status cfm_jacobi_run_noalloc(const cfm_jacobi_params *p, void *f
         return CFM_FAIL(CFM_EINVAL,
                         "jacobi_noalloc: %zu norm slots x %d workgroups exceed the %zu-double scratch array "
                         "(fewer norms, or a plan)", slots, c.norm_grid, kScratchDoubles);
-    // a register-tile grid may be the larger one; it runs on any number of workgroups
-    if (c.tile && slots > 0) c.grid = (int)std::min((size_t)c.grid, kScratchDoubles / slots - 1);
     unsigned char *base = nullptr;
     st = scratch_ptr(c.dev.device, &base);
     if (st != CFM_OK) return st;

@@ -503,20 +503,22 @@ Shape3D shape3d(int per_cu, double step_us, double full_us, double tb_s, double 
 int tiles_along(int n, int span) { return n <= span ? 1 : (n - span + span - 2 * L - 1) / (span - 2 * L) + 1; }
 
 // Estimated microseconds of one pass: the chunk's planes and 2 L more to fill and empty the pipeline,
-// for each round of boxes; the device-wide barrier, the first loads and the last stores, 5 us.
-double pass_us(const cfm_jacobi_params &p, const Shape3D &s, int tiles, int chunks, int cus, double longer = 1.0) {
+// for each round of boxes on `most` workgroups or as many as fit; the device-wide barrier, the first loads and
+// the last stores, 5 us.
+double pass_us(const cfm_jacobi_params &p, const Shape3D &s, int tiles, int chunks, int cus, int most,
+               double longer = 1.0) {
     const int len = (p.nz - 2 + chunks - 1) / chunks;
     const double units = (double)tiles * chunks;
-    const double rounds = std::ceil(units / (cus * s.per_cu));
+    const double rounds = std::ceil(units / std::min(cus * s.per_cu, most));
     const double moved = 2.0 * (p.prec == CFM_F64 ? 8 : 4) * p.nx * (double)p.ny * p.nz;
     return 5.0 + std::max(rounds * (len + 2 * L) * (units > cus ? s.full_us : s.step_us) * longer,
                           moved > 2.0e8 ? moved / (s.tb_s * 1e6) : 0.0);
 }
 
 // Estimated microseconds of `sweeps` sweeps from the start of a run.
-double run_us(const cfm_jacobi_params &p, const Shape3D &s, int tiles, int chunks, int cus, int sweeps) {
-    const double plain = pass_us(p, s, tiles, chunks, cus), norm = pass_us(p, s, tiles, chunks, cus, s.norm),
-                 part = pass_us(p, s, tiles, chunks, cus, s.part);
+double run_us(const cfm_jacobi_params &p, const Shape3D &s, int tiles, int chunks, int cus, int most, int sweeps) {
+    const double plain = pass_us(p, s, tiles, chunks, cus, most), norm = pass_us(p, s, tiles, chunks, cus, most, s.norm),
+                 part = pass_us(p, s, tiles, chunks, cus, most, s.part);
     double us = 0.0;
     for (int k = 0; k < sweeps;) {
         const int steps = jacobi_pipe_steps(k, sweeps, L, p.norm_every, p.bc == CFM_BC_PERIODIC);
@@ -573,12 +575,12 @@ bool jacobi_pipe_configure(const cfm_jacobi_params &p, JacobiConfig *c) {
     const Shape3D *best = nullptr;
     int chunks = 0, ntx = 0, nty = 0;
     double best_us = 1e30;
-    const int interior = p.nz - 2;
+    const int interior = p.nz - 2, most = jacobi_norm_workgroups(*c);
     for (const Shape3D &s : f64 ? s64 : s32) {
         const int tx = tiles_along(p.nx, 64 * s.vx), ty = tiles_along(p.ny, s.r * s.waves);
         if ((double)tx * ty * interior > 1e9) continue;
         for (int ch = 1; ch <= std::min(interior, 2048); ++ch) {  // (some rounds of what fits at once, at any size)
-            const double us = pass_us(p, s, tx * ty, ch, c->dev.cus);
+            const double us = pass_us(p, s, tx * ty, ch, c->dev.cus, most);
             if (us < best_us) best_us = us, best = &s, chunks = ch, ntx = tx, nty = ty;
         }
     }
@@ -589,7 +591,7 @@ bool jacobi_pipe_configure(const cfm_jacobi_params &p, JacobiConfig *c) {
     // norm every 5 9416 / 9312, every 4 9368 / 6215; 3 x 512 x 512, 40 sweeps 251 / 181, with a norm every 3
     // 255 / 277.  (Within the estimates' spread of 5 % the streaming kernels keep a run.)
     const int sweeps = std::min(p.niter, 4096);
-    if (1.05 * run_us(p, *best, ntx * nty, chunks, c->dev.cus, sweeps) > streaming_us(p, *c, sweeps)) return false;
+    if (1.05 * run_us(p, *best, ntx * nty, chunks, c->dev.cus, most, sweeps) > streaming_us(p, *c, sweeps)) return false;
     KernelFn fn = best->fn[p.phase_timers != 0];
     const int block = 64 * best->waves;
     int per_cu = 0;
@@ -606,7 +608,7 @@ bool jacobi_pipe_configure(const cfm_jacobi_params &p, JacobiConfig *c) {
     c->chunks = (interior + c->chunk_len - 1) / c->chunk_len;
     c->depth = L;
     c->pipe = true;
-    c->grid = (int)std::min((long long)std::min(per_cu * c->dev.cus, kMaxGrid), (long long)ntx * nty * c->chunks);
+    c->grid = (int)std::min((long long)std::min(per_cu * c->dev.cus, most), (long long)ntx * nty * c->chunks);
     return true;
 }
 

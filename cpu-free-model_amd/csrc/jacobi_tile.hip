@@ -384,7 +384,7 @@ Split2D split2d(const cfm_jacobi_params &p, const Shape2D &s, int depth) {
 // At 16384^2 FP64 in 14-row, 8-wavefront tiles it gives 890, 1330 and 1800 us for depths 8, 12 and
 // 16, measured 900, 1322 and 1780; at 1024^2 in 6-row tiles 16.1 and 23.2 for depths 12 and 20,
 // measured 17.2 and 24.9.
-double pass_us(const cfm_jacobi_params &p, const Shape2D &s, int depth, int cus) {
+double pass_us(const cfm_jacobi_params &p, const Shape2D &s, int depth, double cus) {
     const Split2D o = split2d(p, s, depth);
     if (o.ntx < 1) return 1e30;
     const bool f64 = p.prec == CFM_F64;
@@ -404,7 +404,7 @@ double pass_us(const cfm_jacobi_params &p, const Shape2D &s, int depth, int cus)
 //   * each round of tiles beyond the first its loads and stores: 1.2 us, 2.2 for pairs of workgroups (16 and
 //     fewer rows of 2,000,000), 3 more where every tile has a face in x (8 to 64 columns);
 //   * a pass with a norm masks all its tiles, and each norm sums up every point.
-double run_us(const cfm_jacobi_params &p, const Shape2D &s, int depth, int cus, int sweeps) {
+double run_us(const cfm_jacobi_params &p, const Shape2D &s, int depth, double cus, int sweeps) {
     const Split2D o = split2d(p, s, depth);
     const bool f64 = p.prec == CFM_F64, pairs = s.waves <= 8;
     const double rounds = std::ceil((double)o.ntx * o.nty / cus), rows = rounds * (s.r * s.waves / 4);
@@ -464,16 +464,22 @@ bool jacobi_tile_configure(const cfm_jacobi_params &p, JacobiConfig *c) {
     const Shape2D *best = nullptr;
     int depth = 0;
     double best_us = 1e30;
+    const int most = jacobi_norm_workgroups(*c);
+    const auto cus_of = [&](const Shape2D &s) {  // as many as `most` workgroups fill
+        const double per_cu = s.waves <= 8 ? 2.0 : 1.0;
+        return std::min(per_cu * c->dev.cus, (double)most) / per_cu;
+    };
     for (const Shape2D &s : f64 ? s64 : s32) {
+        const double cus = cus_of(s);
         const Split2D whole = split2d(p, s, 1);
         if (whole.ntx * whole.nty == 1 && p.bc == CFM_BC_DIRICHLET) {  // one workgroup holds the field
-            const double us = pass_us(p, s, sweeps, c->dev.cus);
+            const double us = pass_us(p, s, sweeps, cus);
             if (us < best_us) best_us = us, best = &s, depth = sweeps;
             continue;
         }
         for (int d = std::min(2, sweeps); d <= std::min(24, sweeps); ++d) {
-            double us = sweeps / d * pass_us(p, s, d, c->dev.cus);
-            if (sweeps % d) us += pass_us(p, s, sweeps % d, c->dev.cus);
+            double us = sweeps / d * pass_us(p, s, d, cus);
+            if (sweeps % d) us += pass_us(p, s, sweeps % d, cus);
             if (us < best_us) best_us = us, best = &s, depth = d;
         }
     }
@@ -484,7 +490,7 @@ bool jacobi_tile_configure(const cfm_jacobi_params &p, JacobiConfig *c) {
     // 1977, 4 1331 / 923, 40 with every norm 11,614 / 9886; 4,000,000 x 5, 40 sweeps 1054 / 4365, 1,000,000 x 32
     // 1643 / 1295.  (Within the estimates' spread of 8 % the streaming kernels keep a run.)
     const int few = std::min(p.niter, 4096);
-    if (1.08 * run_us(p, *best, depth, c->dev.cus, few) > streaming_us(p, *c, few)) return false;
+    if (1.08 * run_us(p, *best, depth, cus_of(*best), few) > streaming_us(p, *c, few)) return false;
     KernelFn fn = best->fn[p.phase_timers != 0];
     const int block = 64 * best->waves;
     int per_cu = 0;
@@ -500,7 +506,7 @@ bool jacobi_tile_configure(const cfm_jacobi_params &p, JacobiConfig *c) {
     c->ntx = o.ntx;
     c->nty = o.nty;
     c->depth = depth;
-    c->grid = (int)std::min((long long)std::min(per_cu * c->dev.cus, kMaxGrid), (long long)o.ntx * o.nty);
+    c->grid = (int)std::min((long long)std::min(per_cu * c->dev.cus, most), (long long)o.ntx * o.nty);
     return true;
 }
 
