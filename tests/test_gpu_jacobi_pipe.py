@@ -36,3 +36,14 @@ def test_boxes_3d(gpu, orc, shape, bc, dtype):
 def test_boxes_3d_tall(gpu, orc, dtype, shape, bc):
     """Fields of many boxes: the eight-row shapes, chunks of many planes."""
     _check(gpu, orc, shape, dtype, 11, bc, 6)
+
+
+@pytest.mark.parametrize("bc", [0, 1])
+@pytest.mark.parametrize("shape", [(80, 300, 241), (90, 260, 256)])
+def test_boxes_3d_of_16_byte_lanes(gpu, orc, shape, bc):
+    """FP64 in lanes of two columns, the shape of the largest fields: an odd row (whose last column is a lane's first,
+    and whose last lane reaches into the next plane) and rows of whole vectors, with and without norms."""
+    p = gpu.jacobi_params(shape[2], shape[1], shape[0], 22, 0, gpu.F64, bc)
+    assert gpu.jacobi_route(p)["kernel"] == "register pipeline"
+    for niter, norm_every in ((22, 0), (14, 5), (9, 4)):
+        _check(gpu, orc, shape, np.float64, niter, bc, norm_every)

@@ -92,3 +92,25 @@ def test_rows_of_2gib_are_no_tiles(gpu, dtype, limit):
     """(whatever the estimates say: their offsets are 32-bit)"""
     assert _route(gpu, (3, limit), 40, 0, dtype)["kernel"] == "streaming"
     assert _route(gpu, (3, limit - 4), 40, 0, dtype)["kernel"] in ("streaming", "register tiles")
+
+
+# runs that keep the streaming kernels: one, two and four sweeps a pass, odd and even pass counts, x tiles, rows that
+# are not whole vectors
+@pytest.mark.parametrize("bc", [0, 1])
+@pytest.mark.parametrize("shape,dtype,niter,norm_every", [
+    ((3, 512, 512), np.float64, 2, 0), ((3, 512, 512), np.float32, 4, 1), ((3, 500, 1022), np.float64, 3, 1),
+    ((3, 700, 1100), np.float32, 4, 1), ((4, 500, 515), np.float64, 2, 1), ((4, 900, 511), np.float64, 3, 1),
+    ((5, 400000), np.float64, 7, 0), ((5, 400001), np.float32, 5, 2), ((6, 300002), np.float64, 4, 1),
+    ((3, 1000000), np.float32, 9, 3)])
+def test_streaming_by_default_bitexact(gpu, orc, shape, dtype, niter, norm_every, bc):
+    assert _route(gpu, shape, niter, norm_every, dtype, bc)["kernel"] == "streaming"
+    init = np.random.default_rng(shape[-1] + niter).uniform(-1, 1, shape).astype(dtype)
+    ref, rnorms = orc.jacobi(init, niter, bc, norm_every)
+    out, norms, _ = gpu.jacobi(init, niter, bc=bc, norm_every=norm_every)
+    assert np.array_equal(out, ref)
+    assert len(norms) == len(rnorms) and np.allclose(norms, rnorms, rtol=1e-10, atol=0.0)
+    nz, ny, nx = (1,) + shape if len(shape) == 2 else shape
+    p = gpu.jacobi_params(nx, ny, nz, niter, norm_every, gpu.F64 if dtype == np.float64 else gpu.F32, bc)
+    with gpu.DeviceBuffer.of(init) as field, gpu.DeviceBuffer(init.nbytes) as work:
+        nnorms, _ = gpu.jacobi_noalloc(p, field, work)
+        assert np.array_equal(field.download(dtype, shape), ref) and np.array_equal(nnorms, norms)
