@@ -109,6 +109,8 @@ __device__ __forceinline__ bool grid_barrier(GridSync *s, unsigned int &epoch) {
     return s_abort == 0;
 }
 
+constexpr int kSc1 = 16;  // buffer instructions' cache policy bit: past the L2
+
 // The same barrier without the agent-scope release and acquire, for kernels in which everything one
 // workgroup reads of another's goes past the L2 on both sides: written through it (an agent-scope
 // store: scope bit sc1) and read past it (an agent-scope load).  Each of the two fences makes the XCD's L2

@@ -162,7 +162,7 @@ __device__ __forceinline__ bool solve_system(const BatchArgs &A, const System &Y
     M.load(A.A, Y.chunk, threadIdx.x, true, Y.first_chunk * kChunk);
     const bool owner = Y.chunk == Y.first_chunk && threadIdx.x == 0;
     double x[kRows], r[kRows], z[kRows], s[kRows], p[kRows], w[kRows], g[kRows][W];
-    double one[1], two[2];
+    double two[2];
     {
         double b[kRows];
         read_rows(Y, A.x0, x);

@@ -7,7 +7,6 @@
 namespace cfm {
 
 constexpr int kRows = 4;  // rows per thread: a chunk over a sub-block
-constexpr int kSc1 = 16;   // buffer instructions' cache policy bit: past the L2
 
 template <typename T>
 __device__ __forceinline__ T load_through(const T *p) {

@@ -32,7 +32,6 @@ namespace cfm {
 namespace {
 
 constexpr int L = 4;        // levels, sweeps of a pass
-constexpr int kSc1 = 16;    // buffer instructions' cache policy bit: past the L2
 constexpr unsigned kNowhere = 0xf0000000u;  // an offset beyond every plane: a store that is dropped
 
 template <typename T, int N>

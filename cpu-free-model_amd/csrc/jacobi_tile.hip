@@ -32,7 +32,6 @@ struct VecAt {
 
 // A lane's N elements at row[x .. x+N), and one of them.  THROUGH: past the L2 (scope bit sc1), for
 // grid_barrier_through; offsets are 32-bit, so jacobi_tile_configure declines rows of 2 GiB and more.
-constexpr int kSc1 = 16;  // buffer instructions' cache policy bit
 template <bool THROUGH, typename T, int N>
 __device__ __forceinline__ typename VecAt<T, N>::type load_at(const T *row, int x) {
     typedef typename VecAt<T, N>::type V;
@@ -185,7 +184,6 @@ __device__ __forceinline__ void pass_tile2d(const JacobiArgs &A, const Place2D &
                                             T *__restrict__ dst, int steps, int it, bool first,
                                             typename Tile2D<T, VX, R, WAVES>::Edge &edge, double *lds) {
     typedef typename VecAt<T, VX>::type V;
-    constexpr int C = 64 * VX;
     const int nx = A.nx, ny = A.ny;
     Tile2D<T, VX, R, WAVES> t;
     t.lane = threadIdx.x & 63;

@@ -364,7 +364,7 @@ __global__ void __launch_bounds__(192, COUT == 16 ? 3 : 1) conv3_wgrad_rows_kern
     constexpr int UP = upsampled_channels(CIN), CINX = CIN - UP;  // channels per point of the input tensor(s)
     constexpr int CW = CIN < 16 ? CIN : 16;  // input channels of this workgroup
     constexpr int CINP = 16;                 // and as many rows as a fragment has
-    constexpr int MT = COUT / 16, KT = 1, WROWS = 3, NTH = 192;
+    constexpr int MT = COUT / 16, WROWS = 3, NTH = 192;
     static_assert(CIN % CW == 0, "channel split");
     const int ci0 = blockIdx.y * CW;
     const bool up = ci0 < UP;  // (uniform; UP is a multiple of 16)
@@ -392,15 +392,13 @@ __global__ void __launch_bounds__(192, COUT == 16 ? 3 : 1) conv3_wgrad_rows_kern
             xT[r * RSTR + c * W + (c >> 3) * 8 + v % W] = (bf16)0.0f;
         }
     }
-    f32x4 acc[WROWS][3][MT][KT], accb[MT];
+    f32x4 acc[WROWS][3][MT], accb[MT];
 #pragma unroll
     for (int a = 0; a < WROWS; ++a)
 #pragma unroll
         for (int d = 0; d < 3; ++d)
 #pragma unroll
-            for (int m = 0; m < MT; ++m)
-#pragma unroll
-                for (int k = 0; k < KT; ++k) acc[a][d][m][k] = f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int m = 0; m < MT; ++m) acc[a][d][m] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int m = 0; m < MT; ++m) accb[m] = f32x4{0.f, 0.f, 0.f, 0.f};
     const bool bias = w == 0 && blockIdx.y == 0;  // (uniform over the wavefront)
@@ -553,26 +551,22 @@ __global__ void __launch_bounds__(192, COUT == 16 ? 3 : 1) conv3_wgrad_rows_kern
                 const int dz = rw / 3, dy = rw % 3;  // offsets + 1
                 int slot = base + rq[h] + dy;
                 if (slot >= R + 2) slot -= R + 2;
+                const bf16 *src = xT + (dz * (R + 2) + slot) * RSTR + nl * W + (nl >> 3) * 8 + xg[h];
+                const bf16x8 lo = *reinterpret_cast<const bf16x8 *>(src);
+                const bf16x8 hi = *reinterpret_cast<const bf16x8 *>(src + 8);
+                typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+                const u32x4 l4 = __builtin_bit_cast(u32x4, lo), h4 = __builtin_bit_cast(u32x4, hi);
+                const u32x4 mid = {__builtin_amdgcn_alignbyte(l4[1], l4[0], 2),
+                                   __builtin_amdgcn_alignbyte(l4[2], l4[1], 2),
+                                   __builtin_amdgcn_alignbyte(l4[3], l4[2], 2),
+                                   __builtin_amdgcn_alignbyte(h4[0], l4[3], 2)};
+                const u32x4 up = {l4[1], l4[2], l4[3], h4[0]};
+                const bf16x8 bv[3] = {lo, __builtin_bit_cast(bf16x8, mid), __builtin_bit_cast(bf16x8, up)};
 #pragma unroll
-                for (int k = 0; k < KT; ++k) {
-                    const bf16 *src = xT + (dz * (R + 2) + slot) * RSTR + (k * 16 + nl) * W + (2 * k + (nl >> 3)) * 8 + xg[h];
-                    const bf16x8 lo = *reinterpret_cast<const bf16x8 *>(src);
-                    const bf16x8 hi = *reinterpret_cast<const bf16x8 *>(src + 8);
-                    typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-                    const u32x4 l4 = __builtin_bit_cast(u32x4, lo), h4 = __builtin_bit_cast(u32x4, hi);
-                    const u32x4 mid = {__builtin_amdgcn_alignbyte(l4[1], l4[0], 2),
-                                       __builtin_amdgcn_alignbyte(l4[2], l4[1], 2),
-                                       __builtin_amdgcn_alignbyte(l4[3], l4[2], 2),
-                                       __builtin_amdgcn_alignbyte(h4[0], l4[3], 2)};
-                    const u32x4 up = {l4[1], l4[2], l4[3], h4[0]};
-                    const bf16x8 bv[3] = {lo, __builtin_bit_cast(bf16x8, mid), __builtin_bit_cast(bf16x8, up)};
+                for (int d = 0; d < 3; ++d)
 #pragma unroll
-                    for (int d = 0; d < 3; ++d)
-#pragma unroll
-                        for (int m = 0; m < MT; ++m)
-                            acc[a][d][m][k] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[m], bv[d], acc[a][d][m][k], 0,
-                                                                                      0, 0);
-                }
+                    for (int m = 0; m < MT; ++m)
+                        acc[a][d][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[m], bv[d], acc[a][d][m], 0, 0, 0);
             }
         }
         if (bias && ((blk - s * S.per_slab) % kBiasBlocks == kBiasBlocks - 1 || blk + 1 == blk_end)) {
@@ -593,7 +587,7 @@ __global__ void __launch_bounds__(192, COUT == 16 ? 3 : 1) conv3_wgrad_rows_kern
             for (int i = 0; i < NX; ++i) put_x(xi[i], base, px[i]);
         }
     }
-    // D[4g+i][nl] = dW[m*16 + 4g + i][tap*CIN + k*16 + nl], tap = 9 dz + 3 dy + dx (offsets + 1)
+    // D[4g+i][nl] = dW[m*16 + 4g + i][tap*CIN + ci0 + nl], tap = 9 dz + 3 dy + dx (offsets + 1)
     float *out = partial + (size_t)s * COUT * (Kp + 1);
 #pragma unroll
     for (int a = 0; a < WROWS; ++a) {
@@ -603,14 +597,10 @@ __global__ void __launch_bounds__(192, COUT == 16 ? 3 : 1) conv3_wgrad_rows_kern
             const int tap = 3 * rw + d;
 #pragma unroll
             for (int m = 0; m < MT; ++m)
+                if (nl < CW)
 #pragma unroll
-                for (int k = 0; k < KT; ++k) {
-                    const int ci = k * 16 + nl;
-                    if (ci < CW)
-#pragma unroll
-                        for (int i = 0; i < 4; ++i)
-                            out[(size_t)(m * 16 + 4 * g + i) * Kp + tap * CIN + ci0 + ci] = acc[a][d][m][k][i];
-                }
+                    for (int i = 0; i < 4; ++i)
+                        out[(size_t)(m * 16 + 4 * g + i) * Kp + tap * CIN + ci0 + nl] = acc[a][d][m][i];
         }
     }
     // (the K tail [27 CIN, Kp) is left as it is: nothing reads it)
