@@ -39,33 +39,35 @@ struct Team {
     unsigned long long epoch;
 };
 
-// The sum of the launch's arrival words.  They only grow, and a workgroup that iterates passes a barrier
-// in every iteration: as long as any does, the sum grows.
+// The sum of the launch's arrival words (zeros beyond its workgroups).  They only grow, and do as long as
+// any team of several workgroups iterates.
 __device__ __forceinline__ unsigned long long arrivals(const TeamSync *s) {
     unsigned long long sum = 0;
-    for (int b = 0; b < (int)gridDim.x; ++b)
+    for (int b = 0; b < kMaxTeamGrid; ++b)
         sum += __hip_atomic_load(&s->arrive[b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     return sum;
 }
 
 // grid_barrier_through for one team: arrivals to its first workgroup, which releases every member on a
 // line of its own (a line that only that member reads: no release of an earlier team can be late).
-// At the first barrier of a later round members may still be at their previous systems, for as long as
-// those take: that wait's clock starts anew while the launch makes progress.  (All others wait for at
-// most an iteration.)
+// At the first barrier of a later round members may still be at their previous systems, which have several
+// workgroups (batch_resident_schedule), for as long as those take: that wait's clock starts anew while the
+// launch makes progress.  (All others wait for at most an iteration.  A word of a workgroup alone in its team
+// would cost it 3 to 6 % of an iteration.)
 __device__ __forceinline__ bool team_barrier(Team &T) {
     __shared__ int s_abort;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     const unsigned long long e = ++T.epoch;
-    TeamSync *s = T.s;
-    if (threadIdx.x == 0)
-        __hip_atomic_store(&s->arrive[T.me], e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (T.size == 1) return true;
+    TeamSync *s = T.s;
     const unsigned long long limit = s->spin_limit_ticks;
     const bool patient = (unsigned)e == 1 && (e >> 32) > 1;
     int ab = 0;
-    if (threadIdx.x == 0) s_abort = 0;
+    if (threadIdx.x == 0) {
+        s_abort = 0;
+        __hip_atomic_store(&s->arrive[T.me], e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
     const bool gather = T.me == T.base;
     if (gather) __syncthreads();
     if (gather || threadIdx.x == 0) {
@@ -74,8 +76,9 @@ __device__ __forceinline__ bool team_barrier(Team &T) {
         const int count = gather ? T.size - (int)threadIdx.x : 1;
         for (int b = 0; b < count && !ab; b += blockDim.x) {
             while (__hip_atomic_load(first + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < e) {
+                const bool stop = __hip_atomic_load(&s->abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 const bool late = spin_expired(t0, limit);
-                if (late && patient) {
+                if (late && patient && !stop) {
                     const unsigned long long now = arrivals(s);
                     if (now != seen) {
                         seen = now;
@@ -83,7 +86,7 @@ __device__ __forceinline__ bool team_barrier(Team &T) {
                         continue;
                     }
                 }
-                if (late || __hip_atomic_load(&s->abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+                if (late || stop) {
                     __hip_atomic_store(&s->abort, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                     ab = 1;
                     break;
@@ -302,6 +305,8 @@ BatchResidentFn batch_resident_kernel(int max_width, const DeviceProps &dev, int
 
 // Largest systems first (they also need the most iterations), each into the first round with room: a
 // round then holds systems of about the same length, with small ones in what the large ones leave.
+// Systems of one chunk go where no larger one comes after them: the members of a team wait for each other
+// as long as arrival words grow, and a workgroup alone in its team has none.
 std::vector<TeamSlot> batch_resident_schedule(const std::vector<int> &chunk0, int grid, int *rounds) {
     const int nsys = (int)chunk0.size() - 1;
     std::vector<int> order(nsys);
@@ -311,9 +316,14 @@ std::vector<TeamSlot> batch_resident_schedule(const std::vector<int> &chunk0, in
     });
     std::vector<TeamSlot> slots;
     std::vector<int> used;  // workgroups taken, per round
+    bool alone = false;     // the systems of one chunk have begun
     for (const int s : order) {
         const int need = chunk0[s + 1] - chunk0[s];
         if (need > grid) return {};
+        if (need == 1 && !alone) {
+            alone = true;
+            for (int k = (int)used.size() - 2; k >= 0; --k) used[k] = std::max(used[k], used[k + 1]);
+        }
         size_t r = 0;
         while (r < used.size() && used[r] + need > grid) ++r;
         if (r == used.size()) {

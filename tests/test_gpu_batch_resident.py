@@ -116,3 +116,24 @@ def test_batch_tune_cache_names_the_candidates(gpu, tmp_path):
     old = cache.read_text().splitlines()[1].split()[0].split("|format=")[0]
     cache.write_text(f"{old} 4 256 0\n")
     assert tune()[3] == 2
+
+
+def test_batch_resident_single_chunks_come_last(gpu):
+    """Systems of one chunk, whose workgroups have no barriers that a later team could see them pass, iterate for a
+    multiple of the watchdog's limit beside systems that take two rounds of almost the whole grid."""
+    limit_us = 1000
+    systems = [_line(1024 * c) for c in (700, 750)] + [_line(1000 + i) for i in range(60)]
+    srp, rp, col, val = gpu.block_diag(systems)
+    b = gpu.uniform(9, 0, int(srp[-1])) - 0.5
+    b[:srp[2]] = 0.0  # the large ones are solved by x0 = 0
+    p = gpu.cg_params(method=gpu.CG_PIPELINED, tol=1e-8, max_iter=3000, spin_limit_us=limit_us)
+    with gpu.CgBatchPlan(srp, rp, col, val, p) as plan:
+        plan.set_rhs(b)
+        plan.set_x0(None)
+        st, iters, stat, _, t = plan.solve()
+        x = plan.x()
+        assert plan.resident() and t["kernel_ms"] > 2e-3 * limit_us
+    assert list(iters[:2]) == [0, 0] and not x[:srp[2]].any()
+    for s in (2, 30, 61):
+        alone = gpu.cg(*systems[s], b[srp[s]:srp[s + 1]], method=gpu.CG_PIPELINED, tol=1e-8, max_iter=3000)
+        assert stat[s] == alone[0] and iters[s] == alone[3] and np.array_equal(x[srp[s]:srp[s + 1]], alone[1])
