@@ -78,10 +78,11 @@ typedef struct {
     int chunks;       /* chunks along the streamed axis; 0 = auto */
     int spin_limit_us;/* device barrier watchdog; 0 = default (10 s) */
     int block_threads;/* 0 = one workgroup per CU (size set by the tile shape), or 256 */
-    int time_block;   /* sweeps per HBM pass of the persistent kernels: 0 = auto (2D with nothing else
-                         set: register tiles, whose passes are as deep as pays; 2D otherwise: Dirichlet 4,
-                         or 3 with 1024-thread workgroups, periodic y 2; 3D with nothing else set: a register
-                         pipeline of 4 sweeps a pass, where norms are not too frequent for it; 3D
+    int time_block;   /* sweeps per HBM pass of the persistent kernels: 0 = auto (with nothing else
+                         set: register tiles in 2D, whose passes are as deep as pays, and a register
+                         pipeline of 4 sweeps a pass in 3D, where an estimate of the whole run, its norms
+                         and its length included, has them ahead (cfm_jacobi_describe tells); 2D otherwise:
+                         Dirichlet 4, or 3 with 1024-thread workgroups, periodic y 2; 3D
                          otherwise: 2, Dirichlet or periodic z (periodic: 512-thread workgroups; nx > 512: x tiles, which need 16-byte aligned rows, a
                          field below 2 GiB and 512-thread workgroups); with the default tile shape,
                          else 1), 1, 2, or 3 and 4 (2D Dirichlet only; 4 in 512-thread workgroups) */
@@ -195,7 +196,9 @@ cfm_status cfm_jacobi_run(const cfm_jacobi_params *p, const void *init_host, voi
  * elements of the plan's type, the initial field in, the result out; work
  * (device, borrowed, same size, distinct): overwritten (it starts as a copy
  * of field).  stream: a hipStream_t, NULL for the null stream; the call
- * returns when the run is done.  Same kernels and bits as the plan path.
+ * returns when the run is done.  The field has the plan path's bits; the norms
+ * too, unless the plan's grid needs more norm partials than the array holds:
+ * then the kernel and a smaller grid are chosen for the array.
  * Refused with CFM_EINVAL: phase_timers, and norm slots x (workgroups + 1)
  * beyond the array's 257,888 FP64 words (e.g. 1003 norms at 256 workgroups).
  * Calls that overlap on one GPU share the array and race.  kernel_ms is the
